@@ -23,6 +23,7 @@ SOURCES = [
     "k_fft.hip",
     "k_stencil.hip",
     "k_blocktri.hip",
+    "k_factor.hip",
     "k_vec.hip",
     "hz_noalloc.hip",
     "k_hodlr.hip",

@@ -29,47 +29,11 @@
 #include <type_traits>
 
 #include "hz_internal.h"
+#include "k_plane.h"
 
 namespace hz {
 namespace {
 
-template <typename T> struct Cx;
-template <> struct Cx<float> { typedef float2 t; };
-template <> struct Cx<double> { typedef double2 t; };
-
-template <typename C> __device__ __forceinline__ C mk(double x, double y) { C r; r.x = x; r.y = y; return r; }
-template <typename C> __device__ __forceinline__ C cmul(C a, C b) {
-  C r; r.x = a.x * b.x - a.y * b.y; r.y = a.x * b.y + a.y * b.x; return r;
-}
-template <typename C> __device__ __forceinline__ C cfma(C a, C b, C c) {  // a*b + c
-  C r; r.x = a.x * b.x - a.y * b.y + c.x; r.y = a.x * b.y + a.y * b.x + c.y; return r;
-}
-template <typename C> __device__ __forceinline__ C cfma_conj(C a, C b, C c) {  // conj(a)*b + c
-  C r; r.x = a.x * b.x + a.y * b.y + c.x; r.y = a.x * b.y - a.y * b.x + c.y; return r;
-}
-template <typename C> __device__ __forceinline__ C cinv(C a) {
-  // 1/a with scaling to avoid overflow in |a|^2
-  double ax = a.x, ay = a.y;
-  double s = fmax(fabs(ax), fabs(ay));
-  C r;
-  if (s == 0.0) { r.x = ax / 0.0; r.y = 0; return r; }
-  double bx = ax / s, by = ay / s;
-  double d = s * (bx * bx + by * by);
-  r.x = bx / d; r.y = -by / d;
-  return r;
-}
-
-struct PlaneTabs {
-  const double2* cmx;
-  const double2* cpx;
-  const double2* cdx;
-  const double2* cdy;
-  const double2* kappa;
-  const double* lamz;
-  const double2* sig;
-};
-
-typedef float hz_v4f __attribute__((ext_vector_type(4)));
 constexpr int FACT_THREADS = 512;
 constexpr int TCM = 64;  // columns per trailing-update chunk on the matrix cores (complex64)
 constexpr int TC = 32;   // columns per trailing-update tile
@@ -3037,6 +3001,30 @@ size_t factor_lds(int n, int nb) {
   return sizeof(C) * ((size_t)nb * n + tc * nb + nb + n) + sizeof(int) * (n + 4);
 }
 
+// one launch of the factor chains (mode, m, jbeg, jend as in k_factor): in
+// registers where a block fits them, else the panel-by-panel kernel
+template <typename T>
+void run_factor_mem(hz_problem* p, int prec, int blocks, int* st, int mode, int m, int jbeg, int jend, hipStream_t s) {
+  typedef typename Cx<T>::t C;
+  const int n = (int)p->nx;
+  Factors& f = p->fac[prec];
+  int nb = 32;
+  while (nb > 4 && factor_lds<T>(n, nb) > 160 * 1024) nb /= 2;
+  const size_t lds = factor_lds<T>(n, nb);
+  HZ_CHECK(lds <= 160 * 1024, HZ_ERR_ARG, "nx=%d too large for the LDS panel", n);
+  set_max_lds((const void*)&k_factor<T>, lds);
+  hipLaunchKernelGGL(k_factor<T>, dim3((unsigned)blocks), dim3(FACT_THREADS), lds, s, f.G.as<C>(), plane_tabs(p), n,
+                     (int)p->ny, nb, st, p->d_splane.as<int>(), mode, m, f.Gb.as<C>(), jbeg, jend);
+  HZ_HIP(hipGetLastError());
+}
+
+void run_factor(hz_problem* p, int prec, int blocks, int* st, int mode, int m, int jbeg, int jend, hipStream_t s) {
+  Factors& f = p->fac[prec];
+  if (launch_factor_reg(p, prec, plane_tabs(p), blocks, st, mode, m, f.G.ptr, f.Gb.ptr, jbeg, jend, s)) return;
+  if (prec == HZ_PREC_FP64) run_factor_mem<double>(p, prec, blocks, st, mode, m, jbeg, jend, s);
+  else run_factor_mem<float>(p, prec, blocks, st, mode, m, jbeg, jend, s);
+}
+
 }  // namespace
 
 void factor_begin(hz_problem* p, int prec, hipStream_t s) {
@@ -3076,31 +3064,11 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   p->pin_misc.reserve(64);
   *p->pin_misc.as<int>() = -1;
   launch_fill(1, make_double2(0, 0), dscal(p, 63), s);
-  PlaneTabs tb = plane_tabs(p);
-  int nb = 32;
-  if (prec == HZ_PREC_FP64) {
-    while (nb > 4 && factor_lds<double>(n, nb) > 160 * 1024) nb /= 2;
-    const size_t lds = factor_lds<double>(n, nb);
-    HZ_CHECK(lds <= 160 * 1024, HZ_ERR_ARG, "nx=%d too large for the LDS panel", n);
-    set_max_lds((const void*)&k_factor<double>, lds);
-    if (p->nslot > 0)
-      hipLaunchKernelGGL(k_factor<double>, dim3((unsigned)p->nslot), dim3(FACT_THREADS), lds, s, f.G.as<double2>(),
-                         tb, n, ny, nb, st, p->d_splane.as<int>(), 0, 0, (double2*)nullptr, 0, ny);
-  } else {
-    while (nb > 4 && factor_lds<float>(n, nb) > 160 * 1024) nb /= 2;
-    const size_t lds = factor_lds<float>(n, nb);
-    HZ_CHECK(lds <= 160 * 1024, HZ_ERR_ARG, "nx=%d too large for the LDS panel", n);
-    set_max_lds((const void*)&k_factor<float>, lds);
-    if (p->nslot > 0) {
-      // with the twisted factors the top-down chain stops at tw_m - 1 (the
-      // rest is completed on the first use of a one-directional kernel)
-      hipLaunchKernelGGL(k_factor<float>, dim3((unsigned)(twist ? 2 * p->nslot : p->nslot)), dim3(FACT_THREADS), lds,
-                         s, f.G.as<float2>(), tb, n, ny, nb, st, p->d_splane.as<int>(), twist ? 1 : 0, f.tw_m,
-                         f.Gb.as<float2>(), 0, f.top_full ? ny : f.tw_m);
-      if (twist)
-        hipLaunchKernelGGL(k_factor<float>, dim3((unsigned)p->nslot), dim3(FACT_THREADS), lds, s, f.G.as<float2>(), tb,
-                           n, ny, nb, st, p->d_splane.as<int>(), 2, f.tw_m, f.Gb.as<float2>(), 0, 0);
-    }
+  // with the twisted factors the top-down chain stops at tw_m - 1 (the rest is
+  // completed on the first use of a one-directional kernel)
+  if (p->nslot > 0) {
+    run_factor(p, prec, twist ? 2 * p->nslot : p->nslot, st, twist ? 1 : 0, f.tw_m, 0, f.top_full ? ny : f.tw_m, s);
+    if (twist) run_factor(p, prec, p->nslot, st, 2, f.tw_m, 0, 0, s);
   }
   HZ_HIP(hipGetLastError());
   HZ_HIP(hipMemcpyAsync(p->pin_misc.ptr, st, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -3150,12 +3118,7 @@ void ensure_dense(hz_problem* p, int prec, hipStream_t s) {
   int* st = reinterpret_cast<int*>(dscal(p, 63));
   *p->pin_misc.as<int>() = -1;
   launch_fill(1, make_double2(0, 0), dscal(p, 63), s);
-  int nb = 32;
-  while (nb > 4 && factor_lds<float>(n, nb) > 160 * 1024) nb /= 2;
-  const size_t lds = factor_lds<float>(n, nb);
-  if (p->nslot > 0)
-    hipLaunchKernelGGL(k_factor<float>, dim3((unsigned)p->nslot), dim3(FACT_THREADS), lds, s, f.G.as<float2>(),
-                       plane_tabs(p), n, ny, nb, st, p->d_splane.as<int>(), 0, f.tw_m, (float2*)nullptr, f.tw_m, ny);
+  if (p->nslot > 0) run_factor(p, prec, p->nslot, st, 0, f.tw_m, f.tw_m, ny, s);
   HZ_HIP(hipGetLastError());
   HZ_HIP(hipMemcpyAsync(p->pin_misc.ptr, st, sizeof(int), hipMemcpyDeviceToHost, s));
   HZ_HIP(hipStreamSynchronize(s));
