@@ -290,7 +290,8 @@ def plane_solve_kernel(nx, tuning):
     """Name of the complex64 single-RHS plane-solve kernel the tuned choice launches."""
     fam = tuning.get("solve_kernel", 0)
     if fam == 6:
-        return "k_solve_twist_pw<%d, 0> + k_solve_twist_pw<%d, 1>" % (nx, nx)
+        nt = (nx + 15) // 16
+        return "k_solve_tri<%d, 0, false> + k_solve_tri<%d, 1, false>" % (nt, nt)
     if fam == 5:
         return "k_solve_sym2<%d, false>" % nx
     if fam == 3:
@@ -535,8 +536,7 @@ def bench_config2(a, hz, np, torch, steps, warmup):
 def traffic_source(n, fam):
     """Where roofline.traffic comes from: it is not measured in this run (the
     counter passes need rocprofv3), it is read from the committed summary."""
-    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md",
-             6: "k_solve_twist_c64_200cube_pmc.md"}
+    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md"}
     if n != 200 or fam not in names or not os.path.exists(os.path.join(ROOT, "profiles", names[fam])):
         return None
     return "committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary profiles/%s (not measured in this run)" % names[fam]
@@ -546,13 +546,15 @@ def plane_solve_bytes(dims, fam, nslot):
     """Algorithmic HBM bytes of one complex64 single-RHS plane solve: 2 ny - 1
     block reads per plane (the full nx^2 block, or for the symmetric kernel the
     upper block triangle of 8x8 tiles, 64 T (T+1)/2 entries with T = nx/8; the
-    twisted solve reads 2 ny packed blocks per factor slot for both of its
-    planes: ny - 1 in phase 0, ny + 1 in phase 1) and four passes over the
-    nx ny nz vector."""
+    twisted solve reads 2 ny packed blocks of 16x16 tiles, 256 T (T+1)/2
+    entries with T = nx/16 rounded up, per factor slot for both of its planes:
+    ny - 1 in phase 0, ny + 1 in phase 1) and four passes over the nx ny nz
+    vector."""
     nx, ny, nz = dims
     if fam in (5, 6):
-        t = nx // 8
-        blk = 64 * t * (t + 1) // 2
+        b = 8 if fam == 5 else 16
+        t = -(-nx // b)
+        blk = b * b * t * (t + 1) // 2
     else:
         blk = nx * nx
     blocks = 2 * ny * nslot if fam == 6 else (2 * ny - 1) * nz
@@ -562,8 +564,7 @@ def plane_solve_bytes(dims, fam, nslot):
 def measured_traffic(n, fam):
     """HBM bytes per launch of the plane solve from the committed rocprofv3
     FETCH_SIZE/WRITE_SIZE passes (scaled by a 1 GiB copy), for the 200^3 grid."""
-    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md",
-             6: "k_solve_twist_c64_200cube_pmc.md"}
+    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md"}
     if n != 200 or fam not in names:
         return None
     path = os.path.join(ROOT, "profiles", names[fam])

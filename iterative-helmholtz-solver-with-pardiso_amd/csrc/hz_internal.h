@@ -103,8 +103,9 @@ struct Factors {
   DevBuf Gsym;
   // twisted factors (complex64): blocks j < tw_m the top-down inverses, block
   // tw_m the middle inverse, blocks j > tw_m the bottom-up inverses (Gb, dense,
-  // [slot][j - tw_m]), packed like Gsym into Gtw; tw_scr passes y_top, y_bot and
-  // f_m between the two phases (3 x TW_RHS x nz x nx complex64)
+  // [slot][j - tw_m]), the upper triangles of their symmetric forms packed in
+  // 16 x 16 tiles into Gtw; tw_scr passes y_top, y_bot and f_m between the two
+  // phases (3 x TW_RHS x nz x nx complex64)
   bool tw_ready = false;
   int tw_m = 0;
   // the top-down chain G_j is complete for every j (with the twisted factors

@@ -1322,12 +1322,11 @@ struct SymLayout {
   static_assert(NX % TB == 0, "tile split");
 };
 
-// P[(s ny + j) BS + ...] = packed X_j D_j of factor slot s, X_j = G_j; with
-// G2 (the twisted factors) X_j = G2[s][j - m] for j >= m
+// P[(s ny + j) BS + ...] = packed G_j D_j of factor slot s
 template <typename C, int NX, int TB>
 __global__ __launch_bounds__(256) void k_pack_sym(const C* __restrict__ G, C* __restrict__ P,
                                                   const double2* __restrict__ dx, const double2* __restrict__ dy,
-                                                  int ny, const C* __restrict__ G2, int m) {
+                                                  int ny) {
   typedef SymLayout<NX, TB> L;
   const int blk = blockIdx.y;
   const int j = blk % ny;
@@ -1336,7 +1335,7 @@ __global__ __launch_bounds__(256) void k_pack_sym(const C* __restrict__ G, C* __
   const bool two = J2 != J1;
   const int H1 = (J1 + 1) * TB, H2 = (J2 + 1) * TB;
   const int sz = H1 * TB + (two ? H2 * TB : 0);
-  const C* Gb = (G2 && j >= m) ? G2 + ((size_t)(blk / ny) * (ny - m) + (j - m)) * NX * NX : G + (size_t)blk * NX * NX;
+  const C* Gb = G + (size_t)blk * NX * NX;
   C* Pb = P + (size_t)blk * L::BS + (size_t)t * L::PAIR;
   const double2 dyj = dy[j];
   for (int e = threadIdx.x; e < sz; e += blockDim.x) {
@@ -1743,454 +1742,6 @@ __global__ __launch_bounds__(dma::NT) void k_solve_sym2(const float2* __restrict
     }
   }
   __builtin_amdgcn_s_waitcnt(dma::wait_vm(0));
-}
-
-// lane l ^ 16 and lane l ^ 32 of a wave (gfx950 permlane swaps)
-__device__ __forceinline__ float xor16_f(float x, int lane) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
-}
-__device__ __forceinline__ float xor32_f(float x, int lane) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 32) ? r[0] : r[1]);
-}
-// ---- twisted packed solve of both planes of a factor slot
-// Planes k and nz - k share a factor slot.  The twisted factors split every
-// slot's chain at m: blocks j < m hold the top-down inverses G_j, block m
-// T_m = (D_m - sig_m G_{m-1} - sig_{m+1} B_{m+1})^{-1} and blocks j > m the
-// bottom-up inverses B_j = (D_j - sig_{j+1} B_{j+1})^{-1} (sig_j = cm_y(j)
-// cp_y(j-1)), all packed like the forward factors.  Phase 0 (forward):
-//   top:    t_0 = f_0, t_j = f_j - cm_y(j) G_{j-1} t_{j-1} (0 < j < m), y_top = G_{m-1} t_{m-1}
-//   bottom: b_{ny-1} = f_{ny-1}, b_j = f_j - cp_y(j) B_{j+1} b_{j+1} (m < j < ny-1), y_bot = B_{m+1} b_{m+1}
-// Phase 1 (backward):
-//   x_m = T_m (f_m - cm_y(m) y_top - cp_y(m) y_bot),
-//   top x_j = G_j (t_j - cp_y(j) x_{j+1}) down to j = 0, bottom x_j = B_j (b_j - cm_y(j) x_{j-1}) up to ny-1.
-// One workgroup per (slot, half) carries both planes of the slot: every packed
-// tile is read once for two right-hand sides and 2 nslot workgroups walk
-// chains of about ny/2 blocks (the one-plane kernel: nz workgroups, 2 ny - 1
-// blocks).  y_top, y_bot and a copy of f_m pass between the phases in scr
-// (phase 1 writes x_m into line m, which the other half reads as f_m).
-//
-// Waves: wave (cg, rb), cg = wave % 4, rb = 64 (wave / 4), takes columns
-// 2cg, 2cg + 1 of both block columns of a tile pair (J1 = t, J2 = T - 1 - t)
-// and row units rb .. rb + 63 (a unit is two rows of one column).  Both
-// products run on the matrix cores (v_mfma_f32_4x4x1f32: 16 blocks of 4x4x1;
-// D(lane 4b+j, reg i) += A(lane 4b+i) B(lane 4b+j)).  The four real columns
-// of every product are the two planes' real and imaginary parts, so no block
-// column idles:
-//   direct, y_r += K(r, c) v'_c: lane l holds row unit rb + l (rows 2(rb+l)
-//     and 2(rb+l)+1); A = Re or Im K of one of those rows, B = the components
-//     of v'_c, so D(lane 4b+j, reg i) is row 2(rb+4b+i) (+1), component j,
-//     accumulated over the step's tiles;
-//   transposed, y_c += K(r, c) v'_r (rows above the diagonal tile): lane 4b+j
-//     holds (row unit rb+16k+b, column c_j) of the wave's four columns;
-//     A = the components of v'_r, B = Re or Im K, so D(lane 4b+j, reg i) sums
-//     block b's rows for column c_j, component i, and is reduced over the 16
-//     blocks at the end of the tile.
-// Components: 0, 1 = Re, Im of plane A; 2, 3 = Re, Im of plane B.  Im K
-// multiplies the rotated components (-Im A, Re A, -Im B, Re B).
-//
-// Tile rings: each wave moves exactly the part of every tile pair that it
-// reads into a ring of its own, so tiles need no barrier: a wave waits for its
-// own transfers only, and the workgroup meets twice per block step (partial
-// sums, then the new right-hand side).  Slot layouts (16-byte units; segments
-// 68 units apart, so the transposed reads of four columns fall in distinct
-// 4-bank groups):
-//   rb = 0:  [0, Hu1), [68, 68 + Hu1)   columns 2cg, 2cg + 1 of J1
-//            [136, 200), [204, 268)    columns 2cg, 2cg + 1 of J2, row units
-//                                      0 .. min(64, Hu2); unit 272 holds zeros
-//   rb = 64: [0, 64), [68, 132)        columns 2cg, 2cg + 1 of J2, row units
-//                                      64 .. Hu2; unit 136 holds zeros
-// (Hu = 4 (J + 1) stored row units of block column J.)  Every tile costs a
-// fixed number of transfers per wave (4, or 2 for rb = 64; lanes past a
-// segment repeat its last unit, tiles without rows for the wave repeat the
-// tile's first unit), so the vmcnt waits count tiles exactly.  The waves of
-// rb = 64 hold no row of J1 (Hu1 <= 64) and skip the tiles whose J2 rows end
-// before unit 64.
-template <int NX, int PH>
-__global__ __launch_bounds__(dma::NT) void k_solve_twist_pw(const float2* __restrict__ P, float2* __restrict__ X,
-                                                            const double2* __restrict__ cmy,
-                                                            const double2* __restrict__ cpy,
-                                                            const double2* __restrict__ symd, int ny, int m, int nz,
-                                                            int64_t n2, int64_t N, const int2* __restrict__ slotp,
-                                                            float2* __restrict__ scr) {
-  typedef float T;
-  typedef float2 C;
-  typedef float4 U;
-  constexpr int RPL = 2, NCG = 4, TB = 8;
-  typedef SymLayout<NX, TB> L;
-  constexpr int n = NX, T_ = L::T, TPS = L::TPS, PAIR = L::PAIR, BS = L::BS;
-  constexpr int PU = n * (int)sizeof(C) / 16;  // units of one y-line
-  constexpr int NW = 5;                        // ring slots per wave
-  // column segments of a slot start at units 0, 68, 136, 204 (distinct
-  // 4-bank groups: the transposed reads of four columns are conflict-free);
-  // the zero unit of a slot is its last unit
-  constexpr int SEG = 68;
-  constexpr int SLO = 273, SHI = 137;          // units per slot (rb = 0, rb = 64)
-  constexpr int LLO = 4, LHI = 2;              // transfers per tile
-  constexpr bool HAS_HI = n / RPL > 64;
-  // transposed blocks of the second row half that can hold a stored row
-  constexpr int KT64 = 4 * (T_ - 1) <= 64 ? 0 : (4 * (T_ - 1) - 64 + 15) / 16;
-  static_assert(n / RPL <= 128 && KT64 <= 4, "two row halves of 64 units");
-  static_assert(TPS * TB / RPL <= 64, "block column J1 lies in the first row half");
-  static_assert(NW <= TPS && TPS * LLO <= 63, "vmcnt range");
-  static_assert(PU <= 128, "line DMA of two waves per plane");
-  static_assert(2 * n <= dma::NT, "one thread per plane and row in the step epilogue");
-  static_assert((size_t)(4 * NW * (SLO + SHI) + (NCG + 2 + 2) * n + 5 * 64) * 16 + n * 8 <= 160 * 1024,
-                "LDS budget");
-  __shared__ U ring[4 * NW * SLO + 4 * NW * SHI];
-  __shared__ U part[NCG * n];   // direct products per column group
-  __shared__ U tdot[2 * n];     // transposed products per row half
-  __shared__ U vq[n], vqr[n];   // v' components and rotated components
-  __shared__ U pbuf[5 * 64];    // lines of planes A (units 0..127) and B (128..255); coefficients at 256..319
-  __shared__ C sdxi[n];
-  const double2* pscal = reinterpret_cast<const double2*>(&pbuf[256]);
-  const T* vqf = reinterpret_cast<const T*>(vq);
-  const T* vqrf = reinterpret_cast<const T*>(vqr);
-  T* tdf = reinterpret_cast<T*>(tdot);
-  T* pf = reinterpret_cast<T*>(part);
-
-  const int slot = blockIdx.x >> 1, half = blockIdx.x & 1;
-  const int2 sp = slotp[slot];
-  const bool twoB = sp.y >= 0;
-  const int pl0 = __builtin_amdgcn_readfirstlane(sp.x);
-  const int pl1 = __builtin_amdgcn_readfirstlane(twoB ? sp.y : sp.x);
-  const int64_t rhs = blockIdx.y;
-  const int nrhs = gridDim.y;
-  C* const xs0 = X + rhs * N + (int64_t)pl0 * n2;
-  C* const xs1 = X + rhs * N + (int64_t)pl1 * n2;
-  auto xs = [&](int s) { return s ? xs1 : xs0; };
-  // scr: [what][rhs][plane][n], what = 0 y_top, 1 y_bot, 2 f_m
-  auto scr_at = [&](int what, int s) { return scr + (((int64_t)what * nrhs + rhs) * nz + (s ? pl1 : pl0)) * n; };
-  const C* Pk = P + (size_t)slot * ny * BS;
-  const double2* dxi = symd + n + ny;
-  const double2* dyi = symd + 2 * n + ny;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cg = wv % NCG;
-  const int bq = lane >> 2, jq = lane & 3;  // the lane's MFMA block and index in the block
-  const int nsteps = PH == 0 ? (half == 0 ? m : ny - 1 - m) : (half == 0 ? m + 1 : ny - m);
-  auto blk_of = [&](int st) {
-    if (PH == 0) return half == 0 ? st : ny - 1 - st;
-    return half == 0 ? m - st : m + st;
-  };
-  // block whose vector the update after step st forms (-1: none; -2: y goes to scr)
-  auto next_of = [&](int st) {
-    const int jb = blk_of(st);
-    if (PH == 0) {
-      if (half == 0) return jb + 1 < m ? jb + 1 : -2;
-      return jb - 1 > m ? jb - 1 : -2;
-    }
-    if (half == 0) return jb > 0 ? jb - 1 : -1;
-    return jb < ny - 1 ? jb + 1 : -1;
-  };
-  const unsigned ring_lds = (unsigned)(size_t)(&ring[0]);
-  const unsigned pbuf_lds = (unsigned)(size_t)(&pbuf[0]);
-
-  if (PH == 0 && half == 0) {
-    // f_m for phase 1 (phase 1 overwrites line m with x_m)
-    for (int i = tid; i < 2 * n; i += dma::NT) {
-      const int s = i / n, c = i - s * n;
-      if (s == 0 || twoB) scr_at(2, s)[c] = xs(s)[(size_t)m * n + c];
-    }
-  }
-  if (nsteps <= 0) return;
-  for (int i = tid; i < 2 * n; i += dma::NT) tdot[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (tid < 8 * NW) {
-    const int w = tid / NW, s = tid - w * NW;
-    const int z = w < 4 ? (w * NW + s) * SLO + SLO - 1 : 4 * NW * SLO + ((w - 4) * NW + s) * SHI + SHI - 1;
-    ring[z] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  for (int i = tid; i < n; i += dma::NT) {
-    const double2 a = dxi[i];
-    sdxi[i] = make_float2((T)a.x, (T)a.y);
-  }
-  __syncthreads();
-  {
-    const int j0 = blk_of(0);
-    const double2 dy0 = dyi[j0];
-    for (int c = tid; c < n; c += dma::NT) {
-      T w[4];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        double fx, fy;
-        if (PH == 0) {
-          const C f = xs(s)[(size_t)j0 * n + c];
-          fx = f.x;
-          fy = f.y;
-        } else {
-          // f_m - cm_y(m) y_top - cp_y(m) y_bot
-          const C f = scr_at(2, s)[c];
-          fx = f.x;
-          fy = f.y;
-          if (m > 0) {
-            const C yt = scr_at(0, s)[c];
-            const double2 cm = cmy[m];
-            fx -= cm.x * yt.x - cm.y * yt.y;
-            fy -= cm.x * yt.y + cm.y * yt.x;
-          }
-          if (m < ny - 1) {
-            const C yb = scr_at(1, s)[c];
-            const double2 cp = cpy[m];
-            fx -= cp.x * yb.x - cp.y * yb.y;
-            fy -= cp.x * yb.y + cp.y * yb.x;
-          }
-        }
-        const C a = sdxi[c];
-        const double dx = (double)a.x * dy0.x - (double)a.y * dy0.y, dy = (double)a.x * dy0.y + (double)a.y * dy0.x;
-        w[2 * s] = (T)(fx * dx - fy * dy);
-        w[2 * s + 1] = (T)(fx * dy + fy * dx);
-      }
-      vq[c] = make_float4(w[0], w[1], w[2], w[3]);
-      vqr[c] = make_float4(-w[1], w[0], -w[3], w[2]);
-    }
-  }
-  __syncthreads();
-
-  auto blk_addr = [&](int st) {
-    return reinterpret_cast<const char*>(Pk + (size_t)blk_of(st < nsteps ? st : 0) * BS);
-  };
-  const hz_v4f z4 = {0.f, 0.f, 0.f, 0.f};
-
-  auto run = [&](auto hi_tag) {
-    constexpr bool HI = decltype(hi_tag)::value;
-    constexpr int SZ = HI ? SHI : SLO, ZU = SZ - 1, LD = HI ? LHI : LLO;
-    constexpr int rb = HI ? 64 : 0, q2 = HI ? 1 : 0;
-    const int wq = HI ? wv - 4 : wv;
-    const int wbase = HI ? 4 * NW * SLO + wq * NW * SHI : wq * NW * SLO;
-    const U* WR = ring + wbase;
-    const unsigned wr_lds = ring_lds + (unsigned)wbase * 16u;
-    const int ca = cg * 2;
-    // the wave's transfers of tile tt of a block into ring slot sl
-    auto tile_dma = [&](const char* blk, int tt, int sl) {
-      const int J1 = tt, J2 = T_ - 1 - tt;
-      const bool two = J2 != J1;
-      const int Hu1 = (J1 + 1) * TB / RPL, Hu2 = (J2 + 1) * TB / RPL;
-      const int ub2 = (J1 + 1) * TB * TB / RPL;
-      const char* base = blk + (size_t)tt * PAIR * sizeof(C);
-      const unsigned dst = wr_lds + (unsigned)(sl * SZ) * 16u;
-      int u[LD];
-      if (!HI) {
-        const int L2 = Hu2 < 64 ? Hu2 : 64;
-        u[0] = ca * Hu1 + min(lane, Hu1 - 1);
-        u[1] = (ca + 1) * Hu1 + min(lane, Hu1 - 1);
-        u[2] = two ? ub2 + ca * Hu2 + min(lane, L2 - 1) : 0;
-        u[3] = two ? ub2 + (ca + 1) * Hu2 + min(lane, L2 - 1) : 0;
-      } else {
-        const bool has = two && Hu2 > 64;
-        u[0] = has ? ub2 + ca * Hu2 + 64 + min(lane, Hu2 - 65) : 0;
-        u[1] = has ? ub2 + (ca + 1) * Hu2 + 64 + min(lane, Hu2 - 65) : 0;
-      }
-#pragma unroll
-      for (int i = 0; i < LD; ++i) dma16_untracked(base + (size_t)u[i] * 16, dst + (unsigned)(i * SEG * 16));
-    };
-#pragma unroll
-    for (int g = 0; g < NW; ++g) tile_dma(blk_addr(0), g, g);
-
-    hz_v4f dE1 = z4, dO1 = z4, dE2 = z4, dO2 = z4;  // direct: even / odd rows, block columns J1 / J2
-    T va[4][2], vr[4][2];                          // transposed A operands of the step
-    int rslot = 0;
-    for (int st = 0; st < nsteps; ++st) {
-      const char* b0 = blk_addr(st);
-      const char* b1 = blk_addr(st + 1);
-      const int jb = blk_of(st), jn = next_of(st);
-#pragma unroll
-      for (int t = 0; t < TPS; ++t) {
-        // this tile's transfers are complete once at most the NW - 1 younger
-        // tiles' transfers are outstanding
-        __builtin_amdgcn_s_waitcnt(dma::wait_vm((NW - 1) * LD));
-        asm volatile("" ::: "memory");
-        const U* SL = WR + rslot * SZ;
-        if (t == 0) {
-          dE1 = z4;
-          dO1 = z4;
-          dE2 = z4;
-          dO2 = z4;
-          // rows 2 (rb + 16 k + b) + e of the transposed products, component i
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-              const int row = 2 * (rb + 16 * k + bq) + e;
-              const int ix = (row < n ? row : 0) * 4 + jq;
-              va[k][e] = row < n ? vqf[ix] : 0.f;
-              vr[k][e] = row < n ? vqrf[ix] : 0.f;
-            }
-          // the lines of this step's update (waves 0-1 plane A, 2-3 plane B)
-          // and its coefficients (wave 4: coupling, 1/dy of the next block)
-          if (jn >= 0) {
-            if (!HI) {
-              const int s = wv >> 1;
-              const char* lb = reinterpret_cast<const char*>(xs(s) + (size_t)jn * n);
-              dma16_untracked(lb + (size_t)min((wv & 1) * 64 + lane, PU - 1) * 16,
-                              pbuf_lds + (unsigned)(wv * 64 * 16));
-            } else if (wv == 4) {
-              const double2* src;
-              if (lane == 1) src = dyi + jn;
-              else src = (PH == 0 ? (half == 0) : (half != 0)) ? cmy + jn : cpy + jn;
-              dma16_untracked(src, pbuf_lds + 256 * 16);
-            }
-          }
-        }
-        {
-          const int J1 = t, J2 = T_ - 1 - t;
-          const int Hu1 = (J1 + 1) * TB / RPL, Hu2 = (J2 + 1) * TB / RPL;
-          const int nu1 = J1 * TB / RPL, nu2 = J2 * TB / RPL;
-          const bool two = J2 != J1;
-          if (!HI || (HAS_HI && two && Hu2 > 64)) {
-            constexpr int KT = HI ? KT64 : 4;
-            // ---- the tile's operands
-            // direct: lane = row unit rb + lane; transposed: lane (b, j) <->
-            // (row unit rb + 16 k + b, column c_j)
-            U a1[2], a2[2], uu[4];
-            T bv1[2], br1[2], bv2[2], br2[2];
-            const bool lo = jq < 2;
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-              if (!HI) {
-                a1[cc] = SL[lane < Hu1 ? cc * SEG + lane : ZU];
-                a2[cc] = SL[two && lane < Hu2 ? (2 + cc) * SEG + lane : ZU];
-                const int c1 = (J1 * TB + ca + cc) * 4 + jq;
-                bv1[cc] = vqf[c1];
-                br1[cc] = vqrf[c1];
-              } else {
-                a2[cc] = SL[lane < Hu2 - 64 ? cc * SEG + lane : ZU];
-              }
-              if (two) {
-                const int c2 = (J2 * TB + ca + cc) * 4 + jq;
-                bv2[cc] = vqf[c2];
-                br2[cc] = vqrf[c2];
-              }
-            }
-#pragma unroll
-            for (int k = 0; k < KT; ++k) {
-              const int rk = rb + 16 * k + bq;
-              int ix;
-              if (!HI) ix = lo ? (rk < nu1 ? jq * SEG + rk : ZU) : (two && rk < nu2 ? jq * SEG + rk : ZU);
-              else ix = !lo && rk < nu2 ? (jq - 2) * SEG + rk - 64 : ZU;
-              uu[k] = SL[ix];
-            }
-            // ---- direct products
-            if (!HI) {
-#pragma unroll
-              for (int cc = 0; cc < 2; ++cc) {
-                dE1 = __builtin_amdgcn_mfma_f32_4x4x1f32(a1[cc].x, bv1[cc], dE1, 0, 0, 0);
-                dO1 = __builtin_amdgcn_mfma_f32_4x4x1f32(a1[cc].z, bv1[cc], dO1, 0, 0, 0);
-                dE1 = __builtin_amdgcn_mfma_f32_4x4x1f32(a1[cc].y, br1[cc], dE1, 0, 0, 0);
-                dO1 = __builtin_amdgcn_mfma_f32_4x4x1f32(a1[cc].w, br1[cc], dO1, 0, 0, 0);
-              }
-            }
-            if (two) {
-#pragma unroll
-              for (int cc = 0; cc < 2; ++cc) {
-                dE2 = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[cc].x, bv2[cc], dE2, 0, 0, 0);
-                dO2 = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[cc].z, bv2[cc], dO2, 0, 0, 0);
-                dE2 = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[cc].y, br2[cc], dE2, 0, 0, 0);
-                dO2 = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[cc].w, br2[cc], dO2, 0, 0, 0);
-              }
-            }
-            if (KT > 0) {
-              // ---- transposed products
-              hz_v4f tA = z4, tB = z4;
-#pragma unroll
-              for (int k = 0; k < KT; ++k) {
-                tA = __builtin_amdgcn_mfma_f32_4x4x1f32(va[k][0], uu[k].x, tA, 0, 0, 0);
-                tB = __builtin_amdgcn_mfma_f32_4x4x1f32(vr[k][0], uu[k].y, tB, 0, 0, 0);
-                tA = __builtin_amdgcn_mfma_f32_4x4x1f32(va[k][1], uu[k].z, tA, 0, 0, 0);
-                tB = __builtin_amdgcn_mfma_f32_4x4x1f32(vr[k][1], uu[k].w, tB, 0, 0, 0);
-              }
-              // sum over the 16 blocks (lane bits 2..5): afterwards lane l holds
-              // component (l >> 2) & 3 of column c_(l & 3)
-              const T w0 = pair_step<0x124>(tA[0] + tB[0], tA[1] + tB[1], lane & 4);
-              const T w1 = pair_step<0x124>(tA[2] + tB[2], tA[3] + tB[3], lane & 4);
-              T sm = pair_step<0x128>(w0, w1, lane & 8);
-              sm += xor16_f(sm, lane);
-              sm += xor32_f(sm, lane);
-              if (lane < 16 && (jq < 2 || two)) {
-                const int col = (jq < 2 ? J1 : J2) * TB + ca + (jq & 1);
-                tdf[(q2 * n + col) * 4 + ((lane >> 2) & 3)] = sm;
-              }
-            }
-          }
-        }
-        {
-          // the tile NW stages ahead into this slot once its reads are done
-          __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);
-          asm volatile("" ::: "memory");
-          const int ta = t + NW;
-          const int tt = ta % TPS;
-          const char* blk = (ta / TPS) == 0 ? b0 : b1;
-          const bool past = (ta / TPS) != 0 && st + 1 >= nsteps;
-          tile_dma(past ? reinterpret_cast<const char*>(Pk) : blk, tt, rslot);
-        }
-        rslot = rslot + 1 == NW ? 0 : rslot + 1;
-        if (t == TPS - 1) {
-          {
-            // direct partials: lane 4b+j, reg i = rows 2(rb+4b+i), +1, component j
-            const hz_v4f dE = dE1 + dE2, dO = dO1 + dO2;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int row = 2 * (rb + 4 * bq + i);
-              if (row < n) {
-                pf[(cg * n + row) * 4 + jq] = dE[i];
-                pf[(cg * n + row + 1) * 4 + jq] = dO[i];
-              }
-            }
-          }
-          // the step's line transfers precede its TPS tiles' transfers
-          __builtin_amdgcn_s_waitcnt(dma::wait_vm(TPS * LD));
-          __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);
-          dma::raw_barrier();
-          // one thread per (plane, row): the plane's partial sums, the
-          // update of the next right-hand side and the stores
-          if (tid < 2 * n) {
-            const int s = tid >= n ? 1 : 0, r = tid - s * n;
-            const C* part2 = reinterpret_cast<const C*>(part);
-            const C* tdot2 = reinterpret_cast<const C*>(tdot);
-            C ys = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int q = 0; q < NCG; ++q) {
-              const C u = part2[(q * n + r) * 2 + s];
-              ys.x += u.x;
-              ys.y += u.y;
-            }
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-              const C u = tdot2[(q * n + r) * 2 + s];
-              ys.x += u.x;
-              ys.y += u.y;
-            }
-            const C a = sdxi[r];
-            const double2 cf = pscal[0], b = pscal[1];
-            const double2 di =
-                make_double2((double)a.x * b.x - (double)a.y * b.y, (double)a.x * b.y + (double)a.y * b.x);
-            const bool wr = s == 0 || twoB;
-            C* x = xs(s);
-            if (wr && PH == 1 && (half == 0 || st > 0)) x[(size_t)jb * n + r] = ys;  // x_jb
-            if (wr && jn == -2) scr_at(half, s)[r] = ys;                             // y_top / y_bot
-            if (jn >= 0) {
-              const C pre = reinterpret_cast<const C*>(pbuf + 128 * s)[r];
-              C nv;
-              nv.x = pre.x - (T)(cf.x * ys.x - cf.y * ys.y);
-              nv.y = pre.y - (T)(cf.x * ys.y + cf.y * ys.x);
-              if (wr && PH == 0) x[(size_t)jn * n + r] = nv;  // t_jn / b_jn
-              const T w0 = (T)((double)nv.x * di.x - (double)nv.y * di.y);
-              const T w1 = (T)((double)nv.x * di.y + (double)nv.y * di.x);
-              reinterpret_cast<C*>(vq)[r * 2 + s] = make_float2(w0, w1);
-              reinterpret_cast<C*>(vqr)[r * 2 + s] = make_float2(-w1, w0);
-            }
-          }
-          __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);
-          dma::raw_barrier();
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(dma::wait_vm(0));
-  };
-  if (wv < 4) run(std::false_type{});
-  else run(std::true_type{});
 }
 
 // ---- complex128 form of the step-unrolled packed solve
@@ -2761,58 +2312,9 @@ bool try_pack_sym(hz_problem* p, int prec, hipStream_t s, bool alloc_only) {
   const double2* dy = dx + NX;
   if (p->nslot == 0 || alloc_only) return true;
   hipLaunchKernelGGL((k_pack_sym<C, NX, TB>), dim3(L::TPS, (unsigned)(p->nslot * p->ny)), dim3(256), 0, s, f.G.as<C>(),
-                     f.Gsym.as<C>(), dx, dy, (int)p->ny, (const C*)nullptr, 0);
+                     f.Gsym.as<C>(), dx, dy, (int)p->ny);
   HZ_HIP(hipGetLastError());
   return true;
-}
-
-// the twisted factors (G for j < m, Gb from m on) packed like Gsym into Gtw
-template <int NX>
-bool try_pack_twist(hz_problem* p, hipStream_t s) {
-  if (p->nx != NX) return false;
-  typedef SymLayout<NX, 8> L;
-  Factors& f = p->fac[HZ_PREC_C64];
-  const size_t bytes = (size_t)p->nslot * p->ny * L::BS * sizeof(float2);
-  if (f.Gtw.bytes != bytes) {
-    f.Gtw.release();
-    f.Gtw.alloc(bytes);
-  }
-  const double2* dx = p->d_symd.as<double2>();
-  hipLaunchKernelGGL((k_pack_sym<float2, NX, 8>), dim3(L::TPS, (unsigned)(p->nslot * p->ny)), dim3(256), 0, s,
-                     f.G.as<float2>(), f.Gtw.as<float2>(), dx, dx + NX, (int)p->ny, f.Gb.as<float2>(), f.tw_m);
-  HZ_HIP(hipGetLastError());
-  return true;
-}
-
-bool pack_twist_any(hz_problem* p, hipStream_t s) {
-  return try_pack_twist<200>(p, s) || try_pack_twist<192>(p, s) || try_pack_twist<160>(p, s) ||
-         try_pack_twist<128>(p, s);
-}
-
-// both phases of the twisted solve, TW_RHS right-hand sides per launch pair
-template <int NX>
-bool try_solve_twist(hz_problem* p, int nrhs, void* x, hipStream_t s) {
-  if (p->nx != NX) return false;
-  const Factors& f = p->fac[HZ_PREC_C64];
-  const float2* P = f.Gtw.as<float2>();
-  const int2* sp = p->d_slotp.as<int2>();
-  float2* scr = f.tw_scr.as<float2>();
-  for (int r0 = 0; r0 < nrhs; r0 += TW_RHS) {
-    const int nr = std::min(TW_RHS, nrhs - r0);
-    float2* xr = reinterpret_cast<float2*>(x) + (size_t)r0 * p->N;
-    const dim3 grid((unsigned)(2 * p->nslot), (unsigned)nr);
-    hipLaunchKernelGGL((k_solve_twist_pw<NX, 0>), grid, dim3(dma::NT), 0, s, P, xr, p->tab(1, 0), p->tab(1, 1),
-                       p->d_symd.as<double2>(), (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N, sp, scr);
-    hipLaunchKernelGGL((k_solve_twist_pw<NX, 1>), grid, dim3(dma::NT), 0, s, P, xr, p->tab(1, 0), p->tab(1, 1),
-                       p->d_symd.as<double2>(), (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N, sp, scr);
-    HZ_HIP(hipGetLastError());
-  }
-  return true;
-}
-
-bool solve_twist_any(hz_problem* p, int nrhs, void* x, hipStream_t s) {
-  return try_solve_twist<200>(p, nrhs, x, s) || try_solve_twist<192>(p, nrhs, x, s) ||
-         try_solve_twist<160>(p, nrhs, x, s) || try_solve_twist<128>(p, nrhs, x, s);
 }
 
 template <int NX>
@@ -2951,15 +2453,30 @@ bool twist_solve_available(const hz_problem* p, int prec) {
 }
 
 namespace {
-// whether plane_solve_kernels takes the twisted solve for this call (the only
-// kernel that runs on an incomplete top-down chain)
-bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, const void* x) {
+// Whether plane_solve_kernels takes the twisted solve for this call (the only
+// kernel that runs on an incomplete top-down chain): where it is asked for or
+// tuned; untuned where no group kernel is built for the width, and otherwise
+// for up to 7 right-hand sides (3 above 160 columns).  One right-hand side,
+// best kernel of before -> twisted: 48^3 0.234 -> 0.083 ms, 64^3 0.167 ->
+// 0.117, 96^3 0.41 -> 0.21, 128^3 0.55 -> 0.34, 160^3 0.81 -> 0.71, 192^3 1.33
+// -> 1.23, 200^3 1.55 -> 1.53, 140 x 140 x 150 1.60 -> 0.55, 239 x 239 x 299
+// 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.12, 128^3 0.80 -> 0.35, 200^3 2.19 ->
+// 1.55.  Four right-hand sides against the group kernel: 128^3 1.00 against
+// 1.41, 160^3 2.09 against 2.47, 192^3 4.75 against 3.70.  Eight: 64^3 0.26
+// (group kernel) against about 0.32.
+// Under stream capture an untuned call also takes it while the top-down chain
+// is incomplete, which cannot be completed there.
+bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
   const Factors& f = p->fac[prec];
-  if (adjoint || prec != HZ_PREC_C64 || !f.tw_ready || reinterpret_cast<uintptr_t>(x) % 16 != 0) return false;
+  if (prec != HZ_PREC_C64 || !f.tw_ready) return false;
   const SolveKernel sk = solve_kernel_choice();
   if (sk == SK_TWIST) return true;
   if (sk != SK_DEFAULT) return false;
-  return t.solve_family == HZ_SOLVE_TWIST || (t.solve_family == HZ_SOLVE_DEFAULT && nrhs == 1);
+  if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
+  if (nrhs < (p->nx > 160 ? 4 : 8) || !mfma_solve_available(prec, (int)p->nx)) return true;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HZ_HIP(hipStreamIsCapturing(s, &cs));
+  return !f.top_full && cs != hipStreamCaptureStatusNone;
 }
 }  // namespace
 
@@ -3034,10 +2551,10 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   f.sym_ready = false;
   f.tw_ready = false;
   f.hodlr.release();
-  // twisted factors (complex64, the packed widths, at most two planes a slot):
+  // twisted factors (complex64, up to 256 columns, at most two planes a slot):
   // the bottom-up chain runs beside the top-down one in the same launch
-  const bool twist = prec == HZ_PREC_C64 && ny >= 2 && p->slot_pairs && sym_solve_available(prec, n) &&
-                     !getenv("HZ_NO_TWIST") && !getenv("HZ_NO_SYM_PACK");
+  const bool twist = prec == HZ_PREC_C64 && ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") &&
+                     !getenv("HZ_NO_SYM_PACK");
   f.tw_m = twist ? ny / 2 : 0;
   f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr;
   if (twist) {
@@ -3089,7 +2606,8 @@ void factor_end(hz_problem* p, int prec, hipStream_t s) {
   // twisted packed copy; the unpacked bottom-up blocks are not kept
   f.tw_ready = false;
   if (f.Gb.ptr && p->nslot > 0) {
-    f.tw_ready = pack_twist_any(p, s);
+    pack_tri(p, s);
+    f.tw_ready = true;
     const size_t sb = (size_t)3 * TW_RHS * p->nz * p->nx * sizeof(float2);
     if (f.tw_scr.bytes != sb) {
       f.tw_scr.release();
@@ -3179,7 +2697,11 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
     HZ_CHECK(f.G.ptr != nullptr, HZ_ERR_STATE,
              "adjoint plane solve: the dense factors were released by HZ_HODLR_FREE_DENSE");
   }
-  if (!f.top_full && !uses_twist(p, prec, nrhs, adjoint, t, x)) ensure_dense(p, prec, s);
+  if (uses_twist(p, prec, nrhs, adjoint, t, s)) {
+    solve_tri(p, nrhs, x, adjoint, s);
+    return;
+  }
+  if (!f.top_full) ensure_dense(p, prec, s);
   const int n = (int)p->nx, ny = (int)p->ny;
   const int ng = std::max(1, APPLY_THREADS / n);
   PlaneTabs tb = plane_tabs(p);
@@ -3210,13 +2732,9 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_STREAM_MFMA) sk = SK_MFMA;
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_SYM) sk = SK_SYM;
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_TWIST) sk = SK_TWIST;
-  // untuned default for one right-hand side: the twisted two-plane packed
-  // solve, else the symmetric packed stream, where they are built
-  if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_DEFAULT && nrhs == 1 && f.tw_ready) sk = SK_TWIST;
+  // untuned default for one right-hand side without twisted factors: the
+  // symmetric packed stream, where it is built
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_DEFAULT && nrhs == 1 && f.sym_ready) sk = SK_SYM;
-  if (!adjoint && sk == SK_TWIST && f.tw_ready && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-      solve_twist_any(p, nrhs, x, s))
-    return;
   if (sk == SK_TWIST) sk = SK_SYM;
   if (!adjoint && ny >= 1 && sk == SK_SYM && f.sym_ready && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
       solve_sym_any(p, prec, nrhs, x, false, s))

@@ -73,22 +73,29 @@ __device__ __forceinline__ double2 to_z(C v) {
 // Circle-method round robin over rr (even) columns: pair s of round t.
 __device__ __forceinline__ int rr_pos(int x, int t, int rr) { return x == 0 ? 0 : ((x - 1 + t) % (rr - 1)) + 1; }
 
-// K(r, c) of block b of the packed symmetric layout (the upper block triangle of
-// K = X D in 8 x 8 tiles, block columns J and T-1-J side by side, each holding
-// rows [0, 8 (J+1)) column-major; below that, K(r, c) = K(c, r))
+// K(r, c) of a packed block of the twisted factors (k_tri.hip: tile row R of T
+// keeps the tile columns R, R + 1, ... (mod T), rows w and w + (T + 1)/2
+// together; the diagonal tile its 4 x 4 blocks on and above the diagonal),
+// elsewhere K(r, c) = K(c, r)
 __device__ __forceinline__ size_t packed_at(int r, int c, int T) {
-  if (r / 8 > c / 8) {
-    const int t = r;
+  int R = r / 16, C = c / 16;
+  const int d = C >= R ? C - R : C - R + T, na = T / 2 + 1, nw = (T + 1) / 2;
+  if (d == 0 ? r / 4 > c / 4 : d >= (T % 2 != 0 || R < T / 2 ? na : na - 1)) {
+    int t = r;
     r = c;
     c = t;
+    t = R;
+    R = C;
+    C = t;
   }
-  const int J = c / 8, H = 8 * (J + 1);
-  const size_t base = J <= T - 1 - J ? (size_t)J * (T + 1) * 64 : (size_t)(T - 1 - J) * (T + 1) * 64 + (size_t)(T - J) * 64;
-  return base + (size_t)(c - 8 * J) * H + r;
+  const int e = C >= R ? C - R : C - R + T;
+  const int tile = R < nw ? R * (T + 1) + e : (R - nw) * (T + 1) + na + e;
+  const int lane = 16 * (c / 4 % 4) + 4 * (r / 4 % 4) + r % 4;
+  return ((size_t)(tile * 2 + c / 2 % 2) * 64 + lane) * 2 + c % 2;
 }
 
 // G: dense blocks ([rec] n x n, column-major; K = G D); with packed != 0 the
-// blocks are read from the packed symmetric form of K itself (n = 8 T)
+// blocks are read from the packed symmetric form of K itself (T tile rows)
 template <typename CIN>
 __global__ __launch_bounds__(HT) void k_hodlr_compress(const CIN* __restrict__ G, int packed, const double2* __restrict__ symd,
                                                        int n, int ny, int nrec, const int4* __restrict__ nodes, int nn,
@@ -122,8 +129,8 @@ __global__ __launch_bounds__(HT) void k_hodlr_compress(const CIN* __restrict__ G
 
   for (int rec = blockIdx.x; rec < nrec; rec += gridDim.x) {
     const int j = rec % ny;
-    const int T = n / 8;
-    const CIN* Gb = G + (size_t)rec * (packed ? (size_t)T * (T + 1) * 32 : (size_t)n * n);
+    const int T = (n + 15) / 16;
+    const CIN* Gb = G + (size_t)rec * (packed ? (size_t)T * (T + 1) * 128 : (size_t)n * n);
     CIN* Sb = stage + (size_t)rec * n * WS;
     const double2 dyj = dy[j];
     auto K = [&](int r, int c) {
@@ -1087,7 +1094,8 @@ void hodlr_compress(hz_problem* p, int prec, double eps, int small, int flags) {
   }
   const bool twisted = (flags & HZ_HODLR_TWISTED) != 0;
   if (twisted) {
-    HZ_CHECK(prec == HZ_PREC_C64 && f.ready && f.tw_ready && f.Gtw.ptr, HZ_ERR_STATE,
+    HZ_CHECK(prec == HZ_PREC_C64 && f.ready && f.tw_ready && f.Gtw.ptr && sym_solve_available(prec, (int)p->nx),
+             HZ_ERR_STATE,
              "twisted compression needs the twisted complex64 factors (widths 128, 160, 192, 200, ny >= 2)");
   } else {
     HZ_CHECK(f.ready && f.G.ptr, HZ_ERR_STATE, "compression needs the dense factors of precision %d", prec);

@@ -1,0 +1,70 @@
+"""The twisted complex64 plane solve (default for few right-hand sides, forward
+and adjoint) over the widths where its 16 x 16 tiles, its wave split (even and
+odd tile counts) and its chains have edges, against the CPU oracle."""
+import numpy as np
+import pytest
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def hz():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return load_pkg()
+
+
+def _rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def _case(hz, mode, nx, ny, nz):
+    pr = hz.problem
+    if mode == "s7":
+        d = pr.cube_geometry((nx, ny, nz), (min(4, (nx - 1) // 2), 0, 1 if nz > 2 else 0),
+                             pr.omega_for_ppw(0.8, 1.0 / max(nx, 8), 8), beta=0.5, pml_c=30.0)
+        return d, 0.8 + 0.4 * np.random.default_rng(nx + ny).random(d.N)
+    d = pr.ref_geometry(n_nopml=nx - 8, pml=4, spg=2, nz_nopml=nz - 4, length=(240.0,) * 3, homo=False)
+    d = d.replace(n=(nx, ny, nz), l=(d.l[0], d.l[0] * ny / nx, d.l[2]), h=(d.h[0], d.h[0], d.h[2]))
+    return d, pr.ref_sound_speed(d)
+
+
+# every tile count 1..16, on both sides of a tile edge or ragged; chains of 2
+# and 3 blocks and longer ones; single-plane slots (k = 0, nz / 2), odd nz
+CASES = [("s7", nx, ny, nz) for nx, ny, nz in (
+    (1, 3, 3), (7, 2, 4), (16, 5, 3), (17, 6, 4), (33, 3, 5), (48, 4, 4), (49, 7, 3), (65, 6, 4), (81, 5, 3), (100, 4, 4),
+    (112, 3, 3), (113, 6, 4), (130, 5, 3), (145, 4, 4), (161, 3, 3), (177, 5, 4), (193, 4, 3), (209, 3, 4), (223, 4, 3),
+    (225, 5, 3), (239, 4, 4), (256, 3, 3))] + [("ref", 30, 12, 9), ("ref", 77, 14, 8), ("ref", 139, 12, 7)]
+
+
+@pytest.mark.parametrize("mode,nx,ny,nz", CASES)
+def test_tri_vs_oracle(hz, oracle, mode, nx, ny, nz):
+    """One and three right-hand sides, forward and adjoint, through the
+    preconditioner: 1e-4, the complex64 preconditioner's bound elsewhere."""
+    print("case tri %s %d %d %d" % (mode, nx, ny, nz), flush=True)
+    d, c = _case(hz, mode, nx, ny, nz)
+    S, P = hz.Solver(d, c), oracle.Problem(d, c)
+    S.factor(hz.abi.PREC_C64)
+    rng = np.random.default_rng(nx)
+    x = rng.standard_normal((3, d.N)) + 1j * rng.standard_normal((3, d.N))
+    for adj in (False, True):
+        want = [P.precond_apply(v, adjoint=adj) for v in x]
+        for nrhs in (1, 3):
+            got = S.precond_apply(torch.from_numpy(x[:nrhs]).cuda(), hz.abi.PREC_C64, adjoint=adj).cpu().numpy()
+            for q in range(nrhs):
+                assert _rel(got[q], want[q]) < 1e-4, (adj, nrhs, q, _rel(got[q], want[q]))
+
+
+def test_tri_widths_past_the_tiles(hz, oracle):
+    """257 columns: no twisted factors, the one-directional kernels as before."""
+    d, c = _case(hz, "s7", 257, 3, 3)
+    S, P = hz.Solver(d, c), oracle.Problem(d, c)
+    S.factor(hz.abi.PREC_C64)
+    x = np.random.default_rng(1).standard_normal(d.N) + 0j
+    for adj in (False, True):
+        got = S.precond_apply(torch.from_numpy(x).cuda(), hz.abi.PREC_C64, adjoint=adj).cpu().numpy()
+        assert _rel(got, P.precond_apply(x, adjoint=adj)) < 1e-4
