@@ -2449,31 +2449,34 @@ bool sym_solve_available(int prec, int nx) {
 }
 
 bool twist_solve_available(const hz_problem* p, int prec) {
-  return prec == HZ_PREC_C64 && p->fac[prec].tw_ready;
+  return p->fac[prec].tw_ready;
 }
 
 namespace {
 // Whether plane_solve_kernels takes the twisted solve for this call (the only
 // kernel that runs on an incomplete top-down chain): where it is asked for or
-// tuned; untuned where no group kernel is built for the width, and otherwise
-// for up to 7 right-hand sides (3 above 160 columns).  One right-hand side,
-// best kernel of before -> twisted: 48^3 0.234 -> 0.083 ms, 64^3 0.167 ->
-// 0.117, 96^3 0.41 -> 0.21, 128^3 0.55 -> 0.34, 160^3 0.81 -> 0.71, 192^3 1.33
-// -> 1.23, 200^3 1.55 -> 1.53, 140 x 140 x 150 1.60 -> 0.55, 239 x 239 x 299
-// 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.12, 128^3 0.80 -> 0.35, 200^3 2.19 ->
-// 1.55.  Four right-hand sides against the group kernel: 128^3 1.00 against
-// 1.41, 160^3 2.09 against 2.47, 192^3 4.75 against 3.70.  Eight: 64^3 0.26
-// (group kernel) against about 0.32.
+// tuned; untuned always in complex128, and in complex64 except for 8 and more
+// right-hand sides at the widths past 96 that have a kernel of groups of 8.
+// One right-hand side, best kernel of before -> twisted, in ms: complex64 48^3
+// 0.234 -> 0.083, 64^3 0.167 -> 0.117, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
+// 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.55 -> 1.52, 140 x 140 x 150
+// 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.12, 128^3
+// 0.80 -> 0.35, 200^3 2.19 -> 1.55; complex128 24 x 22 x 28 0.115 -> 0.053,
+// 64^3 0.25 -> 0.15, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140 x 150
+// 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the group kernels:
+// complex128 128^3 x 8 1.73 against 2.76, 192 x 192 x 100 x 8 4.8 against 7.5;
+// complex64 192^3 x 4 3.59 against 3.70, 96^3 x 8 0.53 against 0.71, but 128^3
+// x 8 1.18 against 1.08 and 192^3 x 8 6.2 against 5.0.
 // Under stream capture an untuned call also takes it while the top-down chain
 // is incomplete, which cannot be completed there.
 bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
   const Factors& f = p->fac[prec];
-  if (prec != HZ_PREC_C64 || !f.tw_ready) return false;
+  if (!f.tw_ready) return false;
   const SolveKernel sk = solve_kernel_choice();
   if (sk == SK_TWIST) return true;
   if (sk != SK_DEFAULT) return false;
   if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
-  if (nrhs < (p->nx > 160 ? 4 : 8) || !mfma_solve_available(prec, (int)p->nx)) return true;
+  if (nrhs < 8 || p->nx <= 96 || !mfma_solve_available(prec, (int)p->nx)) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
   return !f.top_full && cs != hipStreamCaptureStatusNone;
@@ -2551,14 +2554,15 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   f.sym_ready = false;
   f.tw_ready = false;
   f.hodlr.release();
-  // twisted factors (complex64, up to 256 columns, at most two planes a slot):
-  // the bottom-up chain runs beside the top-down one in the same launch
-  const bool twist = prec == HZ_PREC_C64 && ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") &&
+  f.elem = prec == HZ_PREC_FP64 ? sizeof(double2) : sizeof(float2);
+  // twisted factors (up to 256 columns, at most two planes a slot): the
+  // bottom-up chain runs beside the top-down one in the same launch
+  const bool twist = ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") &&
                      !getenv("HZ_NO_SYM_PACK");
   f.tw_m = twist ? ny / 2 : 0;
   f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr;
   if (twist) {
-    const size_t gb = (size_t)p->nslot * (ny - f.tw_m) * (size_t)n * n * sizeof(float2);
+    const size_t gb = (size_t)p->nslot * (ny - f.tw_m) * (size_t)n * n * f.elem;
     if (f.Gb.bytes != gb) {
       f.Gb.release();
       f.Gb.alloc(gb);
@@ -2568,7 +2572,6 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
     f.Gtw.release();
     f.tw_scr.release();
   }
-  f.elem = prec == HZ_PREC_FP64 ? sizeof(double2) : sizeof(float2);
   const size_t bytes = (size_t)p->nslot * ny * (size_t)n * n * f.elem;
   if (f.G.bytes != bytes) {
     f.G.release();
@@ -2606,9 +2609,9 @@ void factor_end(hz_problem* p, int prec, hipStream_t s) {
   // twisted packed copy; the unpacked bottom-up blocks are not kept
   f.tw_ready = false;
   if (f.Gb.ptr && p->nslot > 0) {
-    pack_tri(p, s);
+    pack_tri(p, prec, s);
     f.tw_ready = true;
-    const size_t sb = (size_t)3 * TW_RHS * p->nz * p->nx * sizeof(float2);
+    const size_t sb = (size_t)3 * TW_RHS * p->nz * p->nx * f.elem;
     if (f.tw_scr.bytes != sb) {
       f.tw_scr.release();
       f.tw_scr.alloc(sb);
@@ -2698,7 +2701,7 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
              "adjoint plane solve: the dense factors were released by HZ_HODLR_FREE_DENSE");
   }
   if (uses_twist(p, prec, nrhs, adjoint, t, s)) {
-    solve_tri(p, nrhs, x, adjoint, s);
+    solve_tri(p, prec, nrhs, x, adjoint, s);
     return;
   }
   if (!f.top_full) ensure_dense(p, prec, s);

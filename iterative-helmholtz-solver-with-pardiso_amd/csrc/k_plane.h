@@ -59,10 +59,10 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
                        void* Gb, int jbeg, int jend, hipStream_t s);
 
 
-// Twisted complex64 plane solves (k_tri.hip): whether a width has them, the
-// packing of the factor chains (G, Gb) into Gtw, and the solve of nrhs vectors.
+// Twisted plane solves (k_tri.hip): whether a width has them, the packing of
+// the factor chains (G, Gb) into Gtw, and the solve of nrhs vectors.
 bool tri_available(int nx);
-void pack_tri(hz_problem* p, hipStream_t s);
-void solve_tri(hz_problem* p, int nrhs, void* x, bool adjoint, hipStream_t s);
+void pack_tri(hz_problem* p, int prec, hipStream_t s);
+void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s);
 
 }  // namespace hz

@@ -1,5 +1,5 @@
-// k_tri.hip -- twisted plane solves, complex64: both planes of a factor slot
-// from the packed upper triangle of its symmetric block inverses.
+// k_tri.hip -- twisted plane solves: both planes of a factor slot from one half
+// of its symmetric block inverses, complex64 and complex128.
 //
 // Planes k and nz - k share a factor slot, and a slot's chain is eliminated
 // from both ends (block j < m: top-down inverse G_j, j = m: T_m, j > m:
@@ -33,6 +33,12 @@
 //   transposed, y_c += K(r, c) v'_r: A = the components of v'_r, B = K
 //     transposed within its 4 x 4 block (quad permutes); summed over the tile's
 //     four row groups by row rotations and stored as the tile's partial sum.
+// complex128 takes the 4x4x4 products (v_mfma_f64_4x4x4f64: four blocks, A lane
+// (i = l & 3, block (l >> 2) & 3, k = l >> 4), B lane j for i, D lane (j, block,
+// i)): register p of a lane holds row 4 p + i, column 4 block + k.  The direct
+// products keep one sum per p and add the blocks at the row's end; a product
+// with the identity moves a 4 x 4 block from the A to the B layout exactly, and
+// the transposed products then sum over all rows in the accumulator.
 // No value is added to by two waves: the thread of (plane, row) adds the row's
 // direct sum and its transposed partials in a fixed order.
 //
@@ -43,7 +49,8 @@
 // not depend on the vector.  At 200^3 a solve takes 1.52 ms = 7.5 GB at 4.95
 // TB/s, the rate of a large device copy there (the products and barriers alone,
 // without the loads: 1.00 ms); at 64^3 0.117 ms, 1.8 us a step, of which 0.8 us
-// are barriers, sums and the update.  Measured against it: the kernel it
+// are barriers, sums and the update.  complex128 at 200^3 2.87 ms (15.0 GB, 5.2
+// TB/s), at 140 x 140 x 150 0.92 ms.  Measured against it: the kernel it
 // replaced at 128, 160, 192 and 200 columns (tiles through an LDS ring per
 // wave) 0.55, 0.81, 1.33 and 1.55 ms against 0.34, 0.71, 1.23 and 1.52.
 #include <type_traits>
@@ -63,6 +70,17 @@ __device__ __forceinline__ float tri_dpp(float x) {
 // a's sum over the lane pairs that CTRL joins where !hi, b's where hi
 template <int CTRL>
 __device__ __forceinline__ float tri_pair(float a, float b, bool hi) {
+  return (hi ? b : a) + tri_dpp<CTRL>(hi ? a : b);
+}
+template <int CTRL>
+__device__ __forceinline__ double tri_dpp(double x) {
+  const long long b = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+template <int CTRL>
+__device__ __forceinline__ double tri_pair(double a, double b, bool hi) {
   return (hi ? b : a) + tri_dpp<CTRL>(hi ? a : b);
 }
 // sum over lane bit 4 (5): a's where the bit is 0, b's where it is 1
@@ -114,39 +132,48 @@ __device__ __forceinline__ void tri_quad_transpose(float* k, float* l) {
   l[0] = d0; l[1] = d1; l[2] = d2; l[3] = d3;
 }
 
-template <int NT>
+template <typename T, int NT>
 struct TriShape {
   static constexpr int NW = (NT + 1) / 2;  // waves: tile rows w and w + NW (the last wave of an odd NT: one row)
   static constexpr int NA = NT / 2 + 1;    // tiles of row w
   static constexpr int NB = NT - NT / 2;   // tiles of row w + NW
   static constexpr int NS = NA + NB;       // NT + 1
   static constexpr int THREADS = 64 * NW;  // >= 2 * 16 NT: one thread per (plane, row) in the update
-  static constexpr int NP = 64 * ((16 * NT - 16 + 63) / 64) + 16;  // floats a component: 16 mod 64, the four
+  static constexpr int NP = 64 * ((16 * NT - 16 + 63) / 64) + 16;  // values a component: 16 mod 64, the four
                                                                    // components' reads fall in distinct banks
-  static constexpr size_t lds = sizeof(float) * (8 * (size_t)NP + 64 * ((size_t)(NT + 1) * NA + NT + 1));
+  // tiles in flight a wave: a whole block's, or (complex128, whose tiles take
+  // 16 registers) a half or a third of them where they would not fit
+  static constexpr int RD = sizeof(T) == 4 || NS <= 9 ? NS : NS <= 11 ? (NS + 1) / 2 : (NS + 2) / 3;
+  static constexpr int NSR = (NS + RD - 1) / RD * RD;  // slots of a block, the last possibly empty
+  static constexpr size_t lds = sizeof(T) * (8 * (size_t)NP + 64 * ((size_t)(NT + 1) * NA + NT + 1));
 };
 
-template <int NT, int PH, bool ADJ>
-__global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
-    const float2* __restrict__ P, float2* __restrict__ X, const double2* __restrict__ cmy,
+template <typename T, int NT, int PH, bool ADJ>
+__global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
+    const typename Cx<T>::t* __restrict__ P, typename Cx<T>::t* __restrict__ X, const double2* __restrict__ cmy,
     const double2* __restrict__ cpy, const double2* __restrict__ symd, int n, int ny, int m, int nz, int64_t n2,
-    int64_t N, const int2* __restrict__ slotp, float2* __restrict__ scr) {
-  typedef float2 C;
-  typedef TriShape<NT> S;
+    int64_t N, const int2* __restrict__ slotp, int nslot, int nrhs, typename Cx<T>::t* __restrict__ scr) {
+  typedef typename Cx<T>::t C;
+  typedef TriShape<T, NT> S;
+  constexpr bool F32 = sizeof(T) == 4;
   constexpr int NP = S::NP;
   constexpr int BS = NT * (NT + 1) / 2 * 256;  // complex values of a packed block
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  float* const vq = reinterpret_cast<float*>(smem_raw);  // [4][NP] components of v'
-  float* const vr = vq + 4 * NP;                         // [4][NP] rotated: (-Im A, Re A, -Im B, Re B)
-  float* const dsum = vr + 4 * NP;                       // [NT + 1][2][16][2] direct sums (plane, row, re/im)
-  float* const tsum = dsum + 64 * (NT + 1);              // [C][d][2][16][2] transposed sums of tile (C - d, C)
-                                                         // (the last of either: sums nobody reads)
+  T* const vq = reinterpret_cast<T*>(smem_raw);  // [4][NP] components of v'
+  T* const vr = vq + 4 * NP;                     // [4][NP] rotated: (-Im A, Re A, -Im B, Re B)
+  T* const dsum = vr + 4 * NP;                   // [NT + 1][2][16][2] direct sums (plane, row, re/im)
+  T* const tsum = dsum + 64 * (NT + 1);          // [C][d][2][16][2] transposed sums of tile (C - d, C)
+                                                 // (the last of either: sums nobody reads)
 
-  const int slot = blockIdx.x >> 1, half = blockIdx.x & 1;
+  // Workgroups go to the 8 XCDs in turn: the right-hand sides of one (slot,
+  // half) take every eighth place, so they run side by side on one XCD and
+  // share its L2's copy of the blocks.
+  const int place = blockIdx.x >> 3, pair = place / nrhs * 8 + (blockIdx.x & 7);
+  const int slot = pair >> 1, half = pair & 1;
+  if (slot >= nslot) return;
   const int2 sp = slotp[slot];
   const bool twoB = sp.y >= 0;
-  const int64_t rhs = blockIdx.y;
-  const int nrhs = gridDim.y;
+  const int64_t rhs = place % nrhs;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bi = lane >> 2, qi = lane & 3, rg = bi & 3, cg = bi >> 2;
@@ -183,7 +210,7 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
     if (!ADJ) return f;
     const double2 d = cmul_d(dxr, dy[j]);
     const double2 v = cmul_d(make_double2(f.x, -(double)f.y), d);
-    return make_float2((float)v.x, (float)v.y);
+    return mk<C>(v.x, v.y);
   };
 
   if (PH == 0 && half == 0 && wr) *scr_at(2) = load_f(xs[(int64_t)m * n], m);
@@ -194,29 +221,31 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
   // into sums that nobody reads.)
   const int ra = w, rb = w + S::NW < NT ? w + S::NW : w;
   const bool spare = w + S::NW >= NT;
-  const C* const tiles = Pk + (size_t)w * S::NS * 256 + 2 * lane;
-  float4 q[S::NS][2];
+  constexpr int UL = F32 ? 2 : 1, UQ = F32 ? 2 : 4;  // complex values a unit, units a lane and tile
+  const C* const tiles = Pk + (size_t)w * S::NS * 256 + UL * lane;
+  struct alignas(16) Unit { C c[UL]; };
+  Unit q[S::RD][UQ];
   // (no branch around a load: with one, the compiler cannot count the younger
   // loads in flight and waits for all of them before each tile)
   auto load_slot = [&](int t, const C* blk) {
     const C* const a = blk + (spare && t >= S::NA ? t - S::NA : t) * 256;
-    q[t][0] = *reinterpret_cast<const float4*>(a);
-    q[t][1] = *reinterpret_cast<const float4*>(a + 128);
+#pragma unroll
+    for (int u = 0; u < UQ; ++u) q[t % S::RD][u] = *reinterpret_cast<const Unit*>(a + u * 64 * UL);
   };
   {
     const C* const blk = tiles + (size_t)blk_of(0) * BS;
 #pragma unroll
-    for (int t = 0; t < S::NS; ++t) {
+    for (int t = 0; t < S::RD; ++t) {
       load_slot(t, blk);
       __builtin_amdgcn_sched_barrier(0);  // in the order of use, as in the steps: the waits count on it
     }
   }
 
   // ---- v' of the first block
-  for (int e = tid; e < 8 * NP; e += S::THREADS) vq[e] = 0.f;
+  for (int e = tid; e < 8 * NP; e += S::THREADS) vq[e] = (T)0;
   __syncthreads();
   auto put_v = [&](double2 v) {  // v' = D^-1 v of this thread's row
-    const float a = (float)v.x, b = (float)v.y;
+    const T a = (T)v.x, b = (T)v.y;
     vq[(2 * ps) * NP + pr] = a;
     vq[(2 * ps + 1) * NP + pr] = b;
     vr[(2 * ps) * NP + pr] = -b;
@@ -251,90 +280,158 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
 
   for (int st = 0; st < nsteps; ++st) {
     const int jb = blk_of(st), jn = next_of(st);
+    const C* const cblk = tiles + (size_t)jb * BS;
     const C* const nblk = tiles + (size_t)blk_of(st + 1 < nsteps ? st + 1 : st) * BS;
-    const C pre = xs[(int64_t)(jn >= 0 ? jn : jb) * n];
-
-    // Software pipeline over the tiles, one scheduling region each: tile t's
-    // direct products, transposes and reload, tile t - 1's transposed products
-    // and tile t - 2's sum over the row groups.  (Without the fences the
-    // compiler moves the reloads to the end of the step.)
-    const hz_v4f z4 = {0.f, 0.f, 0.f, 0.f};
-    hz_v4f da0 = z4, da1 = z4, db0 = z4, db1 = z4;  // direct sums of rows ra, rb
-    // components of the rows' v' (A operands of the transposed products)
-    const float4 va = *reinterpret_cast<const float4*>(vq + qi * NP + 16 * ra + 4 * rg);
-    const float4 vb = *reinterpret_cast<const float4*>(vr + qi * NP + 16 * ra + 4 * rg);
-    const float4 wa = *reinterpret_cast<const float4*>(vq + qi * NP + 16 * rb + 4 * rg);
-    const float4 wb = *reinterpret_cast<const float4*>(vr + qi * NP + 16 * rb + 4 * rg);
-    float tk[2][8];
-    hz_v4f ts[2];
-    float4 cv[2], cr[2];  // components of the tile column's v', one tile ahead
+    // the slot that takes tile t's registers (past the empty slots of a block,
+    // the next block's)
+    auto reload = [&](int t) {
+      int u = t + S::RD;
+      if (u < S::NS) {
+        load_slot(u, cblk);
+      } else {
+        if (u < S::NSR) u += S::RD;
+        load_slot(u - S::NSR, nblk);
+      }
+    };
     auto col_of = [&](int t) {
       const int c = t < S::NA ? ra + t : rb + t - S::NA;
       return c < NT ? c : c - NT;
     };
-    auto load_col = [&](int t) {
-      const int at = qi * NP + 16 * col_of(t) + 4 * cg;
-      cv[t & 1] = *reinterpret_cast<const float4*>(vq + at);
-      cr[t & 1] = *reinterpret_cast<const float4*>(vr + at);
-    };
-    load_col(0);
-#pragma unroll
-    for (int t = 0; t < S::NS + 2; ++t) {
-      if (t + 1 < S::NS) load_col(t + 1);
-      if (t < S::NS) {
-        float kr[4] = {q[t][0].x, q[t][0].z, q[t][1].x, q[t][1].z};
-        float ki[4] = {q[t][0].y, q[t][0].w, q[t][1].y, q[t][1].w};
-        const float4 u = cv[t & 1], v = cr[t & 1];
-        hz_v4f& d0 = t < S::NA ? da0 : db0;
-        hz_v4f& d1 = t < S::NA ? da1 : db1;
-        d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[0], u.x, d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[0], v.x, d1, 0, 0, 0);
-        d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[1], u.y, d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[1], v.y, d1, 0, 0, 0);
-        d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[2], u.z, d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[2], v.z, d1, 0, 0, 0);
-        d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[3], u.w, d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[3], v.w, d1, 0, 0, 0);
-        tri_quad_transpose(kr, ki);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          tk[t & 1][i] = kr[i];
-          tk[t & 1][4 + i] = ki[i];
+    const C pre = xs[(int64_t)(jn >= 0 ? jn : jb) * n];
+
+    if constexpr (F32) {
+      // Software pipeline over the tiles, one scheduling region each: tile t's
+      // direct products, transposes and reload, tile t - 1's transposed products
+      // and tile t - 2's sum over the row groups.  (Without the fences the
+      // compiler moves the reloads to the end of the step.)
+      const hz_v4f z4 = {0.f, 0.f, 0.f, 0.f};
+      hz_v4f da0 = z4, da1 = z4, db0 = z4, db1 = z4;  // direct sums of rows ra, rb
+      // components of the rows' v' (A operands of the transposed products)
+      const float4 va = *reinterpret_cast<const float4*>(vq + qi * NP + 16 * ra + 4 * rg);
+      const float4 vb = *reinterpret_cast<const float4*>(vr + qi * NP + 16 * ra + 4 * rg);
+      const float4 wa = *reinterpret_cast<const float4*>(vq + qi * NP + 16 * rb + 4 * rg);
+      const float4 wb = *reinterpret_cast<const float4*>(vr + qi * NP + 16 * rb + 4 * rg);
+      float tk[2][8];
+      hz_v4f ts[2];
+      float4 cv[2], cr[2];  // components of the tile column's v', one tile ahead
+      auto load_col = [&](int t) {
+        const int at = qi * NP + 16 * col_of(t) + 4 * cg;
+        cv[t & 1] = *reinterpret_cast<const float4*>(vq + at);
+        cr[t & 1] = *reinterpret_cast<const float4*>(vr + at);
+      };
+      load_col(0);
+  #pragma unroll
+      for (int t = 0; t < S::NS + 2; ++t) {
+        if (t + 1 < S::NS) load_col(t + 1);
+        if (t < S::NS) {
+          float kr[4], ki[4];
+  #pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            kr[i] = q[t][i / 2].c[i % UL].x;
+            ki[i] = q[t][i / 2].c[i % UL].y;
+          }
+          const float4 u = cv[t & 1], v = cr[t & 1];
+          hz_v4f& d0 = t < S::NA ? da0 : db0;
+          hz_v4f& d1 = t < S::NA ? da1 : db1;
+          d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[0], u.x, d0, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[0], v.x, d1, 0, 0, 0);
+          d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[1], u.y, d0, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[1], v.y, d1, 0, 0, 0);
+          d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[2], u.z, d0, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[2], v.z, d1, 0, 0, 0);
+          d0 = __builtin_amdgcn_mfma_f32_4x4x1f32(kr[3], u.w, d0, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ki[3], v.w, d1, 0, 0, 0);
+          tri_quad_transpose(kr, ki);
+  #pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            tk[t & 1][i] = kr[i];
+            tk[t & 1][4 + i] = ki[i];
+          }
+          reload(t);
         }
-        load_slot(t, nblk);
-      }
-      if (t >= 1 && t <= S::NS) {
-        const int u = t - 1;
-        const float4 a = u < S::NA ? va : wa, b = u < S::NA ? vb : wb;
-        // the diagonal tiles' own 4 x 4 blocks have no transposed product
-        // (their lower blocks are stored as zeros)
-        const bool off = (u != 0 && u != S::NA) || cg > rg;
-        const float av[4] = {off ? a.x : 0.f, off ? a.y : 0.f, off ? a.z : 0.f, off ? a.w : 0.f};
-        const float bv[4] = {off ? b.x : 0.f, off ? b.y : 0.f, off ? b.z : 0.f, off ? b.w : 0.f};
-        hz_v4f x = z4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          x = __builtin_amdgcn_mfma_f32_4x4x1f32(av[i], tk[u & 1][i], x, 0, 0, 0);
-          x = __builtin_amdgcn_mfma_f32_4x4x1f32(bv[i], tk[u & 1][4 + i], x, 0, 0, 0);
+        if (t >= 1 && t <= S::NS) {
+          const int u = t - 1;
+          const float4 a = u < S::NA ? va : wa, b = u < S::NA ? vb : wb;
+          // the diagonal tiles' own 4 x 4 blocks have no transposed product
+          // (their lower blocks are stored as zeros)
+          const bool off = (u != 0 && u != S::NA) || cg > rg;
+          const float av[4] = {off ? a.x : 0.f, off ? a.y : 0.f, off ? a.z : 0.f, off ? a.w : 0.f};
+          const float bv[4] = {off ? b.x : 0.f, off ? b.y : 0.f, off ? b.z : 0.f, off ? b.w : 0.f};
+          hz_v4f x = z4;
+  #pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(av[i], tk[u & 1][i], x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(bv[i], tk[u & 1][4 + i], x, 0, 0, 0);
+          }
+          ts[u & 1] = x;
         }
-        ts[u & 1] = x;
+        if (t >= 2) {
+          // lane (rg, cg, j) gets component rg of column 4 cg + j
+          const int u = t - 2;
+          const hz_v4f x = ts[u & 1];
+          const float s = tri_pair<0x128>(tri_pair<0x124>(x[0], x[1], b2), tri_pair<0x124>(x[2], x[3], b2), b3);
+          const int d = u < S::NA ? u : u - S::NA, at = u < S::NA || !spare ? col_of(u) : NT;
+          tsum[64 * (at * S::NA + d) + (rg >> 1) * 32 + (4 * cg + qi) * 2 + (rg & 1)] = s;
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (t >= 2) {
-        // lane (rg, cg, j) gets component rg of column 4 cg + j
-        const int u = t - 2;
-        const hz_v4f x = ts[u & 1];
-        const float s = tri_pair<0x128>(tri_pair<0x124>(x[0], x[1], b2), tri_pair<0x124>(x[2], x[3], b2), b3);
-        const int d = u < S::NA ? u : u - S::NA, at = u < S::NA || !spare ? col_of(u) : NT;
-        tsum[64 * (at * S::NA + d) + (rg >> 1) * 32 + (4 * cg + qi) * 2 + (rg & 1)] = s;
+      // the direct sums over the column groups (lane bits 4, 5)
+      {
+        const hz_v4f a = da0 + da1, b = db0 + db1;
+        const int at = (qi >> 1) * 32 + (4 * rg + cg) * 2 + (qi & 1);
+        dsum[64 * ra + at] = tri_sum32(tri_sum16(a[0], a[1]), tri_sum16(a[2], a[3]));
+        dsum[64 * (spare ? NT : rb) + at] = tri_sum32(tri_sum16(b[0], b[1]), tri_sum16(b[2], b[3]));
       }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // the direct sums over the column groups (lane bits 4, 5)
-    {
-      const hz_v4f a = da0 + da1, b = db0 + db1;
-      const int at = (qi >> 1) * 32 + (4 * rg + cg) * 2 + (qi & 1);
-      dsum[64 * ra + at] = tri_sum32(tri_sum16(a[0], a[1]), tri_sum16(a[2], a[3]));
-      dsum[64 * (spare ? NT : rb) + at] = tri_sum32(tri_sum16(b[0], b[1]), tri_sum16(b[2], b[3]));
+    } else {
+      const int i4 = lane >> 4;  // k of an operand, i of a result
+      const double one = i4 == qi ? 1.0 : 0.0;  // the identity, as B operand
+      double va[4], vb[4], dp[4];
+      auto row_operands = [&](int R) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          va[p] = vq[qi * NP + 16 * R + 4 * p + i4];
+          vb[p] = vr[qi * NP + 16 * R + 4 * p + i4];
+          dp[p] = 0.0;
+        }
+      };
+      // sum over the blocks (lane bits 2, 3): block b gets the rows 4 b ..
+      auto flush_row = [&](int out) {
+        const double s = tri_pair<0x128>(tri_pair<0x124>(dp[0], dp[1], b2), tri_pair<0x124>(dp[2], dp[3], b2), b3);
+        dsum[64 * out + (qi >> 1) * 32 + (4 * rg + i4) * 2 + (qi & 1)] = s;
+      };
+      row_operands(ra);
+#pragma unroll
+      for (int t = 0; t < S::NS; ++t) {
+        if (t == S::NA) {
+          flush_row(ra);
+          row_operands(rb);
+        }
+        const int cc = col_of(t), d = t < S::NA ? t : t - S::NA;
+        const double u = vq[qi * NP + 16 * cc + 4 * rg + i4], v = vr[qi * NP + 16 * cc + 4 * rg + i4];
+        double kr[4], ki[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const C k = q[t % S::RD][p].c[0];
+          dp[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(k.x, u, dp[p], 0, 0, 0);
+          kr[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(k.x, one, 0.0, 0, 0, 0);
+          dp[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, v, dp[p], 0, 0, 0);
+          ki[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, one, 0.0, 0, 0, 0);
+        }
+        reload(t);
+        double x = 0.0;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          // the diagonal tile's own 4 x 4 blocks have no transposed product
+          // (its lower blocks are stored as zeros)
+          const bool off = d > 0 || rg > p;
+          x = __builtin_amdgcn_mfma_f64_4x4x4f64(off ? va[p] : 0.0, kr[p], x, 0, 0, 0);
+          x = __builtin_amdgcn_mfma_f64_4x4x4f64(off ? vb[p] : 0.0, ki[p], x, 0, 0, 0);
+        }
+        const int at = t < S::NA || !spare ? cc : NT;
+        tsum[64 * (at * S::NA + d) + (i4 >> 1) * 32 + (4 * rg + qi) * 2 + (i4 & 1)] = x;
+        __builtin_amdgcn_sched_barrier(0);  // the reloads stay in order
+      }
+      flush_row(spare ? NT : rb);
     }
     __syncthreads();
 
@@ -346,14 +443,14 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
         const C u = *reinterpret_cast<const C*>(tsum + 64 * (rt * S::NA + d) + at);
         // even NT: tile (C - NT/2, C) is kept where C - NT/2 is below NT/2
         const bool kept = NT % 2 != 0 || d < NT / 2 || rt >= NT / 2;
-        y.x += kept ? u.x : 0.f;
-        y.y += kept ? u.y : 0.f;
+        y.x += kept ? u.x : (T)0;
+        y.y += kept ? u.y : (T)0;
       }
       if (wr && PH == 1 && (half == 0 || st > 0)) {  // x_jb
         C o = y;
         if (ADJ) {
           const double2 z = cmul_d(make_double2(y.x, y.y), cmul_d(dxir, dyi[jb]));
-          o = make_float2((float)z.x, -(float)z.y);
+          o = mk<C>(z.x, -z.y);
         }
         xs[(int64_t)jb * n] = o;
       }
@@ -363,8 +460,8 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
         const double2 cf = lower ? cmy[jn] : cpy[jn];
         const C f = PH == 0 ? load_f(pre, jn) : pre;
         C nv;
-        nv.x = f.x - (float)(cf.x * y.x - cf.y * y.y);
-        nv.y = f.y - (float)(cf.x * y.y + cf.y * y.x);
+        nv.x = f.x - (T)(cf.x * y.x - cf.y * y.y);
+        nv.y = f.y - (T)(cf.x * y.y + cf.y * y.x);
         if (wr && PH == 0) xs[(int64_t)jn * n] = nv;  // t_jn / b_jn
         put_v(cmul_d(make_double2(nv.x, nv.y), cmul_d(dxir, dyi[jn])));
       }
@@ -375,65 +472,53 @@ __global__ __launch_bounds__(TriShape<NT>::THREADS) void k_solve_tri(
 
 // Packed blocks of the slots' twisted chains: tile blockIdx.x of block
 // blockIdx.y = slot ny + j, X_j from G (j < m) or Gb (j >= m), times D_j.
-__global__ __launch_bounds__(256) void k_pack_tri(const float2* __restrict__ G, const float2* __restrict__ Gb,
-                                                  float2* __restrict__ P, const double2* __restrict__ dx,
+template <typename T>
+__global__ __launch_bounds__(256) void k_pack_tri(const typename Cx<T>::t* __restrict__ G,
+                                                  const typename Cx<T>::t* __restrict__ Gb,
+                                                  typename Cx<T>::t* __restrict__ P, const double2* __restrict__ dx,
                                                   const double2* __restrict__ dy, int n, int ny, int m, int nt) {
-  __shared__ float2 v[16][17];
+  typedef typename Cx<T>::t C;
+  __shared__ C v[16][17];
   const int j = blockIdx.y % ny, slot = blockIdx.y / ny, tid = threadIdx.x;
   const size_t nn = (size_t)n * n;
-  const float2* const B = j >= m ? Gb + ((size_t)slot * (ny - m) + (j - m)) * nn : G + ((size_t)slot * ny + j) * nn;
+  const C* const B = j >= m ? Gb + ((size_t)slot * (ny - m) + (j - m)) * nn : G + ((size_t)slot * ny + j) * nn;
   // slot t of wave w: tile row w, then tile row w + nw
   const int nw = (nt + 1) / 2, na = nt / 2 + 1;
   const int w = blockIdx.x / (nt + 1), t = blockIdx.x - w * (nt + 1);
-  const int R = t < na ? w : w + nw, d = t < na ? t : t - na, C = R + d < nt ? R + d : R + d - nt;
+  const int R = t < na ? w : w + nw, d = t < na ? t : t - na, c0 = R + d < nt ? R + d : R + d - nt;
   {
-    const int r = tid & 15, c = tid >> 4, gr = 16 * R + r, gc = 16 * C + c;
-    float2 o = make_float2(0.f, 0.f);
-    if (gr < n && gc < n && (R != C || r / 4 <= c / 4)) {
+    const int r = tid & 15, c = tid >> 4, gr = 16 * R + r, gc = 16 * c0 + c;
+    C o = mk<C>(0.0, 0.0);
+    if (gr < n && gc < n && (R != c0 || r / 4 <= c / 4)) {
       // K(r, c) = K(c, r) from the upper triangle
-      const int ur = R <= C ? gr : gc, uc = R <= C ? gc : gr;
-      const float2 g = B[ur + (size_t)n * uc];
+      const int ur = R <= c0 ? gr : gc, uc = R <= c0 ? gc : gr;
+      const C g = B[ur + (size_t)n * uc];
       const double2 a = dx[uc], b = dy[j];
       const double sx = a.x * b.x - a.y * b.y, sy = a.x * b.y + a.y * b.x;
-      o = make_float2((float)((double)g.x * sx - (double)g.y * sy), (float)((double)g.x * sy + (double)g.y * sx));
+      o = mk<C>((double)g.x * sx - (double)g.y * sy, (double)g.x * sy + (double)g.y * sx);
     }
     v[c][r] = o;
   }
   __syncthreads();
-  const int h = tid >> 7, l = (tid >> 1) & 63, e = tid & 1;
-  const int r = 4 * ((l >> 2) & 3) + (l & 3), c = 4 * (l >> 4) + 2 * h + e;
+  int r, c;
+  if (sizeof(T) == 4) {
+    const int h = tid >> 7, l = (tid >> 1) & 63, e = tid & 1;
+    r = 4 * ((l >> 2) & 3) + (l & 3);
+    c = 4 * (l >> 4) + 2 * h + e;
+  } else {
+    const int p = tid >> 6, l = tid & 63;
+    r = 4 * p + (l & 3);
+    c = 4 * ((l >> 2) & 3) + (l >> 4);
+  }
   P[((size_t)blockIdx.y * (nt * (nt + 1) / 2) + blockIdx.x) * 256 + tid] = v[c][r];
 }
 
-template <int NT, bool ADJ>
-void launch_tri(hz_problem* p, int nrhs, float2* x, hipStream_t s) {
-  const Factors& f = p->fac[HZ_PREC_C64];
-  constexpr size_t lds = TriShape<NT>::lds;
-  static_assert(lds <= 160 * 1024, "LDS");
-  set_max_lds((const void*)&k_solve_tri<NT, 0, ADJ>, lds);
-  set_max_lds((const void*)&k_solve_tri<NT, 1, ADJ>, lds);
-  for (int r0 = 0; r0 < nrhs; r0 += TW_RHS) {
-    const int nr = std::min(TW_RHS, nrhs - r0);
-    const dim3 grid((unsigned)(2 * p->nslot), (unsigned)nr), block(TriShape<NT>::THREADS);
-    float2* const xr = x + (size_t)r0 * p->N;
-    hipLaunchKernelGGL((k_solve_tri<NT, 0, ADJ>), grid, block, lds, s, f.Gtw.as<float2>(), xr, p->tab(1, 0),
-                       p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
-                       p->d_slotp.as<int2>(), f.tw_scr.as<float2>());
-    hipLaunchKernelGGL((k_solve_tri<NT, 1, ADJ>), grid, block, lds, s, f.Gtw.as<float2>(), xr, p->tab(1, 0),
-                       p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
-                       p->d_slotp.as<int2>(), f.tw_scr.as<float2>());
-    HZ_HIP(hipGetLastError());
-  }
-}
-
-}  // namespace
-
-bool tri_available(int nx) { return nx <= 16 * TRI_MAX_NT; }
-
-void pack_tri(hz_problem* p, hipStream_t s) {
-  Factors& f = p->fac[HZ_PREC_C64];
+template <typename T>
+void pack_tri_t(hz_problem* p, int prec, hipStream_t s) {
+  typedef typename Cx<T>::t C;
+  Factors& f = p->fac[prec];
   const int nt = ((int)p->nx + 15) / 16, tiles = nt * (nt + 1) / 2;
-  const size_t bytes = (size_t)p->nslot * p->ny * tiles * 256 * sizeof(float2);
+  const size_t bytes = (size_t)p->nslot * p->ny * tiles * 256 * sizeof(C);
   if (f.Gtw.bytes != bytes) {
     f.Gtw.release();
     f.Gtw.alloc(bytes);
@@ -443,27 +528,65 @@ void pack_tri(hz_problem* p, hipStream_t s) {
   const int per = 32768 / (int)p->ny > 0 ? 32768 / (int)p->ny : 1;
   for (int s0 = 0; s0 < p->nslot; s0 += per) {
     const int ns = std::min(per, p->nslot - s0);
-    hipLaunchKernelGGL(k_pack_tri, dim3((unsigned)tiles, (unsigned)(ns * p->ny)), dim3(256), 0, s,
-                       f.G.as<float2>() + (size_t)s0 * p->ny * p->nx * p->nx,
-                       f.Gb.as<float2>() + (size_t)s0 * (p->ny - f.tw_m) * p->nx * p->nx,
-                       f.Gtw.as<float2>() + (size_t)s0 * p->ny * tiles * 256, dx, dx + p->nx, (int)p->nx, (int)p->ny,
+    hipLaunchKernelGGL(k_pack_tri<T>, dim3((unsigned)tiles, (unsigned)(ns * p->ny)), dim3(256), 0, s,
+                       f.G.as<C>() + (size_t)s0 * p->ny * p->nx * p->nx,
+                       f.Gb.as<C>() + (size_t)s0 * (p->ny - f.tw_m) * p->nx * p->nx,
+                       f.Gtw.as<C>() + (size_t)s0 * p->ny * tiles * 256, dx, dx + p->nx, (int)p->nx, (int)p->ny,
                        f.tw_m, nt);
     HZ_HIP(hipGetLastError());
   }
 }
 
-void solve_tri(hz_problem* p, int nrhs, void* x, bool adjoint, hipStream_t s) {
+template <typename T, int NT, bool ADJ>
+void launch_tri(hz_problem* p, int prec, int nrhs, void* xv, hipStream_t s) {
+  typedef typename Cx<T>::t C;
+  const Factors& f = p->fac[prec];
+  C* const x = (C*)xv;
+  constexpr size_t lds = TriShape<T, NT>::lds;
+  static_assert(lds <= 160 * 1024, "LDS");
+  set_max_lds((const void*)&k_solve_tri<T, NT, 0, ADJ>, lds);
+  set_max_lds((const void*)&k_solve_tri<T, NT, 1, ADJ>, lds);
+  for (int r0 = 0; r0 < nrhs; r0 += TW_RHS) {
+    const int nr = std::min(TW_RHS, nrhs - r0);
+    const dim3 grid((unsigned)((2 * p->nslot + 7) / 8 * 8 * nr)), block(TriShape<T, NT>::THREADS);
+    C* const xr = x + (size_t)r0 * p->N;
+    hipLaunchKernelGGL((k_solve_tri<T, NT, 0, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
+                       p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
+                       p->d_slotp.as<int2>(), p->nslot, nr, f.tw_scr.as<C>());
+    hipLaunchKernelGGL((k_solve_tri<T, NT, 1, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
+                       p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
+                       p->d_slotp.as<int2>(), p->nslot, nr, f.tw_scr.as<C>());
+    HZ_HIP(hipGetLastError());
+  }
+}
+
+template <typename T>
+void solve_tri_t(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s) {
   switch (((int)p->nx + 15) / 16) {
-#define HZ_TRI(NT)                                                \
-  case NT:                                                        \
-    if (adjoint) launch_tri<NT, true>(p, nrhs, (float2*)x, s);    \
-    else launch_tri<NT, false>(p, nrhs, (float2*)x, s);           \
+#define HZ_TRI(NT)                                                   \
+  case NT:                                                           \
+    if (adjoint) launch_tri<T, NT, true>(p, prec, nrhs, x, s);       \
+    else launch_tri<T, NT, false>(p, prec, nrhs, x, s);              \
     break;
     HZ_TRI(1) HZ_TRI(2) HZ_TRI(3) HZ_TRI(4) HZ_TRI(5) HZ_TRI(6) HZ_TRI(7) HZ_TRI(8)
     HZ_TRI(9) HZ_TRI(10) HZ_TRI(11) HZ_TRI(12) HZ_TRI(13) HZ_TRI(14) HZ_TRI(15) HZ_TRI(16)
 #undef HZ_TRI
     default: HZ_CHECK(false, HZ_ERR_ARG, "nx=%d", (int)p->nx);
   }
+}
+
+}  // namespace
+
+bool tri_available(int nx) { return nx <= 16 * TRI_MAX_NT; }
+
+void pack_tri(hz_problem* p, int prec, hipStream_t s) {
+  if (prec == HZ_PREC_FP64) pack_tri_t<double>(p, prec, s);
+  else pack_tri_t<float>(p, prec, s);
+}
+
+void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s) {
+  if (prec == HZ_PREC_FP64) solve_tri_t<double>(p, prec, nrhs, x, adjoint, s);
+  else solve_tri_t<float>(p, prec, nrhs, x, adjoint, s);
 }
 
 }  // namespace hz

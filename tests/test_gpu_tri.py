@@ -1,5 +1,5 @@
-"""The twisted complex64 plane solve (default for few right-hand sides, forward
-and adjoint) over the widths where its 16 x 16 tiles, its wave split (even and
+"""The twisted plane solve (default for few right-hand sides and in complex128,
+forward and adjoint) over the widths where its 16 x 16 tiles, its wave split (even and
 odd tile counts) and its chains have edges, against the CPU oracle."""
 import numpy as np
 import pytest
@@ -44,27 +44,32 @@ CASES = [("s7", nx, ny, nz) for nx, ny, nz in (
 @pytest.mark.parametrize("mode,nx,ny,nz", CASES)
 def test_tri_vs_oracle(hz, oracle, mode, nx, ny, nz):
     """One and three right-hand sides, forward and adjoint, through the
-    preconditioner: 1e-4, the complex64 preconditioner's bound elsewhere."""
+    preconditioner: 1e-4 in complex64 and 1e-10 in complex128, the
+    preconditioners' bounds elsewhere."""
     print("case tri %s %d %d %d" % (mode, nx, ny, nz), flush=True)
     d, c = _case(hz, mode, nx, ny, nz)
     S, P = hz.Solver(d, c), oracle.Problem(d, c)
-    S.factor(hz.abi.PREC_C64)
+    tol = {hz.abi.PREC_C64: 1e-4, hz.abi.PREC_FP64: 1e-10}
+    for prec in tol:
+        S.factor(prec)
     rng = np.random.default_rng(nx)
     x = rng.standard_normal((3, d.N)) + 1j * rng.standard_normal((3, d.N))
     for adj in (False, True):
         want = [P.precond_apply(v, adjoint=adj) for v in x]
-        for nrhs in (1, 3):
-            got = S.precond_apply(torch.from_numpy(x[:nrhs]).cuda(), hz.abi.PREC_C64, adjoint=adj).cpu().numpy()
-            for q in range(nrhs):
-                assert _rel(got[q], want[q]) < 1e-4, (adj, nrhs, q, _rel(got[q], want[q]))
+        for prec in tol:
+            for nrhs in (1, 3):
+                got = S.precond_apply(torch.from_numpy(x[:nrhs]).cuda(), prec, adjoint=adj).cpu().numpy()
+                for q in range(nrhs):
+                    assert _rel(got[q], want[q]) < tol[prec], (adj, prec, nrhs, q, _rel(got[q], want[q]))
 
 
 def test_tri_widths_past_the_tiles(hz, oracle):
     """257 columns: no twisted factors, the one-directional kernels as before."""
     d, c = _case(hz, "s7", 257, 3, 3)
     S, P = hz.Solver(d, c), oracle.Problem(d, c)
-    S.factor(hz.abi.PREC_C64)
     x = np.random.default_rng(1).standard_normal(d.N) + 0j
-    for adj in (False, True):
-        got = S.precond_apply(torch.from_numpy(x).cuda(), hz.abi.PREC_C64, adjoint=adj).cpu().numpy()
-        assert _rel(got, P.precond_apply(x, adjoint=adj)) < 1e-4
+    for prec, tol in ((hz.abi.PREC_C64, 1e-4), (hz.abi.PREC_FP64, 1e-10)):
+        S.factor(prec)
+        for adj in (False, True):
+            got = S.precond_apply(torch.from_numpy(x).cuda(), prec, adjoint=adj).cpu().numpy()
+            assert _rel(got, P.precond_apply(x, adjoint=adj)) < tol
