@@ -25,6 +25,7 @@ SOURCES = [
     "k_blocktri.hip",
     "k_factor.hip",
     "k_tri.hip",
+    "k_rows.hip",
     "k_vec.hip",
     "hz_noalloc.hip",
     "k_hodlr.hip",

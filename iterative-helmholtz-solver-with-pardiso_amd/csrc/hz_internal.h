@@ -139,6 +139,10 @@ struct hz_problem {
   // the planes of each slot (int2[nslot]: the first plane, the second or -1);
   // slot_pairs: no slot holds more than two planes
   hz::DevBuf d_slotp;
+  // int2[ntwo]: the factored planes by twos, the two of a slot first, then the
+  // planes that have a slot alone (at most one place, the last, is empty: -1)
+  hz::DevBuf d_two;
+  int ntwo = 0;
   bool slot_pairs = false;
   std::vector<double2> kappa;                  // (nx*ny) (w/cb)^2 (1 + i beta)
   std::vector<double2> c0;                     // (nx*ny) background speed
@@ -275,8 +279,9 @@ bool twist_solve_available(const hz_problem* p, int prec);
 // factorisation stopped it at the twisted factors' middle; synchronous, and an
 // error under stream capture
 void ensure_dense(hz_problem* p, int prec, hipStream_t s);
-// whether the 8-RHS MFMA streaming kernel is instantiated for this width/precision
-bool mfma_solve_available(int prec, int nx);
+// whether the matrix-core kernel for groups of 8 right-hand sides is built for
+// this problem and precision
+bool mfma_solve_available(const hz_problem* p, int prec);
 // whether the single-RHS ring kernel is instantiated for this width/precision
 bool single_ring_available(int prec, int nx);
 

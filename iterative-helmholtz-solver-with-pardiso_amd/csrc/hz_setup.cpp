@@ -207,6 +207,16 @@ static void build_plane_map(hz_problem* p) {
     }
     p->d_slotp.alloc(p->nslot * sizeof(int2));
     HZ_HIP(hipMemcpy(p->d_slotp.ptr, sp.data(), p->nslot * sizeof(int2), hipMemcpyHostToDevice));
+    std::vector<int2> two, one;
+    for (const int2& v : sp) {
+      if (v.y >= 0) two.push_back(v);
+      else if (one.empty() || one.back().y >= 0) one.push_back(v);
+      else one.back().y = v.x;
+    }
+    two.insert(two.end(), one.begin(), one.end());
+    p->ntwo = (int)two.size();
+    p->d_two.alloc(two.size() * sizeof(int2));
+    HZ_HIP(hipMemcpy(p->d_two.ptr, two.data(), two.size() * sizeof(int2), hipMemcpyHostToDevice));
   } else {
     p->slot_pairs = false;
   }

@@ -120,7 +120,7 @@ void autotune(hz_problem* p, int prec, int nrhs, hz_tune_info* info) {
       t.solve_family = HZ_SOLVE_TWIST;
       cand.push_back(t);
     }
-    if (nrhs >= 8 && mfma_solve_available(prec, (int)p->nx)) {
+    if (nrhs >= 8 && mfma_solve_available(p, prec)) {
       Tuning t;
       t.solve_family = HZ_SOLVE_STREAM_MFMA;
       cand.push_back(t);

@@ -1028,279 +1028,6 @@ __global__ __launch_bounds__(dma::NT) void k_solve_mr(const typename Cx<T>::t* _
   __builtin_amdgcn_s_waitcnt(dma::wait_vm(0));
 }
 
-// ------------------------------------------- 8-RHS streaming solve on MFMA
-// Same LDS ring as k_solve_mr, for groups of 8 complex64 right-hand sides, with
-// the block product Y = G V (n x 8 complex) on the matrix cores: per 16-row x
-// 4-column tile of G two v_mfma_f32_16x16x4f32 accumulate
-//   C += Re(G) [Re V | Im V]  +  Im(G) [-Im V | Re V]  =  [Re Y | Im Y]
-// into one 16 x 16 FP32 tile (columns 0-7 real parts of the 8 vectors, 8-15
-// imaginary parts).  Operand layout of 16x16x4 f32 (wave64): A lane l holds
-// A[l % 16][l / 16], B lane l holds B[l / 16][l % 16], C lane l holds rows
-// 4 (l / 16) + 0..3 of column l % 16.  The B operands of a k-slice come from
-// the vectors in LDS once per wave and serve every row tile of the wave.
-// Wave w owns row tiles w and w + 8.
-
-template <int NX, int TCOL>
-struct MfShape {
-  static constexpr int n = NX;
-  static constexpr int RT = (n + 15) / 16;                    // row tiles
-  static constexpr int KS = TCOL / 4;                         // k-slices per tile
-  static constexpr int tps = n / TCOL;
-  static constexpr int units = TCOL * n / 2;                  // 16-byte units per tile
-  static constexpr int R = (units + dma::NT - 1) / dma::NT;
-  static constexpr int WE = (tps < 3 ? tps : 3) * R;
-  static constexpr int TPW = (RT + 7) / 8;                    // row tiles per wave (max)
-  static constexpr size_t lds = 4 * (size_t)R * dma::NT * 16 + (size_t)n * 8 * sizeof(float2) +
-                                (size_t)8 * TPW * 64 * 16;
-  static_assert(n % TCOL == 0 && TCOL % 4 == 0 && n % 2 == 0, "tile split");
-  static_assert(TPW <= 2, "row tiles per wave");
-  // the last row tile may read up to 15 rows past the block inside the slot
-  static_assert((size_t)(TCOL - 1) * n + 16 * RT <= (size_t)R * dma::NT * 2, "slot slack for the last row tile");
-  static_assert(2 * R <= 63 && WE <= 63, "vmcnt range");
-  static_assert(lds <= 160 * 1024, "LDS budget");
-};
-
-// ADJ: the adjoint sweep in conjugated variables with G_j^H = conj(D_j^-1 G_j D_j)
-// (G_j D_j symmetric, D_j = diag(dx(i) dy(j)) from symd = dx | dy | 1/dx | 1/dy):
-// the vector v holds D_j u_j, the product z = G_j v gives Y_j = D_j^-1 z; forward
-// u_{j+1} = conj(b_{j+1}) - cp_j Y_j (Y_j stored), backward X_j = Y_j - D_j^-1 z,
-// x_j = conj(X_j), u = cm_j X_j.  Same block sequence as the forward solve.
-template <int NX, int TCOL, bool ADJ>
-__global__ __launch_bounds__(dma::NT) void k_solve_mfma8(const float2* __restrict__ G, float2* __restrict__ X,
-                                                         const double2* __restrict__ cmy,
-                                                         const double2* __restrict__ cpy,
-                                                         const double2* __restrict__ symd, int ny, int64_t n2,
-                                                         int64_t N,
-    const int* __restrict__ fmap) {
-  typedef MfShape<NX, TCOL> S;
-  typedef float4 U;
-  constexpr int n = S::n, RT = S::RT, KS = S::KS, tps = S::tps, units = S::units, R = S::R, TPW = S::TPW;
-  constexpr int NR = 8;
-  __shared__ U s0[R * dma::NT], s1[R * dma::NT], s2[R * dma::NT], s3[R * dma::NT];
-  __shared__ U pbuf[8 * TPW * 64];
-  __shared__ float2 v[n * NR];
-  __shared__ float2 sdx[ADJ ? n : 1], sdxi[ADJ ? n : 1];  // dx, 1/dx (adjoint only)
-
-  const int k = blockIdx.x;
-  const int kf = fmap[k];  // factor slot; -1: a skipped plane (zeroed after the solve)
-  if (kf < 0) return;
-  const int64_t rhs0 = (int64_t)blockIdx.y * NR;
-  float2* xk = X + rhs0 * N + (int64_t)k * n2;
-  const size_t nn = (size_t)n * n;
-  const float2* Gk = G + (size_t)kf * ny * nn;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
-  const int li = lane & 15, lg = lane >> 4;  // operand row/column index, k / row-group index
-  const int nsteps = 2 * ny - 1;
-  const int TT = nsteps * tps;
-  auto blk_of = [&](int s) { return s <= ny - 1 ? s : 2 * ny - 2 - s; };
-
-#define HZ_MF_TILE(TC_, SLOT)                                                                           \
-  {                                                                                                     \
-    const int tc_ = (TC_) >= TT ? 0 : (TC_); /* past the end: re-read tile 0 */                        \
-    const int s_ = tc_ / tps, t_ = tc_ - s_ * tps;                                                      \
-    const unsigned char* base_ = reinterpret_cast<const unsigned char*>(Gk + (size_t)blk_of(s_) * nn) + \
-                                 (size_t)t_ * TCOL * n * sizeof(float2);                                \
-    _Pragma("unroll") for (int r_ = 0; r_ < R; ++r_) {                                                  \
-      const int p_ = r_ * dma::NT + tid;                                                                \
-      const int u_ = p_ < units ? p_ : units - 1;                                                       \
-      __builtin_amdgcn_global_load_lds((const void*)(base_ + (size_t)u_ * 16),                          \
-                                       (HZ_LDS void*)(&SLOT[r_ * dma::NT + wv * 64]), 16, 0, 0);        \
-    }                                                                                                   \
-  }
-  // the next line's operand for this wave's epilogue: lane l loads unit
-  // 8 rt + 2 g + (l & 1) of right-hand side q, consumer (g, q) = (l >> 1) / 8, % 8
-#define HZ_MF_LINE(J_)                                                                                  \
-  {                                                                                                     \
-    _Pragma("unroll") for (int a_ = 0; a_ < TPW; ++a_) {                                                \
-      const int rt_ = wv + 8 * a_;                                                                      \
-      if (rt_ < RT) {                                                                                   \
-        const int c_ = lane >> 1, g_ = c_ >> 3, q_ = c_ & 7;                                            \
-        int u_ = 8 * rt_ + 2 * g_ + (lane & 1);                                                         \
-        u_ = u_ < n / 2 ? u_ : n / 2 - 1;                                                               \
-        const float2* src_ = xk + (int64_t)q_ * N + (size_t)n * (J_) + 2 * (size_t)u_;                  \
-        __builtin_amdgcn_global_load_lds((const void*)src_, (HZ_LDS void*)(&pbuf[(wv * TPW + a_) * 64]), \
-                                         16, 0, 0);                                                     \
-      }                                                                                                 \
-    }                                                                                                   \
-  }
-  hz_v4f acc[TPW];
-#define HZ_MF_EPILOGUE(S_)                                                                                \
-  {                                                                                                       \
-    const int se_ = (S_);                                                                                 \
-    __builtin_amdgcn_s_waitcnt(dma::wait_vm(S::WE));                                                      \
-    __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);                                                          \
-    dma::raw_barrier(); /* every wave is done reading v of this step */                                  \
-    _Pragma("unroll") for (int a_ = 0; a_ < TPW; ++a_) {                                                  \
-      const int rt_ = wv + 8 * a_;                                                                        \
-      float im_[4];                                                                                       \
-      _Pragma("unroll") for (int r_ = 0; r_ < 4; ++r_) im_[r_] = __shfl_xor(acc[a_][r_], 8);             \
-      if (rt_ < RT && li < 8) {                                                                           \
-        const int q_ = li;                                                                                \
-        const U p0_ = pbuf[(wv * TPW + a_) * 64 + 2 * (8 * lg + q_)];                                     \
-        const U p1_ = pbuf[(wv * TPW + a_) * 64 + 2 * (8 * lg + q_) + 1];                                 \
-        const float2 pre_[4] = {make_float2(p0_.x, p0_.y), make_float2(p0_.z, p0_.w),                   \
-                                make_float2(p1_.x, p1_.y), make_float2(p1_.z, p1_.w)};                  \
-        float2 out_[4];                                                                                   \
-        _Pragma("unroll") for (int r_ = 0; r_ < 4; ++r_) {                                                \
-          const int row_ = 16 * rt_ + 4 * lg + r_;                                                        \
-          const float2 y_ = make_float2(acc[a_][r_], im_[r_]);                                            \
-          float2 nv_;                                                                                     \
-          if (ADJ) {                                                                                      \
-            const int jc_ = blk_of(se_);                                                                  \
-            const double2 dyi_ = symd[2 * n + ny + jc_];                                                  \
-            const float2 sxi_ = sdxi[row_ < n ? row_ : 0];                                                \
-            const double sx_ = (double)sxi_.x * dyi_.x - (double)sxi_.y * dyi_.y;                         \
-            const double sy_ = (double)sxi_.x * dyi_.y + (double)sxi_.y * dyi_.x;                         \
-            const double zx_ = y_.x * sx_ - y_.y * sy_, zy_ = y_.x * sy_ + y_.y * sx_;                    \
-            double ux_, uy_;                                                                              \
-            int jn_;                                                                                      \
-            if (se_ < ny - 1) {                                                                           \
-              const double2 cp = cpy[se_];                                                                \
-              out_[r_] = make_float2((float)zx_, (float)zy_);                                             \
-              ux_ = (double)pre_[r_].x - (cp.x * zx_ - cp.y * zy_);                                       \
-              uy_ = -(double)pre_[r_].y - (cp.x * zy_ + cp.y * zx_);                                      \
-              jn_ = se_ + 1;                                                                              \
-            } else {                                                                                      \
-              const double Xx_ = se_ >= ny ? (double)pre_[r_].x - zx_ : zx_;                              \
-              const double Xy_ = se_ >= ny ? (double)pre_[r_].y - zy_ : zy_;                              \
-              out_[r_] = make_float2((float)Xx_, (float)(-Xy_));                                          \
-              const double2 cm = cmy[jc_];                                                                \
-              ux_ = cm.x * Xx_ - cm.y * Xy_;                                                              \
-              uy_ = cm.x * Xy_ + cm.y * Xx_;                                                              \
-              jn_ = jc_ > 0 ? jc_ - 1 : 0;                                                                \
-            }                                                                                             \
-            const double2 dyn_ = symd[n + jn_];                                                           \
-            const float2 sxn_ = sdx[row_ < n ? row_ : 0];                                                 \
-            const double tx_ = (double)sxn_.x * dyn_.x - (double)sxn_.y * dyn_.y;                         \
-            const double ty_ = (double)sxn_.x * dyn_.y + (double)sxn_.y * dyn_.x;                         \
-            nv_ = make_float2((float)(ux_ * tx_ - uy_ * ty_), (float)(ux_ * ty_ + uy_ * tx_));            \
-          } else if (se_ < ny - 1) {                                                                      \
-            const double2 cm = cmy[se_ + 1];                                                              \
-            nv_.x = pre_[r_].x - (float)(cm.x * y_.x - cm.y * y_.y);                                      \
-            nv_.y = pre_[r_].y - (float)(cm.x * y_.y + cm.y * y_.x);                                      \
-            out_[r_] = nv_;                                                                               \
-          } else {                                                                                        \
-            const int j = 2 * ny - 2 - se_;                                                               \
-            out_[r_] = y_;                                                                                \
-            if (j > 0) {                                                                                  \
-              const double2 cp = cpy[j - 1];                                                              \
-              nv_.x = pre_[r_].x - (float)(cp.x * y_.x - cp.y * y_.y);                                    \
-              nv_.y = pre_[r_].y - (float)(cp.x * y_.y + cp.y * y_.x);                                    \
-            } else {                                                                                      \
-              nv_ = y_;                                                                                   \
-            }                                                                                             \
-          }                                                                                               \
-          if (row_ < n) v[row_ * NR + q_] = nv_;                                                          \
-        }                                                                                                 \
-        const int line_ = ADJ ? blk_of(se_) : (se_ < ny - 1 ? se_ + 1 : 2 * ny - 2 - se_);                \
-        float2* xq_ = xk + (int64_t)q_ * N + (size_t)n * line_ + 16 * rt_ + 4 * lg;                       \
-        if (16 * rt_ + 4 * lg + 1 < n)                                                                    \
-          *reinterpret_cast<U*>(xq_) = make_float4(out_[0].x, out_[0].y, out_[1].x, out_[1].y);           \
-        if (16 * rt_ + 4 * lg + 3 < n)                                                                    \
-          *reinterpret_cast<U*>(xq_ + 2) = make_float4(out_[2].x, out_[2].y, out_[3].x, out_[3].y);       \
-      }                                                                                                   \
-    }                                                                                                     \
-    __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);                                                          \
-  }
-#define HZ_MF_STAGE(TC_, SLOT, NEXT)                                                          \
-  {                                                                                           \
-    const int Tc = (TC_);                                                                     \
-    const int s = Tc / tps, t = Tc - s * tps;                                                 \
-    __builtin_amdgcn_s_waitcnt(dma::wait_vm(2 * R));                                          \
-    __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);                                              \
-    dma::raw_barrier();                                                                       \
-    if (Tc < TT && t == 0) {                                                                  \
-      _Pragma("unroll") for (int a = 0; a < TPW; ++a) acc[a] = hz_v4f{0.f, 0.f, 0.f, 0.f};    \
-      int slot_line = 0;                                                                      \
-      if (s < ny - 1) slot_line = s + 1;                                                      \
-      else if (ADJ && s >= ny) slot_line = 2 * ny - 2 - s;                                    \
-      else if (!ADJ && 2 * ny - 2 - s > 0) slot_line = 2 * ny - 3 - s;                        \
-      HZ_MF_LINE(slot_line)                                                                   \
-    }                                                                                         \
-    if (Tc < TT) {                                                                            \
-      const float2* sl = reinterpret_cast<const float2*>(SLOT);                               \
-      _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) {                                     \
-        const float2 vv = v[(t * TCOL + 4 * ks + lg) * NR + (li & 7)];                        \
-        const float b1 = li < 8 ? vv.x : vv.y;                                                \
-        const float b2 = li < 8 ? -vv.y : vv.x;                                               \
-        _Pragma("unroll") for (int a = 0; a < TPW; ++a) {                                     \
-          const int rt = wv + 8 * a;                                                          \
-          if (rt < RT) {                                                                      \
-            const float2 ga = sl[(4 * ks + lg) * n + 16 * rt + li];                           \
-            acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(ga.x, b1, acc[a], 0, 0, 0);         \
-            acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(ga.y, b2, acc[a], 0, 0, 0);         \
-          }                                                                                   \
-        }                                                                                     \
-      }                                                                                       \
-    }                                                                                         \
-    HZ_MF_TILE(Tc + 3, NEXT)                                                                  \
-    if (Tc < TT && t == tps - 1) HZ_MF_EPILOGUE(s)                                            \
-  }
-
-  if (ADJ) {
-    for (int i = tid; i < n; i += dma::NT) {
-      const double2 a = symd[i], b = symd[n + ny + i];
-      sdx[i] = make_float2((float)a.x, (float)a.y);
-      sdxi[i] = make_float2((float)b.x, (float)b.y);
-    }
-    __syncthreads();
-  }
-  for (int i = tid; i < n * NR; i += dma::NT) {
-    const int q = i % NR, row = i / NR;
-    const float2 b = xk[(int64_t)q * N + row];
-    if (ADJ) {
-      // v = D_0 conj(b_0)
-      const float2 a = sdx[row];
-      const double2 d0 = symd[n];
-      const double tx = (double)a.x * d0.x - (double)a.y * d0.y, ty = (double)a.x * d0.y + (double)a.y * d0.x;
-      v[i] = make_float2((float)(b.x * tx + b.y * ty), (float)(b.x * ty - b.y * tx));
-    } else {
-      v[i] = b;
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(dma::WAIT_LGKM0);
-  HZ_MF_TILE(0, s0)
-  HZ_MF_TILE(1, s1)
-  HZ_MF_TILE(2, s2)
-  for (int T0 = 0; T0 < TT; T0 += 4) {
-    HZ_MF_STAGE(T0, s0, s3)
-    HZ_MF_STAGE(T0 + 1, s1, s0)
-    HZ_MF_STAGE(T0 + 2, s2, s1)
-    HZ_MF_STAGE(T0 + 3, s3, s2)
-  }
-#undef HZ_MF_STAGE
-#undef HZ_MF_EPILOGUE
-#undef HZ_MF_LINE
-#undef HZ_MF_TILE
-  __builtin_amdgcn_s_waitcnt(dma::wait_vm(0));
-}
-
-template <int NX, int TCOL>
-bool try_launch_mfma8(int n, int ny, int nz, int groups, hipStream_t s, const void* G, void* x, const double2* cmy,
-                      const double2* cpy, const double2* symd, bool adjoint, int64_t n2, int64_t N, const int* fmap) {
-  if (n != NX) return false;
-  const dim3 grid((unsigned)nz, (unsigned)groups);
-  if (adjoint)
-    hipLaunchKernelGGL((k_solve_mfma8<NX, TCOL, true>), grid, dim3(dma::NT), 0, s, (const float2*)G, (float2*)x, cmy,
-                       cpy, symd, ny, n2, N, fmap);
-  else
-    hipLaunchKernelGGL((k_solve_mfma8<NX, TCOL, false>), grid, dim3(dma::NT), 0, s, (const float2*)G, (float2*)x,
-                       cmy, cpy, symd, ny, n2, N, fmap);
-  HZ_HIP(hipGetLastError());
-  return true;
-}
-
-bool launch_mfma8_any(int n, int ny, int nz, int groups, hipStream_t s, const void* G, void* x, const double2* cmy,
-                      const double2* cpy, const double2* symd, bool adjoint, int64_t n2, int64_t N, const int* fmap) {
-  return try_launch_mfma8<200, 20>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap) ||
-         try_launch_mfma8<192, 16>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap) ||
-         try_launch_mfma8<160, 20>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap) ||
-         try_launch_mfma8<128, 32>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap) ||
-         try_launch_mfma8<96, 32>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap) ||
-         try_launch_mfma8<64, 32>(n, ny, nz, groups, s, G, x, cmy, cpy, symd, adjoint, n2, N, fmap);
-}
-
 // ------------------------------------------ symmetric packed plane solve
 // D_j^{-1} M_k is complex symmetric for D_j = diag(dx(i) dy(j)), hence so is
 // K_j = G_j D_j, and G_j v = K_j (D_j^{-1} v).  The packed form keeps the upper
@@ -2455,18 +2182,26 @@ bool twist_solve_available(const hz_problem* p, int prec) {
 namespace {
 // Whether plane_solve_kernels takes the twisted solve for this call (the only
 // kernel that runs on an incomplete top-down chain): where it is asked for or
-// tuned; untuned always in complex128, and in complex64 except for 8 and more
-// right-hand sides at the widths past 96 that have a kernel of groups of 8.
+// tuned; untuned always in complex128, and in complex64 unless 8 and more
+// right-hand sides go to the groups of solve_rows, up to 208 columns.
 // One right-hand side, best kernel of before -> twisted, in ms: complex64 48^3
 // 0.234 -> 0.083, 64^3 0.167 -> 0.117, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
 // 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.55 -> 1.52, 140 x 140 x 150
 // 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.12, 128^3
 // 0.80 -> 0.35, 200^3 2.19 -> 1.55; complex128 24 x 22 x 28 0.115 -> 0.053,
 // 64^3 0.25 -> 0.15, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140 x 150
-// 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the group kernels:
+// 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the other kernels:
 // complex128 128^3 x 8 1.73 against 2.76, 192 x 192 x 100 x 8 4.8 against 7.5;
-// complex64 192^3 x 4 3.59 against 3.70, 96^3 x 8 0.53 against 0.71, but 128^3
-// x 8 1.18 against 1.08 and 192^3 x 8 6.2 against 5.0.
+// complex64 192^3 x 4 3.59 against 3.70.  Twisted against rows, complex64 x 8
+// and x 16: 64^3 0.172 / 0.190 and 0.231 / 0.194, 96^3 0.53 / 0.51 and 0.88 /
+// 0.54, 128^3 1.15 / 1.07 and 1.93 / 1.14, 140^3 2.61 / 1.62 and 4.70 / 2.95,
+// 192^3 6.25 / 3.46 and 11.6 / 6.08, 200^3 7.04 / 4.65 and 13.1 / 8.26, but 239
+// x 239 x 150 x 8 6.9 / 8.1.  A twisted solve has a workgroup per end, slot and
+// vector, and wins while these are fewer than 3 for each of the 256 compute
+// units (48^3 x 9, 450 of them: equal; 96^3 x 8, 784: rows).  That line is
+// drawn up to 96 columns; past them the rows stay on the factors that the other
+// group families also run on, so that a tuned call changes its time alone
+// (few planes pay for it: 131 x 40 x 30 x 8 0.37 against 0.19, 0.63 before).
 // Under stream capture an untuned call also takes it while the top-down chain
 // is incomplete, which cannot be completed there.
 bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
@@ -2476,16 +2211,15 @@ bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tun
   if (sk == SK_TWIST) return true;
   if (sk != SK_DEFAULT) return false;
   if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
-  if (nrhs < 8 || p->nx <= 96 || !mfma_solve_available(prec, (int)p->nx)) return true;
+  if (nrhs < 8 || !mfma_solve_available(p, prec) || p->nx > 208) return true;
+  if (p->nx <= 96 && 2 * (int64_t)p->nslot * nrhs < 768) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
   return !f.top_full && cs != hipStreamCaptureStatusNone;
 }
 }  // namespace
 
-bool mfma_solve_available(int prec, int nx) {
-  return prec == HZ_PREC_C64 && (nx == 200 || nx == 192 || nx == 160 || nx == 128 || nx == 96 || nx == 64);
-}
+bool mfma_solve_available(const hz_problem* p, int prec) { return prec == HZ_PREC_C64 && rows_available(p); }
 
 bool single_ring_available(int prec, int nx) {
   (void)prec;
@@ -2713,21 +2447,18 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
   dim3 grid((unsigned)p->nz, (unsigned)nrhs);
   SolveKernel sk = solve_kernel_choice();
   // adjoint sweeps (the tuned families are forward kernels): complex64 groups
-  // of 8 on the matrix cores with G_j^H = conj(D_j^-1 G_j D_j), the rest on the
-  // packed symmetric factors with G_j^H = conj(D_j^-1 P_j conj(.)), unless the
-  // environment asks for another kernel family
-  if (adjoint && ny >= 1 && prec == HZ_PREC_C64 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  // of 8 on the matrix cores, the rest on the packed symmetric factors with
+  // G_j^H = conj(D_j^-1 P_j conj(.)), unless the environment asks for another
+  // kernel family
+  if (adjoint && ny >= 1 && prec == HZ_PREC_C64 &&
       (sk == SK_DEFAULT || sk == SK_SYM || sk == SK_MFMA || sk == SK_TWIST)) {
-    if (sk != SK_SYM && nrhs >= 8 && mfma_solve_available(prec, n)) {
-      const int g = nrhs / 8;
-      launch_mfma8_any(n, ny, (int)p->nz, g, s, f.G.ptr, x, cmy, cpy, p->d_symd.as<double2>(), true, p->n2, p->N,
-                       p->d_fmap.as<int>());
-      nrhs -= 8 * g;
-      if (nrhs == 0) return;
-      x = reinterpret_cast<float2*>(x) + (size_t)8 * g * p->N;
-      grid = dim3((unsigned)p->nz, (unsigned)nrhs);
+    if (sk != SK_SYM && nrhs >= 8 && mfma_solve_available(p, prec)) {
+      solve_rows(p, nrhs, x, true, s);
+      return;
     }
-    if (sk != SK_MFMA && f.sym_ready && solve_sym_any(p, prec, nrhs, x, true, s)) return;
+    if (sk != SK_MFMA && f.sym_ready && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+        solve_sym_any(p, prec, nrhs, x, true, s))
+      return;
   }
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_STREAM) sk = SK_MR;
   if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_CHUNKED) sk = SK_FAST;
@@ -2746,20 +2477,20 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
 
   // untuned defaults: complex64 groups of 8 on the matrix cores, one
   // right-hand side on the single-RHS ring where they are instantiated
-  if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_DEFAULT && prec == HZ_PREC_C64 && nrhs >= 8 &&
-      mfma_solve_available(prec, n))
-    sk = SK_MFMA;
+  if (sk == SK_DEFAULT && t.solve_family == HZ_SOLVE_DEFAULT && nrhs >= 8 && mfma_solve_available(p, prec)) sk = SK_MFMA;
   if (sk == SK_DEFAULT && nrhs == 1 && single_ring_available(prec, n)) sk = SK_DMA;
-  if (!adjoint && ny >= 1 && (sk == SK_MFMA || sk == SK_MFMA_SYM) && prec == HZ_PREC_C64 && nrhs >= 8 &&
-      mfma_solve_available(prec, n) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
-    // groups of 8 on the matrix cores, the remainder on the VALU streaming
-    // kernel; HZ_SOLVE_KERNEL=mfma_sym takes the packed symmetric factors
-    // instead of the full blocks (half the bytes, the same MFMA work plus the
-    // transposed tiles' idle rows: slower at 8 right-hand sides)
+  if (sk == SK_MFMA_SYM && !f.sym_ready) sk = SK_MFMA;
+  if (!adjoint && ny >= 1 && sk == SK_MFMA && nrhs >= 8 && mfma_solve_available(p, prec)) {
+    solve_rows(p, nrhs, x, false, s);
+    return;
+  }
+  if (!adjoint && ny >= 1 && sk == SK_MFMA_SYM && prec == HZ_PREC_C64 && nrhs >= 8 && f.sym_ready &&
+      reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    // HZ_SOLVE_KERNEL=mfma_sym: groups of 8 on the packed symmetric factors
+    // (half the bytes, the same matrix products plus the transposed tiles' idle
+    // rows: slower), the remainder on the VALU streaming kernel
     const int g = nrhs / 8;
-    if (!(sk == SK_MFMA_SYM && f.sym_ready && solve_sym_mfma8_any(p, g, x, s)))
-      launch_mfma8_any(n, ny, (int)p->nz, g, s, f.G.ptr, x, cmy, cpy, p->d_symd.as<double2>(), false, p->n2, p->N,
-                       p->d_fmap.as<int>());
+    HZ_CHECK(solve_sym_mfma8_any(p, g, x, s), HZ_ERR_STATE, "no packed group kernel for nx=%d", n);
     const int rest = nrhs - 8 * g;
     if (rest == 0) return;
     x = reinterpret_cast<float2*>(x) + (size_t)8 * g * p->N;

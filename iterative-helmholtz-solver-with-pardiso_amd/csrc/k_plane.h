@@ -65,4 +65,9 @@ bool tri_available(int nx);
 void pack_tri(hz_problem* p, int prec, hipStream_t s);
 void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s);
 
+// Groups of 8 complex64 right-hand sides on the one-directional factors
+// (k_rows.hip): whether a problem has them, and the solve of nrhs vectors.
+bool rows_available(const hz_problem* p);
+void solve_rows(hz_problem* p, int nrhs, void* x, bool adjoint, hipStream_t s);
+
 }  // namespace hz
