@@ -125,15 +125,90 @@ __global__ __launch_bounds__(RT) void k_axpy_dot_partial(int64_t n, const double
 
 
 // ------------------------------------------------ one-pass Gram-Schmidt blocks
-// Multi-dot over a group of MD vectors: r_q = V_q^H w and (vj != nullptr)
-// l_q = V_q^H vj for q in the group; partial[(group * RB + block) * 2 MD + ...].
+// Multi-dot over a group of MD vectors: r_q = V_q^H w and l_q = V_q^H vj for q
+// in the group; partial[(group * blocks + block) * 2 MD + ...].
 constexpr int MD = 12;
 
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+// Sums of 16 H values over the 64 lanes: lane l ends with the sums of values
+// H (l / 4) .. + H - 1.  Each of the first four exchanges also halves what a
+// lane holds, the first two as swaps of half waves and of rows of 16 lanes:
+// 36 swaps and 15 shuffles of doubles for 48 values instead of 288 shuffles.
+template <bool ROWS>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const unsigned xl = (unsigned)x, xh = (unsigned)(x >> 32), yl = (unsigned)y, yh = (unsigned)(y >> 32);
+  const auto lo = ROWS ? __builtin_amdgcn_permlane16_swap(xl, yl, false, false)
+                       : __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
+  const auto hi = ROWS ? __builtin_amdgcn_permlane16_swap(xh, yh, false, false)
+                       : __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
+  const unsigned l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+  return __builtin_bit_cast(double, (uint64_t)h0 << 32 | l0) + __builtin_bit_cast(double, (uint64_t)h1 << 32 | l1);
 }
 
+template <int H>
+__device__ __forceinline__ void wave_sums(double (&v)[16 * H], int lane) {
+#pragma unroll
+  for (int i = 0; i < 8 * H; ++i) v[i] = swap_add<false>(v[i], v[8 * H + i]);
+#pragma unroll
+  for (int i = 0; i < 4 * H; ++i) v[i] = swap_add<true>(v[i], v[4 * H + i]);
+#pragma unroll
+  for (int c = 2 * H, m = 8; m >= 4; c /= 2, m /= 2)
+#pragma unroll
+    for (int i = 0; i < c; ++i) {
+      const bool up = lane & m;
+      v[i] = (up ? v[c + i] : v[i]) + __shfl_xor(up ? v[i] : v[c + i], m);
+    }
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    v[i] += __shfl_xor(v[i], 2);
+    v[i] += __shfl_xor(v[i], 1);
+  }
+}
+
+// One block's partials of a group of up to 4 H vectors: the loads of all 4 H
+// (past the group's end its last vector again) leave together, the loop waits
+// on them once.
+template <int H>
+__device__ __forceinline__ void multidot_block(int64_t n, int nq, const double2* __restrict__ V, int64_t vs,
+                                               const double2* __restrict__ w, const double2* __restrict__ vj,
+                                               double2* __restrict__ out, double (&sm)[RT / 64][MD * 4]) {
+  double acc[16 * H];  // of vector g: r, l (re, im) at 4 g
+#pragma unroll
+  for (int i = 0; i < 16 * H; ++i) acc[i] = 0.0;
+  const int64_t stride = (int64_t)gridDim.x * RT;
+  for (int64_t l = (int64_t)blockIdx.x * RT + threadIdx.x; l < n; l += stride) {
+    const double2 wv = w[l], jv = vj[l];
+    double2 a[4 * H];
+#pragma unroll
+    for (int g = 0; g < 4 * H; ++g) a[g] = ldv(V + (int64_t)min(g, nq - 1) * vs + l);
+#pragma unroll
+    for (int g = 0; g < 4 * H; ++g) {
+      acc[4 * g] += a[g].x * wv.x + a[g].y * wv.y;
+      acc[4 * g + 1] += a[g].x * wv.y - a[g].y * wv.x;
+      acc[4 * g + 2] += a[g].x * jv.x + a[g].y * jv.y;
+      acc[4 * g + 3] += a[g].x * jv.y - a[g].y * jv.x;
+    }
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  wave_sums<H>(acc, lane);
+  if ((lane & 3) == 0)
+#pragma unroll
+    for (int i = 0; i < H; ++i) sm[wave][H * (lane >> 2) + i] = acc[i];
+  __syncthreads();
+  if (threadIdx.x < 16 * H) {
+    double t = 0.0;
+    for (int i = 0; i < RT / 64; ++i) t += sm[i][threadIdx.x];
+    // layout: [r_0..r_{MD-1}, l_0..l_{MD-1}] as double2
+    const int g = threadIdx.x / 4, c = threadIdx.x % 4;
+    reinterpret_cast<double*>(out)[2 * ((c < 2) ? g : MD + g) + (c & 1)] = t;
+  }
+}
+
+// What bounds it: the vectors' bytes, and the sums over 48 values that each
+// block adds, so small vectors take fewer blocks (multidot_blocks).  Mean over
+// a solve's steps: 48^3, 4 members, restart 40 223 -> 28 us (5 TB/s); 64^3,
+// restart 35 61 -> 18; before, 1024 blocks at every length, full butterflies,
+// and a wait for each vector's load.
 __global__ __launch_bounds__(RT) void k_multidot_partial(int64_t n, int nv, const double2* __restrict__ V,
                                                          int64_t vs, const double2* __restrict__ w,
                                                          const double2* __restrict__ vj,
@@ -141,49 +216,15 @@ __global__ __launch_bounds__(RT) void k_multidot_partial(int64_t n, int nv, cons
                                                          uint64_t mask) {
   // blockIdx.z: a batch member (vectors ms, partials ps apart; members not in mask skip)
   if (!((mask >> blockIdx.z) & 1ull)) return;
-  V += (int64_t)blockIdx.z * ms;
-  w += (int64_t)blockIdx.z * ms;
-  if (vj) vj += (int64_t)blockIdx.z * ms;
-  partial += (int64_t)blockIdx.z * ps;
-  const int group = blockIdx.y;
-  const int q0 = group * MD;
-  const int nq = min(MD, nv - q0);
-  double ar[MD][2], al[MD][2];
-#pragma unroll
-  for (int g = 0; g < MD; ++g) { ar[g][0] = ar[g][1] = al[g][0] = al[g][1] = 0.0; }
-  const int64_t stride = (int64_t)RB * RT;
-  for (int64_t l = (int64_t)blockIdx.x * RT + threadIdx.x; l < n; l += stride) {
-    const double2 wv = w[l];
-    const double2 jv = vj ? vj[l] : make_double2(0, 0);
-#pragma unroll
-    for (int g = 0; g < MD; ++g) {
-      if (g < nq) {
-        const double2 a = ldv(V + (int64_t)(q0 + g) * vs + l);
-        ar[g][0] += a.x * wv.x + a.y * wv.y;
-        ar[g][1] += a.x * wv.y - a.y * wv.x;
-        al[g][0] += a.x * jv.x + a.y * jv.y;
-        al[g][1] += a.x * jv.y - a.y * jv.x;
-      }
-    }
-  }
   __shared__ double sm[RT / 64][MD * 4];
-  const int lane = threadIdx.x & 63, wv_ = threadIdx.x >> 6;
-#pragma unroll
-  for (int g = 0; g < MD; ++g) {
-    const double s0 = wave_sum(ar[g][0]), s1 = wave_sum(ar[g][1]);
-    const double s2 = wave_sum(al[g][0]), s3 = wave_sum(al[g][1]);
-    if (lane == 0) { sm[wv_][4 * g] = s0; sm[wv_][4 * g + 1] = s1; sm[wv_][4 * g + 2] = s2; sm[wv_][4 * g + 3] = s3; }
-  }
-  __syncthreads();
-  if (threadIdx.x < MD * 4) {
-    double t = 0.0;
-    for (int i = 0; i < RT / 64; ++i) t += sm[i][threadIdx.x];
-    // layout: [r_0..r_{MD-1}, l_0..l_{MD-1}] as double2
-    const int g = threadIdx.x / 4, c = threadIdx.x % 4;
-    double* out = reinterpret_cast<double*>(partial + ((int64_t)group * RB + blockIdx.x) * 2 * MD);
-    const int slot = (c < 2) ? g : MD + g;
-    out[2 * slot + (c & 1)] = t;
-  }
+  const int q0 = blockIdx.y * MD, nq = min(MD, nv - q0);
+  V += (int64_t)blockIdx.z * ms + (int64_t)q0 * vs;
+  w += (int64_t)blockIdx.z * ms;
+  vj += (int64_t)blockIdx.z * ms;
+  partial += (int64_t)blockIdx.z * ps + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 2 * MD;
+  if (nq > 8) multidot_block<3>(n, nq, V, vs, w, vj, partial, sm);
+  else if (nq > 4) multidot_block<2>(n, nq, V, vs, w, vj, partial, sm);
+  else multidot_block<1>(n, nq, V, vs, w, vj, partial, sm);
 }
 
 __device__ __forceinline__ double basis_scale(const double2* S, int k) { return k == 0 ? 1.0 : S[k].x; }
@@ -193,7 +234,7 @@ __device__ __forceinline__ double basis_scale(const double2* S, int k) { return 
 __global__ __launch_bounds__(RT) void k_multidot_final(const double2* __restrict__ partial, int nv,
                                                        double2* __restrict__ out_r, double2* __restrict__ out_l,
                                                        int64_t ps, int64_t os, uint64_t mask,
-                                                       const double2* __restrict__ S, int jv) {
+                                                       const double2* __restrict__ S, int jv, int nb) {
   if (!((mask >> blockIdx.z) & 1ull)) return;
   partial += (int64_t)blockIdx.z * ps;
   out_r += (int64_t)blockIdx.z * os;
@@ -202,8 +243,8 @@ __global__ __launch_bounds__(RT) void k_multidot_final(const double2* __restrict
   const int q = blockIdx.x;
   const int group = q / MD, g = q % MD;
   double sx = 0, sy = 0, tx = 0, ty = 0;
-  for (int b = threadIdx.x; b < RB; b += RT) {
-    const double2* pb = partial + ((int64_t)group * RB + b) * 2 * MD;
+  for (int b = threadIdx.x; b < nb; b += RT) {
+    const double2* pb = partial + ((int64_t)group * nb + b) * 2 * MD;
     sx += pb[g].x; sy += pb[g].y;
     tx += pb[MD + g].x; ty += pb[MD + g].y;
   }
@@ -653,6 +694,12 @@ void launch_scale_inv_guard(int64_t n, const double2* coef, double thr, const do
   HZ_HIP(hipGetLastError());
 }
 
+// blocks of the multi-dot pass of one member and group, by the vectors' length
+// alone: the sums' order is the same in every batch
+static int multidot_blocks(int64_t n) {
+  return (int)std::min<int64_t>(RB, std::max<int64_t>((n + 4 * RT - 1) / (4 * RT), std::min<int64_t>(64, (n + RT - 1) / RT)));
+}
+
 void launch_gs_members(hz_problem* p, int64_t n, int nr, uint64_t mask, int j, int m, int ldh, const double2* V,
                        int64_t vs, const double2* w, double2* mem, int64_t msz, int offR, int offL, int offLg,
                        int offH, int offS, int offCS, int offSN, int offG, const double2* beta, const double2* nf,
@@ -662,15 +709,16 @@ void launch_gs_members(hz_problem* p, int64_t n, int nr, uint64_t mask, int j, i
   HZ_CHECK(nr >= 1 && nr <= 64, HZ_ERR_ARG, "%d batch members (at most 64)", nr);
   const int nv = j + 1;
   const int ng = (nv + MD - 1) / MD;
-  const int64_t ps = (int64_t)ng * RB * 2 * MD;  // multi-dot partials of one member
+  const int nb = multidot_blocks(n);
+  const int64_t ps = (int64_t)ng * nb * 2 * MD;  // multi-dot partials of one member
   HZ_CHECK(p->red.bytes >= (size_t)nr * (size_t)std::max<int64_t>(ps, RBA) * sizeof(double2), HZ_ERR_STATE,
            "reduction workspace not sized for %d members", nr);
   double2* red = p->red.as<double2>();
   double2* h = mem + offH + (int64_t)ldh * j;
-  hipLaunchKernelGGL(k_multidot_partial, dim3(RB, ng, nr), dim3(RT), 0, s, n, nv, V, vs, w, V + (int64_t)j * vs, red,
+  hipLaunchKernelGGL(k_multidot_partial, dim3(nb, ng, nr), dim3(RT), 0, s, n, nv, V, vs, w, V + (int64_t)j * vs, red,
                      n, ps, mask);
   hipLaunchKernelGGL(k_multidot_final, dim3(nv, 1, nr), dim3(RT), 0, s, red, nv, mem + offR, mem + offL, ps, msz,
-                     mask, mem + offS, j);
+                     mask, mem + offS, j, nb);
   hipLaunchKernelGGL(k_icwy, dim3(1, 1, nr), dim3(64), (size_t)nv * nv * sizeof(double2), s, j, ldh, mem + offR,
                      mem + offL, mem + offLg, h, msz, mask);
   hipLaunchKernelGGL(k_multi_axpy_norm_partial, dim3(RBA, 1, nr), dim3(RT), nv * sizeof(double2), s, n, nv, V, vs, h,
