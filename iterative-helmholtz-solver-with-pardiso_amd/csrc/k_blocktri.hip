@@ -2185,21 +2185,21 @@ namespace {
 // tuned; untuned always in complex128, and in complex64 unless 8 and more
 // right-hand sides go to the groups of solve_rows, up to 208 columns.
 // One right-hand side, best kernel of before -> twisted, in ms: complex64 48^3
-// 0.234 -> 0.083, 64^3 0.167 -> 0.117, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
+// 0.234 -> 0.063, 64^3 0.167 -> 0.093, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
 // 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.55 -> 1.52, 140 x 140 x 150
-// 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.12, 128^3
-// 0.80 -> 0.35, 200^3 2.19 -> 1.55; complex128 24 x 22 x 28 0.115 -> 0.053,
-// 64^3 0.25 -> 0.15, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140 x 150
+// 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.10, 128^3
+// 0.80 -> 0.35, 200^3 2.19 -> 1.55; complex128 24 x 22 x 28 0.115 -> 0.044,
+// 64^3 0.25 -> 0.11, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140 x 150
 // 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the other kernels:
 // complex128 128^3 x 8 1.73 against 2.76, 192 x 192 x 100 x 8 4.8 against 7.5;
 // complex64 192^3 x 4 3.59 against 3.70.  Twisted against rows, complex64 x 8
-// and x 16: 64^3 0.172 / 0.190 and 0.231 / 0.194, 96^3 0.53 / 0.51 and 0.88 /
+// and x 16: 64^3 0.16 / 0.19 and 0.245 / 0.194, 96^3 0.53 / 0.51 and 0.88 /
 // 0.54, 128^3 1.15 / 1.07 and 1.93 / 1.14, 140^3 2.61 / 1.62 and 4.70 / 2.95,
 // 192^3 6.25 / 3.46 and 11.6 / 6.08, 200^3 7.04 / 4.65 and 13.1 / 8.26, but 239
 // x 239 x 150 x 8 6.9 / 8.1.  A twisted solve has a workgroup per end, slot and
-// vector, and wins while these are fewer than 3 for each of the 256 compute
-// units (48^3 x 9, 450 of them: equal; 96^3 x 8, 784: rows).  That line is
-// drawn up to 96 columns; past them the rows stay on the factors that the other
+// vector, and wins while these are fewer than about 4 for each of the 256
+// compute units (48^3 x 16, 800 of them: 0.110 / 0.122; 64^3 x 16, 1056: rows).
+// That line is drawn up to 96 columns; past them the rows stay on the factors that the other
 // group families also run on, so that a tuned call changes its time alone
 // (few planes pay for it: 131 x 40 x 30 x 8 0.37 against 0.19, 0.63 before).
 // Under stream capture an untuned call also takes it while the top-down chain
@@ -2212,7 +2212,7 @@ bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tun
   if (sk != SK_DEFAULT) return false;
   if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
   if (nrhs < 8 || !mfma_solve_available(p, prec) || p->nx > 208) return true;
-  if (p->nx <= 96 && 2 * (int64_t)p->nslot * nrhs < 768) return true;
+  if (p->nx <= 96 && 2 * (int64_t)p->nslot * nrhs < 1024) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
   return !f.top_full && cs != hipStreamCaptureStatusNone;

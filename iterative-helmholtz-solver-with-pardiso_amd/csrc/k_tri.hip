@@ -22,7 +22,7 @@
 // its 16 x 16 tiles, taken round the diagonals: tile row R holds the tile
 // columns R, R + 1, ... (mod NT), NT/2 + 1 of them (even NT: NT/2 where R >=
 // NT/2), so every pair of tiles (R, C), (C, R) is kept once and every wave gets
-// the same static program: rows w and w + NW.  Tiles go straight from memory
+// the same static program: rows w and w + NW, or row w alone.  Tiles go straight from memory
 // into registers: lane 4 b + i holds row 4 (b & 3) + i and the four columns
 // 4 (b >> 2) .. + 3 (two 16-byte units), so a load instruction reads 1 KB in
 // order.  Each value serves both products on the matrix cores
@@ -46,13 +46,15 @@
 // about 60 instructions a tile.  A slot's registers are refilled with the next
 // block's tile as soon as they are read, so a whole block (186 KB at 200
 // columns) is in flight per CU across the two barriers of a step; the loads do
-// not depend on the vector.  At 200^3 a solve takes 1.52 ms = 7.5 GB at 4.95
-// TB/s, the rate of a large device copy there (the products and barriers alone,
-// without the loads: 1.00 ms); at 64^3 0.117 ms, 1.8 us a step, of which 0.8 us
-// are barriers, sums and the update.  complex128 at 200^3 2.87 ms (15.0 GB, 5.2
-// TB/s), at 140 x 140 x 150 0.92 ms.  Measured against it: the kernel it
-// replaced at 128, 160, 192 and 200 columns (tiles through an LDS ring per
-// wave) 0.55, 0.81, 1.33 and 1.55 ms against 0.34, 0.71, 1.23 and 1.52.
+// not depend on the vector.  Small grids are bound by a step's two barriers, its
+// sums and its update, some 0.6 us, so what the update can know before the
+// products is formed before them.  At 200^3 a solve takes 1.52 ms = 7.5 GB at
+// 4.95 TB/s, the rate of a large device copy there (the products and barriers
+// alone, without the loads: 1.00 ms); at 64^3 0.093 ms, 1.2 us a step.
+// complex128 at 200^3 2.87 ms (15.0 GB, 5.2 TB/s), at 140 x 140 x 150 0.92 ms.
+// Measured against it: the kernel it replaced at 128, 160, 192 and 200 columns
+// (tiles through an LDS ring per wave) 0.55, 0.81, 1.33 and 1.55 ms against
+// 0.34, 0.71, 1.23 and 1.52.
 #include <type_traits>
 
 #include "hz_internal.h"
@@ -138,18 +140,27 @@ struct TriShape {
   static constexpr int NA = NT / 2 + 1;    // tiles of row w
   static constexpr int NB = NT - NT / 2;   // tiles of row w + NW
   static constexpr int NS = NA + NB;       // NT + 1
-  static constexpr int THREADS = 64 * NW;  // >= 2 * 16 NT: one thread per (plane, row) in the update
+  // up to 4 tile rows: a wave for each row, NA tiles each (a row of NB < NA: its
+  // last one is dead), so that the four SIMDs of a compute unit share them.
+  // 48^3 0.081 -> 0.063 ms, 64^3 0.114 -> 0.094, x 7 0.172 -> 0.133; complex128
+  // 64^3 0.145 -> 0.109.  Past 4 the SIMDs have no fewer tiles each: one vector
+  // gained (96^3 0.206 -> 0.195, 112^3 0.274 -> 0.229), but several on a compute
+  // unit lost (96^3 x 4 0.32 -> 0.38, 128^3 x 4 0.74 -> 0.86).
+  static constexpr bool SPLIT = NT <= 4;
+  static constexpr int WAVES = SPLIT ? NT : NW;
+  static constexpr int NSW = SPLIT ? NA : NS;  // tiles a wave
+  static constexpr int THREADS = 64 * WAVES;   // >= 2 * 16 NT: one thread per (plane, row) in the update
   static constexpr int NP = 64 * ((16 * NT - 16 + 63) / 64) + 16;  // values a component: 16 mod 64, the four
                                                                    // components' reads fall in distinct banks
   // tiles in flight a wave: a whole block's, or (complex128, whose tiles take
   // 16 registers) a half or a third of them where they would not fit
-  static constexpr int RD = sizeof(T) == 4 || NS <= 9 ? NS : NS <= 11 ? (NS + 1) / 2 : (NS + 2) / 3;
-  static constexpr int NSR = (NS + RD - 1) / RD * RD;  // slots of a block, the last possibly empty
+  static constexpr int RD = sizeof(T) == 4 || NS <= 9 ? NSW : NS <= 10 ? (NS + 1) / 2 : (NS + 2) / 3;
+  static constexpr int NSR = (NSW + RD - 1) / RD * RD;  // slots of a block, the last possibly empty
   static constexpr size_t lds = sizeof(T) * (8 * (size_t)NP + 64 * ((size_t)(NT + 1) * NA + NT + 1));
 };
 
 template <typename T, int NT, int PH, bool ADJ>
-__global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
+__global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
     const typename Cx<T>::t* __restrict__ P, typename Cx<T>::t* __restrict__ X, const double2* __restrict__ cmy,
     const double2* __restrict__ cpy, const double2* __restrict__ symd, int n, int ny, int m, int nz, int64_t n2,
     int64_t N, const int2* __restrict__ slotp, int nslot, int nrhs, typename Cx<T>::t* __restrict__ scr) {
@@ -205,30 +216,37 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
   auto scr_at = [&](int what) { return scr + (((int64_t)what * nrhs + rhs) * nz + pl) * n + pr; };
   const double2 dxr = dx[pr], dxir = dxi[pr];
   auto cmul_d = [](double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
+  // Values of the lines' tables are fetched a step ahead by vector loads: scalar
+  // loads would be waited for with the step's first LDS reads.
+  int vz;
+  asm("v_mov_b32 %0, 0" : "=v"(vz));
   // a line value of the right-hand side: f, or D conj(f) for the adjoint
-  auto load_f = [&](C f, int j) {
+  auto load_f = [&](C f, double2 dyj) {
     if (!ADJ) return f;
-    const double2 d = cmul_d(dxr, dy[j]);
+    const double2 d = cmul_d(dxr, dyj);
     const double2 v = cmul_d(make_double2(f.x, -(double)f.y), d);
     return mk<C>(v.x, v.y);
   };
 
-  if (PH == 0 && half == 0 && wr) *scr_at(2) = load_f(xs[(int64_t)m * n], m);
+  if (PH == 0 && half == 0 && wr) *scr_at(2) = load_f(xs[(int64_t)m * n], dy[m]);
   if (nsteps <= 0) return;
 
   // ---- this wave's tiles: NA of row ra, NB of row rb.  (The last wave of an
   // odd NT has no second row: it computes some row's first tiles once more,
   // into sums that nobody reads.)
   const int ra = w, rb = w + S::NW < NT ? w + S::NW : w;
-  const bool spare = w + S::NW >= NT;
+  const bool spare = S::SPLIT ? w >= S::NW && S::NB < S::NA : w + S::NW >= NT;
+  // the first slot of a wave that holds no tile of its own, where spare
+  constexpr int SP0 = S::SPLIT ? S::NB : S::NA;
   constexpr int UL = F32 ? 2 : 1, UQ = F32 ? 2 : 4;  // complex values a unit, units a lane and tile
-  const C* const tiles = Pk + (size_t)w * S::NS * 256 + UL * lane;
+  const C* const tiles =
+      Pk + (S::SPLIT && w >= S::NW ? (size_t)(w - S::NW) * S::NS + S::NA : (size_t)w * S::NS) * 256 + UL * lane;
   struct alignas(16) Unit { C c[UL]; };
   Unit q[S::RD][UQ];
   // (no branch around a load: with one, the compiler cannot count the younger
   // loads in flight and waits for all of them before each tile)
   auto load_slot = [&](int t, const C* blk) {
-    const C* const a = blk + (spare && t >= S::NA ? t - S::NA : t) * 256;
+    const C* const a = blk + (spare && t >= SP0 ? t - SP0 : t) * 256;
 #pragma unroll
     for (int u = 0; u < UQ; ++u) q[t % S::RD][u] = *reinterpret_cast<const Unit*>(a + u * 64 * UL);
   };
@@ -255,7 +273,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
     const int j0 = blk_of(0);
     double2 f;
     if (PH == 0) {
-      const C v = load_f(xs[(int64_t)j0 * n], j0);
+      const C v = load_f(xs[(int64_t)j0 * n], dy[j0]);
       if (ADJ && wr) xs[(int64_t)j0 * n] = v;
       f = make_double2(v.x, v.y);
     } else {
@@ -278,6 +296,22 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
   }
   __syncthreads();
 
+  // what the update after step st takes of its next line jn: the line's value,
+  // its coefficient, 1 / dy(jn) and (adjoint, first phase) dy(jn)
+  struct Line { C f; double2 cf, di, d; };
+  const bool lower = PH == 0 ? half == 0 : half != 0;
+  auto fetch = [&](int st) {
+    const int jn = next_of(st), j = jn >= 0 ? jn : blk_of(st);
+    Line l;
+    l.f = xs[(int64_t)j * n];
+    l.cf = (lower ? cmy : cpy)[j + vz];
+    l.di = dyi[j + vz];
+    if (ADJ && PH == 0) l.d = dy[j + vz];
+    return l;
+  };
+  Line line = fetch(0);
+  double2 sb = cmul_d(dxir, dyi[blk_of(0)]);  // D^-1 of this row, block jb
+
   for (int st = 0; st < nsteps; ++st) {
     const int jb = blk_of(st), jn = next_of(st);
     const C* const cblk = tiles + (size_t)jb * BS;
@@ -286,7 +320,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
     // the next block's)
     auto reload = [&](int t) {
       int u = t + S::RD;
-      if (u < S::NS) {
+      if (u < S::NSW) {
         load_slot(u, cblk);
       } else {
         if (u < S::NSR) u += S::RD;
@@ -294,10 +328,16 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
       }
     };
     auto col_of = [&](int t) {
+      // a dead tile: the vector's zeros past the last column
+      if (S::SPLIT && spare && t >= SP0) return NP / 16 - 1;
       const int c = t < S::NA ? ra + t : rb + t - S::NA;
       return c < NT ? c : c - NT;
     };
-    const C pre = xs[(int64_t)(jn >= 0 ? jn : jb) * n];
+    // v' = D^-1 (f - cf y) = ef - ec y, all but y known before the products
+    const C f = PH == 0 ? load_f(line.f, line.d) : line.f;
+    const double2 cf = line.cf, sn = cmul_d(dxir, line.di);
+    const double2 ef = cmul_d(sn, make_double2(f.x, f.y)), ec = cmul_d(sn, cf);
+    line = fetch(st + 1 < nsteps ? st + 1 : st);
 
     if constexpr (F32) {
       // Software pipeline over the tiles, one scheduling region each: tile t's
@@ -321,9 +361,9 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
       };
       load_col(0);
   #pragma unroll
-      for (int t = 0; t < S::NS + 2; ++t) {
-        if (t + 1 < S::NS) load_col(t + 1);
-        if (t < S::NS) {
+      for (int t = 0; t < S::NSW + 2; ++t) {
+        if (t + 1 < S::NSW) load_col(t + 1);
+        if (t < S::NSW) {
           float kr[4], ki[4];
   #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -349,7 +389,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
           }
           reload(t);
         }
-        if (t >= 1 && t <= S::NS) {
+        if (t >= 1 && t <= S::NSW) {
           const int u = t - 1;
           const float4 a = u < S::NA ? va : wa, b = u < S::NA ? vb : wb;
           // the diagonal tiles' own 4 x 4 blocks have no transposed product
@@ -370,7 +410,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
           const int u = t - 2;
           const hz_v4f x = ts[u & 1];
           const float s = tri_pair<0x128>(tri_pair<0x124>(x[0], x[1], b2), tri_pair<0x124>(x[2], x[3], b2), b3);
-          const int d = u < S::NA ? u : u - S::NA, at = u < S::NA || !spare ? col_of(u) : NT;
+          const int d = u < S::NA ? u : u - S::NA, at = u < SP0 || !spare ? col_of(u) : NT;
           tsum[64 * (at * S::NA + d) + (rg >> 1) * 32 + (4 * cg + qi) * 2 + (rg & 1)] = s;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -380,7 +420,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
         const hz_v4f a = da0 + da1, b = db0 + db1;
         const int at = (qi >> 1) * 32 + (4 * rg + cg) * 2 + (qi & 1);
         dsum[64 * ra + at] = tri_sum32(tri_sum16(a[0], a[1]), tri_sum16(a[2], a[3]));
-        dsum[64 * (spare ? NT : rb) + at] = tri_sum32(tri_sum16(b[0], b[1]), tri_sum16(b[2], b[3]));
+        if (!S::SPLIT) dsum[64 * (spare ? NT : rb) + at] = tri_sum32(tri_sum16(b[0], b[1]), tri_sum16(b[2], b[3]));
       }
     } else {
       const int i4 = lane >> 4;  // k of an operand, i of a result
@@ -401,7 +441,7 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
       };
       row_operands(ra);
 #pragma unroll
-      for (int t = 0; t < S::NS; ++t) {
+      for (int t = 0; t < S::NSW; ++t) {
         if (t == S::NA) {
           flush_row(ra);
           row_operands(rb);
@@ -427,11 +467,11 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
           x = __builtin_amdgcn_mfma_f64_4x4x4f64(off ? va[p] : 0.0, kr[p], x, 0, 0, 0);
           x = __builtin_amdgcn_mfma_f64_4x4x4f64(off ? vb[p] : 0.0, ki[p], x, 0, 0, 0);
         }
-        const int at = t < S::NA || !spare ? cc : NT;
+        const int at = t < SP0 || !spare ? cc : NT;
         tsum[64 * (at * S::NA + d) + (i4 >> 1) * 32 + (4 * rg + qi) * 2 + (i4 & 1)] = x;
         __builtin_amdgcn_sched_barrier(0);  // the reloads stay in order
       }
-      flush_row(spare ? NT : rb);
+      flush_row(S::SPLIT ? ra : spare ? NT : rb);
     }
     __syncthreads();
 
@@ -446,26 +486,25 @@ __global__ __launch_bounds__(64 * ((NT + 1) / 2)) void k_solve_tri(
         y.x += kept ? u.x : (T)0;
         y.y += kept ? u.y : (T)0;
       }
+      if (jn >= 0)
+        put_v(make_double2(ef.x - (ec.x * y.x - ec.y * y.y), ef.y - (ec.x * y.y + ec.y * y.x)));
       if (wr && PH == 1 && (half == 0 || st > 0)) {  // x_jb
         C o = y;
         if (ADJ) {
-          const double2 z = cmul_d(make_double2(y.x, y.y), cmul_d(dxir, dyi[jb]));
+          const double2 z = cmul_d(make_double2(y.x, y.y), sb);
           o = mk<C>(z.x, -z.y);
         }
         xs[(int64_t)jb * n] = o;
       }
       if (wr && jn == -2) *scr_at(half) = y;  // y_top / y_bot
-      if (jn >= 0) {
-        const bool lower = PH == 0 ? half == 0 : half != 0;
-        const double2 cf = lower ? cmy[jn] : cpy[jn];
-        const C f = PH == 0 ? load_f(pre, jn) : pre;
+      if (wr && PH == 0 && jn >= 0) {         // t_jn / b_jn
         C nv;
         nv.x = f.x - (T)(cf.x * y.x - cf.y * y.y);
         nv.y = f.y - (T)(cf.x * y.y + cf.y * y.x);
-        if (wr && PH == 0) xs[(int64_t)jn * n] = nv;  // t_jn / b_jn
-        put_v(cmul_d(make_double2(nv.x, nv.y), cmul_d(dxir, dyi[jn])));
+        xs[(int64_t)jn * n] = nv;
       }
     }
+    sb = sn;
     __syncthreads();
   }
 }
