@@ -142,13 +142,13 @@ enum {
   HZ_SOLVE_STREAM_MFMA = 4, /* streaming solve with the block products of groups of 8 RHS on FP32 MFMA (complex64) */
   HZ_SOLVE_SYM = 5,         /* symmetric packed factors (upper block triangle of G_j D_j), one RHS per pass */
   HZ_SOLVE_TWIST = 6        /* twisted packed factors (chains from both ends meeting at y-line ny/2), the
-                               two planes of each factor slot per pass (complex64) */
+                               two planes of each factor slot per pass; up to 256 columns */
 };
 typedef struct {
   int32_t solve_kernel; /* HZ_SOLVE_* */
   int32_t group_cap;    /* right-hand sides per streaming pass: 8, 4, 2 or 1 */
   int32_t fft_lines;    /* (x,y) lines per z-FFT workgroup: 8, 16 or 32 (LDS Stockham), 0 for the
-                           register-resident kernel of nz = 64, 96, 128, 160, 192, 200 */
+                           register-resident kernels (nz a product of two small factors) */
   int32_t from_cache;   /* 1 when read from the HZ_TUNE_CACHE file */
   double solve_ms;      /* plane solve of nrhs vectors with the choice */
   double fft_ms;        /* one forward z-FFT of nrhs vectors with the choice */

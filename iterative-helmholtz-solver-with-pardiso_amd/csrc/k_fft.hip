@@ -7,8 +7,11 @@
 // between complex128 and complex64 and fusing the reference's
 // g = w - deltaL * (L0^{-1} w) epilogue into the backward pass
 // (functions.cpp:5571-5574).  Forward is unscaled with e^{-2 pi i jk/n},
-// backward scales by 1/n (DFTI settings of functions.cpp:5864-5869).
+// backward scales by 1/n (DFTI settings of functions.cpp:5864-5869).  Lengths
+// that are a product of two factors small enough for registers take one of the
+// register-resident kernels instead.
 #include <cstdlib>
+#include <type_traits>
 
 #include "hz_internal.h"
 
@@ -269,7 +272,32 @@ struct RegDft {
       const C i2 = cmul_si(csub(cscale(d1, s2), cscale(d2, s1)), SIGN);
       v[0] = cadd(a0, cadd(b1, b2)); v[1] = cadd(r1, i1); v[4] = csub(r1, i1); v[2] = cadd(r2, i2); v[3] = csub(r2, i2);
     } else {
-      static_assert(N <= 5, "in-register DFT: unsupported prime factor");
+      // odd primes: the sums and differences of j and N - j
+      static_assert(N == 7 || N == 11 || N == 13, "in-register DFT: unsupported prime factor");
+      constexpr int H = (N - 1) / 2;
+      const C a0 = v[0];
+      C b[H], d[H], sum = a0;
+#pragma unroll
+      for (int j = 0; j < H; ++j) {
+        b[j] = cadd(v[1 + j], v[N - 1 - j]);
+        d[j] = csub(v[1 + j], v[N - 1 - j]);
+        sum = cadd(sum, b[j]);
+      }
+      v[0] = sum;
+#pragma unroll
+      for (int k = 1; k <= H; ++k) {
+        C re = a0, im;
+        im.x = 0; im.y = 0;
+#pragma unroll
+        for (int j = 1; j <= H; ++j) {
+          const double ang = 2.0 * 3.14159265358979323846 * (double)(j * k % N) / (double)N;
+          re = cadd(re, cscale(b[j - 1], (T)cos(ang)));
+          im = cadd(im, cscale(d[j - 1], (T)sin(ang)));
+        }
+        im = cmul_si(im, SIGN);
+        v[k] = cadd(re, im);
+        v[N - k] = csub(re, im);
+      }
     }
   }
 };
@@ -358,7 +386,7 @@ bool try_fft_reg(hz_problem* p, int sign, int nrhs, const void* in, void* out, c
   return true;
 }
 
-// lengths of the configurations: 64 = 8 x 8, 96 = 8 x 12, 128 = 8 x 16,
+// lengths with a kernel of their own (larger line groups): 64 = 8 x 8, 96 = 8 x 12, 128 = 8 x 16,
 // 160 = 10 x 16, 192 = 12 x 16, 200 = 8 x 25
 template <typename T, typename TI, typename TO, int EPI>
 bool launch_reg(hz_problem* p, int sign, int nrhs, const void* in, void* out, const double2* w, const double2* dL,
@@ -369,6 +397,135 @@ bool launch_reg(hz_problem* p, int sign, int nrhs, const void* in, void* out, co
          try_fft_reg<T, TI, TO, EPI, 8, 16>(p, sign, nrhs, in, out, w, dL, s) ||
          try_fft_reg<T, TI, TO, EPI, 8, 12>(p, sign, nrhs, in, out, w, dL, s) ||
          try_fft_reg<T, TI, TO, EPI, 8, 8>(p, sign, nrhs, in, out, w, dL, s);
+}
+
+// ---- any other length that is a product of two register transforms: the same
+// two steps with the factors na <= nb chosen at run time (uniform branches to
+// one body per factor).  What bounds it: one pass over the vectors; the general
+// kernel above reads and writes LDS once per prime factor with run-time strides.
+// Call times in us (some 20 of them the launch and the wait), general -> this:
+// complex128 24 x 22 x 28 29 -> 23, 100^3 52 -> 25, 140 x 140 x 150 115 -> 36,
+// x 8 821 -> 159 (4.7 TB/s), 200 x 200 x 143 206 -> 48; complex64 150 x 8 418 ->
+// 158, 48^3 x 4 29 -> 24.  Faster at every length tried.  complex64 below 32
+// points keeps the general kernel's rounding: a launch there is mostly latency
+// (28 points 28 -> 23 with its wait), and solves of hundreds of steps on such
+// grids count their iterations to +-1 between equal problems.
+template <typename F>
+__device__ __forceinline__ void with_factor(int n, F&& f) {
+  switch (n) {
+#define HZ_FACTOR(K) case K: f(std::integral_constant<int, K>{}); break;
+    HZ_FACTOR(2) HZ_FACTOR(3) HZ_FACTOR(4) HZ_FACTOR(5) HZ_FACTOR(6) HZ_FACTOR(7) HZ_FACTOR(8) HZ_FACTOR(9)
+    HZ_FACTOR(10) HZ_FACTOR(11) HZ_FACTOR(12) HZ_FACTOR(13) HZ_FACTOR(14) HZ_FACTOR(15) HZ_FACTOR(16) HZ_FACTOR(18)
+    HZ_FACTOR(20)
+#undef HZ_FACTOR
+  }
+}
+
+// the nearest two factors of n that with_factor has
+bool fft_factors(int n, int* na, int* nb) {
+  auto built = [](int k) { return (k >= 2 && k <= 16) || k == 18 || k == 20; };
+  for (int a = 20; a >= 2; --a)
+    if (n % a == 0 && a <= n / a && built(a) && built(n / a)) {
+      *na = a;
+      *nb = n / a;
+      return true;
+    }
+  return false;
+}
+
+template <typename T>
+struct TwoShape {
+  static constexpr int LINES = sizeof(T) == 4 ? 32 : 16;  // 256-byte rows
+  static constexpr int MAX = LINES * 20;
+};
+
+template <typename T, typename TI, typename TO, int EPI, int SIGN>
+__global__ __launch_bounds__(TwoShape<T>::MAX) void k_fft_two(const TI* __restrict__ in, TO* __restrict__ out,
+                                                              int64_t n2, int64_t N, int na, int nb,
+                                                              const typename Cx<T>::t* __restrict__ twg, T scale,
+                                                              const double2* __restrict__ w,
+                                                              const double2* __restrict__ dL) {
+  typedef typename Cx<T>::t C;
+  constexpr int LINES = TwoShape<T>::LINES;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  C* const A = reinterpret_cast<C*>(smem_raw);  // A[(z1 nb + k2) LINES + l]
+  C* const tw = A + LINES * na * nb;            // exp(-2 pi i t / n)
+  const int tid = threadIdx.x, l = tid % LINES;
+  const int64_t rhs = blockIdx.y;
+  const int64_t g = (int64_t)blockIdx.x * LINES + l;
+  const TI* const src = in + rhs * N + (g < n2 ? g : n2 - 1);
+  TO* const dst = out + rhs * N;
+  for (int i = tid; i < na * nb; i += blockDim.x) tw[i] = twg[i];
+  __syncthreads();
+  // nb-point transforms of the samples z1 + na z2 (blockDim is LINES nb >= LINES na)
+  const int z = tid / LINES;
+  if (z < na)
+    with_factor(nb, [&](auto len) {
+      constexpr int L = decltype(len)::value;
+      C v[L];
+#pragma unroll
+      for (int z2 = 0; z2 < L; ++z2) v[z2] = load_c<C>(src + n2 * (int64_t)(z + na * z2));
+      RegDft<T, L, SIGN>::run(v);
+#pragma unroll
+      for (int k2 = 0; k2 < L; ++k2) {
+        C wt = tw[z * k2];  // z k2 < n: no wrap
+        if (SIGN > 0) wt.y = -wt.y;
+        A[(z * L + k2) * LINES + l] = k2 == 0 ? v[k2] : cmul(v[k2], wt);
+      }
+    });
+  __syncthreads();
+  // na-point transforms of the columns k2 = z
+  if (z < nb && g < n2)
+    with_factor(na, [&](auto len) {
+      constexpr int L = decltype(len)::value;
+      C u[L];
+#pragma unroll
+      for (int a = 0; a < L; ++a) u[a] = A[(a * nb + z) * LINES + l];
+      RegDft<T, L, SIGN>::run(u);
+#pragma unroll
+      for (int k1 = 0; k1 < L; ++k1) {
+        const int64_t gi = g + n2 * (int64_t)(z + nb * k1);
+        TO r;
+        if (EPI == 1) {
+          const double2 ww = w[rhs * N + gi], dd = dL[gi];
+          const double vx = (double)u[k1].x * (double)scale, vy = (double)u[k1].y * (double)scale;
+          r.x = ww.x - (dd.x * vx - dd.y * vy);
+          r.y = ww.y - (dd.x * vy + dd.y * vx);
+        } else {
+          r.x = u[k1].x * scale;
+          r.y = u[k1].y * scale;
+        }
+        store_nt(dst + gi, r);
+      }
+    });
+}
+
+template <typename T, typename TI, typename TO, int EPI>
+bool launch_two(hz_problem* p, int sign, int nrhs, const void* in, void* out, const double2* w, const double2* dL,
+                hipStream_t s) {
+  int na, nb;
+  if (sizeof(T) == 4 && p->fft.n < 32) return false;
+  // lengths past the general kernel's LDS stay refused in its words
+  if (!fft_factors(p->fft.n, &na, &nb) || !fft_lines_fit(sizeof(T) == 8 ? HZ_PREC_FP64 : HZ_PREC_C64, p->fft.n, 16))
+    return false;
+  constexpr int LINES = TwoShape<T>::LINES;
+  typedef typename Cx<T>::t C;
+  const C* tw = sizeof(T) == 8 ? (const C*)p->fft.tw64.ptr : (const C*)p->fft.tw32.ptr;
+  const size_t lds = (size_t)(LINES + 1) * p->fft.n * sizeof(C);  // 400 at most: 109 KB
+  const dim3 grid((unsigned)((p->n2 + LINES - 1) / LINES), (unsigned)nrhs), block((LINES * nb + 63) / 64 * 64);
+  const T scale = sign > 0 ? (T)(1.0 / (double)p->fft.n) : (T)1;
+  if (lds > 64 * 1024) {
+    set_max_lds((const void*)&k_fft_two<T, TI, TO, EPI, -1>, lds);
+    set_max_lds((const void*)&k_fft_two<T, TI, TO, EPI, 1>, lds);
+  }
+  if (sign < 0)
+    hipLaunchKernelGGL((k_fft_two<T, TI, TO, EPI, -1>), grid, block, lds, s, (const TI*)in, (TO*)out, p->n2, p->N, na,
+                       nb, tw, scale, w, dL);
+  else
+    hipLaunchKernelGGL((k_fft_two<T, TI, TO, EPI, 1>), grid, block, lds, s, (const TI*)in, (TO*)out, p->n2, p->N, na,
+                       nb, tw, scale, w, dL);
+  HZ_HIP(hipGetLastError());
+  return true;
 }
 
 template <typename T, typename TI, typename TO, int EPI, int LINES>
@@ -394,7 +551,9 @@ void launch_lines(hz_problem* p, int sign, int nrhs, const void* in, void* out, 
 template <typename T, typename TI, typename TO, int EPI>
 void launch_typed(hz_problem* p, int lines, int sign, int nrhs, const void* in, void* out, const double2* w,
                   const double2* dL, hipStream_t s) {
-  if (lines == 0 && launch_reg<T, TI, TO, EPI>(p, sign, nrhs, in, out, w, dL, s)) return;
+  if (lines == 0 && (launch_reg<T, TI, TO, EPI>(p, sign, nrhs, in, out, w, dL, s) ||
+                     launch_two<T, TI, TO, EPI>(p, sign, nrhs, in, out, w, dL, s)))
+    return;
   if (lines == 32 && fft_lines_fit(sizeof(T) == 8 ? HZ_PREC_FP64 : HZ_PREC_C64, p->fft.n, 32))
     launch_lines<T, TI, TO, EPI, 32>(p, sign, nrhs, in, out, w, dL, s);
   else if (lines == 8)
@@ -406,7 +565,8 @@ void launch_typed(hz_problem* p, int lines, int sign, int nrhs, const void* in, 
 }  // namespace
 
 bool fft_reg_available(int nz) {
-  return nz == 200 || nz == 192 || nz == 160 || nz == 128 || nz == 96 || nz == 64;
+  int na, nb;
+  return nz == 200 || nz == 192 || nz == 160 || nz == 128 || nz == 96 || nz == 64 || fft_factors(nz, &na, &nb);
 }
 
 bool fft_lines_fit(int prec, int nz, int lines) {
