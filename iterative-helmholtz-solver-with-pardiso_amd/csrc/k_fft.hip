@@ -433,6 +433,13 @@ bool fft_factors(int n, int* na, int* nb) {
   return false;
 }
 
+// Whether k_fft_two transforms length n in precision prec, and its factors.
+// Lengths past the general kernel's LDS stay refused in its words.
+bool fft_two_takes(int prec, int n, int* na, int* nb) {
+  if (prec == HZ_PREC_C64 && n < 32) return false;
+  return fft_factors(n, na, nb) && fft_lines_fit(prec, n, 16);
+}
+
 template <typename T>
 struct TwoShape {
   static constexpr int LINES = sizeof(T) == 4 ? 32 : 16;  // 256-byte rows
@@ -504,10 +511,7 @@ template <typename T, typename TI, typename TO, int EPI>
 bool launch_two(hz_problem* p, int sign, int nrhs, const void* in, void* out, const double2* w, const double2* dL,
                 hipStream_t s) {
   int na, nb;
-  if (sizeof(T) == 4 && p->fft.n < 32) return false;
-  // lengths past the general kernel's LDS stay refused in its words
-  if (!fft_factors(p->fft.n, &na, &nb) || !fft_lines_fit(sizeof(T) == 8 ? HZ_PREC_FP64 : HZ_PREC_C64, p->fft.n, 16))
-    return false;
+  if (!fft_two_takes(sizeof(T) == 8 ? HZ_PREC_FP64 : HZ_PREC_C64, p->fft.n, &na, &nb)) return false;
   constexpr int LINES = TwoShape<T>::LINES;
   typedef typename Cx<T>::t C;
   const C* tw = sizeof(T) == 8 ? (const C*)p->fft.tw64.ptr : (const C*)p->fft.tw32.ptr;
@@ -564,13 +568,14 @@ void launch_typed(hz_problem* p, int lines, int sign, int nrhs, const void* in, 
 
 }  // namespace
 
-bool fft_reg_available(int nz) {
+// whether length nz has a register-resident kernel in precision prec
+static bool fft_reg_available(int prec, int nz) {
   int na, nb;
-  return nz == 200 || nz == 192 || nz == 160 || nz == 128 || nz == 96 || nz == 64 || fft_factors(nz, &na, &nb);
+  return nz == 200 || nz == 192 || nz == 160 || nz == 128 || nz == 96 || nz == 64 || fft_two_takes(prec, nz, &na, &nb);
 }
 
 bool fft_lines_fit(int prec, int nz, int lines) {
-  if (lines == 0) return fft_reg_available(nz);
+  if (lines == 0) return fft_reg_available(prec, nz);
   const size_t c = prec == HZ_PREC_FP64 ? 16 : 8;
   const size_t ld = lines + (prec == HZ_PREC_FP64 ? 1 : 2);
   return (2 * ld + 1) * nz * c <= 160 * 1024;
@@ -581,7 +586,7 @@ void launch_fft_z(hz_problem* p, int prec, int sign, int nrhs, const void* in, i
   // HZ_FFT_LINES=0|8|16|32 forces the lines per workgroup, 0 being the
   // register-resident kernel (timing and tests)
   int lines = p->tuning(prec, nrhs).fft_lines;
-  if (lines < 0) lines = fft_reg_available((int)p->nz) ? 0 : 16;
+  if (lines < 0) lines = fft_reg_available(prec, (int)p->nz) ? 0 : 16;
   if (const char* e = getenv("HZ_FFT_LINES")) {
     const int v = atoi(e);
     if ((v == 0 || v == 8 || v == 16 || v == 32) && fft_lines_fit(prec, (int)p->nz, v)) lines = v;
