@@ -145,12 +145,12 @@ enum {
                                two planes of each factor slot per pass; up to 256 columns */
 };
 typedef struct {
-  int32_t solve_kernel; /* HZ_SOLVE_* */
+  int32_t solve_kernel; /* HZ_SOLVE_*: the fastest family; calls take it where it beats the untuned kernel */
   int32_t group_cap;    /* right-hand sides per streaming pass: 8, 4, 2 or 1 */
   int32_t fft_lines;    /* (x,y) lines per z-FFT workgroup: 8, 16 or 32 (LDS Stockham), 0 for the
                            register-resident kernels (nz a product of two small factors) */
   int32_t from_cache;   /* 1 when read from the HZ_TUNE_CACHE file */
-  double solve_ms;      /* plane solve of nrhs vectors with the choice */
+  double solve_ms;      /* plane solve of nrhs vectors as calls take it */
   double fft_ms;        /* one forward z-FFT of nrhs vectors with the choice */
 } hz_tune_info;
 

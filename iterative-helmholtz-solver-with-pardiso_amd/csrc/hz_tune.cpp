@@ -3,7 +3,9 @@
 // sides).  Variants: the plane-solve kernel family (streaming multi-RHS or
 // chunked), the streaming kernel's right-hand-side group cap (one pass over the
 // factors serves up to 8 vectors; smaller groups put more workgroups on the
-// chip when nz is below the CU count) and the z-FFT lines per workgroup.
+// chip when nz is below the CU count) and the z-FFT lines per workgroup.  The
+// kernel that untuned calls take is timed beside them and kept where no family
+// is faster.
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
@@ -46,6 +48,10 @@ std::string cache_key(const hz_problem* p, int prec, int nrhs) {
   return k.str();
 }
 
+// What calls take under a key of an earlier set of kernels says nothing about
+// this one: raised when a kernel or a rule of the dispatch changes.
+constexpr int KERNEL_SET = 2;
+
 std::mutex g_cache_mu;
 
 bool cache_read(const std::string& path, const std::string& key, Tuning& t) {
@@ -54,7 +60,9 @@ bool cache_read(const std::string& path, const std::string& key, Tuning& t) {
   std::string line;
   bool found = false;
   while (std::getline(in, line)) {
-    // "<arch> nx ny nz prec nrhs | family cap lines"
+    // "<arch> nx ny nz prec nrhs | family cap lines": the fastest family, and
+    // "<arch> nx ny nz prec nrhs set <n> | ...": what calls take (family 0: the
+    // untuned kernel)
     const size_t bar = line.find('|');
     if (bar == std::string::npos) continue;
     std::string k = line.substr(0, bar);
@@ -85,8 +93,9 @@ void autotune(hz_problem* p, int prec, int nrhs, hz_tune_info* info) {
   ensure_dense(p, prec, p->stream);  // every candidate timed on complete factors
   const char* cpath = getenv("HZ_TUNE_CACHE");
   const std::string key = cache_key(p, prec, nrhs);
-  Tuning best;
-  bool from_cache = cpath && cpath[0] && cache_read(cpath, key, best);
+  const std::string taken_key = key + " set " + std::to_string(KERNEL_SET);
+  Tuning best, taken;
+  const bool from_cache = cpath && cpath[0] && cache_read(cpath, taken_key, taken) && cache_read(cpath, key, best);
 
   // work vectors: complex128 input of the forward FFT and the plane-solve buffer
   const size_t vb = (size_t)p->N * nrhs * sizeof(double2);
@@ -135,16 +144,23 @@ void autotune(hz_problem* p, int prec, int nrhs, hz_tune_info* info) {
       t.solve_family = HZ_SOLVE_CHUNKED;
       cand.push_back(t);
     }
+    const auto solve_ms = [&](const Tuning& t) {
+      return time_ms(p, [&] { launch_plane_solve_with(p, prec, nrhs, p->w_a.ptr, false, t, p->stream); }, reps);
+    };
     best_solve = -1;
     for (const Tuning& t : cand) {
-      const double ms = time_ms(p, [&] { launch_plane_solve_with(p, prec, nrhs, p->w_a.ptr, false, t, p->stream); },
-                                reps);
+      const double ms = solve_ms(t);
       if (best_solve < 0 || ms < best_solve) {
         best_solve = ms;
         best.solve_family = t.solve_family;
         best.group_cap = t.group_cap;
       }
     }
+    // the untuned kernel, kept unless a family is faster by more than the
+    // timings scatter
+    const double untuned = solve_ms(Tuning());
+    if (untuned <= 1.02 * best_solve) best_solve = untuned;
+    else taken = best;
     // forward z-FFT (complex128 in, the precision's plane layout out)
     best_fft = -1;
     for (int lines : {0, 8, 16, 32}) {
@@ -158,15 +174,19 @@ void autotune(hz_problem* p, int prec, int nrhs, hz_tune_info* info) {
         best.fft_lines = lines;
       }
     }
-    if (cpath && cpath[0]) cache_append(cpath, key, best);
+    taken.fft_lines = best.fft_lines;
+    if (cpath && cpath[0]) {
+      cache_append(cpath, key, best);
+      cache_append(cpath, taken_key, taken);
+    }
   } else {
-    best_solve = time_ms(p, [&] { launch_plane_solve_with(p, prec, nrhs, p->w_a.ptr, false, best, p->stream); }, 1);
+    best_solve = time_ms(p, [&] { launch_plane_solve_with(p, prec, nrhs, p->w_a.ptr, false, taken, p->stream); }, 1);
     best_fft = time_ms(p, [&] {
       launch_fft_z_lines(p, best.fft_lines, prec, -1, nrhs, p->w_b.ptr, 0, p->w_a.ptr, prec == HZ_PREC_C64 ? 1 : 0,
                          0, nullptr, nullptr, p->stream);
     }, 1);
   }
-  p->tuned[{prec, nrhs}] = best;
+  p->tuned[{prec, nrhs}] = taken;
   if (info) {
     info->solve_kernel = best.solve_family;
     info->group_cap = best.group_cap;
