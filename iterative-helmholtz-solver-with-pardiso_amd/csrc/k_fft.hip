@@ -207,6 +207,35 @@ __global__ __launch_bounds__(256) void k_fft_z(const TI* __restrict__ in, TO* __
 // transforms them in registers and writes X[k2 + N2 k1].  The in-register
 // DFTs are compile-time mixed-radix Cooley-Tukey with constant twiddles.
 
+// cos and sin of 2 pi k / n within a unit of the last place, for constants: the angle is folded
+// into the first octant in whole numbers, and what its rounding leaves out
+// enters to first order.  (cos(2 pi k / n) as written rounds the angle at up to
+// 2 pi: constants off by up to 4 units of the last place, twice the error of a
+// 13-point transform.)
+struct UnitRoot {
+  double c, s;
+};
+__device__ __forceinline__ constexpr UnitRoot unit_root(int k, int n) {
+  k %= n;
+  const bool neg = 2 * k > n;  // sin < 0
+  if (neg) k = n - k;
+  const bool obt = 4 * k > n;  // cos < 0
+  int u = obt ? n - 2 * k : 2 * k;  // angle pi u / n, in 0 .. pi / 2
+  const bool swp = 4 * u > n;       // past pi / 4: pi / 2 - angle
+  int den = n;
+  if (swp) {
+    u = n - 2 * u;
+    den = 2 * n;
+  }
+  const double ph = 3.14159265358979311600, pl = 1.22464679914735317723e-16;  // pi
+  const double q = ph * u, qe = __builtin_fma(ph, (double)u, -q), t = q / den;
+  const double e = (__builtin_fma(-t, (double)den, q) + qe + pl * u) / den;
+  const double ct = __builtin_cos(t), st = __builtin_sin(t);
+  const double c = ct - e * st, s = st + e * ct;
+  const double cc = swp ? s : c, ss = swp ? c : s;
+  return UnitRoot{obt ? -cc : cc, neg ? -ss : ss};
+}
+
 // out[k] = sum_j in[j] e^{sign 2 pi i j k / N}  (in place, compile-time N)
 template <typename T, int N, int SIGN>
 struct RegDft {
@@ -228,10 +257,10 @@ struct RegDft {
         RegDft<T, M, SIGN>::run(sub);
 #pragma unroll
         for (int k = 0; k < M; ++k) {
-          const double ang = (double)SIGN * 2.0 * 3.14159265358979323846 * (double)(p * k) / (double)N;
+          const UnitRoot r = unit_root(p * k, N);
           C w;
-          w.x = (T)cos(ang);
-          w.y = (T)sin(ang);
+          w.x = (T)r.c;
+          w.y = (T)(SIGN * r.s);
           t[p * M + k] = (p * k == 0) ? sub[k] : cmul(sub[k], w);
         }
       }
@@ -290,9 +319,9 @@ struct RegDft {
         im.x = 0; im.y = 0;
 #pragma unroll
         for (int j = 1; j <= H; ++j) {
-          const double ang = 2.0 * 3.14159265358979323846 * (double)(j * k % N) / (double)N;
-          re = cadd(re, cscale(b[j - 1], (T)cos(ang)));
-          im = cadd(im, cscale(d[j - 1], (T)sin(ang)));
+          const UnitRoot r = unit_root(j * k, N);
+          re = cadd(re, cscale(b[j - 1], (T)r.c));
+          im = cadd(im, cscale(d[j - 1], (T)r.s));
         }
         im = cmul_si(im, SIGN);
         v[k] = cadd(re, im);
@@ -406,10 +435,10 @@ bool launch_reg(hz_problem* p, int sign, int nrhs, const void* in, void* out, co
 // Call times in us (some 20 of them the launch and the wait), general -> this:
 // complex128 24 x 22 x 28 29 -> 23, 100^3 52 -> 25, 140 x 140 x 150 115 -> 36,
 // x 8 821 -> 159 (4.7 TB/s), 200 x 200 x 143 206 -> 48; complex64 150 x 8 418 ->
-// 158, 48^3 x 4 29 -> 24.  Faster at every length tried.  complex64 below 32
-// points keeps the general kernel's rounding: a launch there is mostly latency
-// (28 points 28 -> 23 with its wait), and solves of hundreds of steps on such
-// grids count their iterations to +-1 between equal problems.
+// 158, 48^3 x 4 29 -> 24.  Faster at every length tried, with errors within 4%
+// of the general kernel's (complex128, 2 .. 400 points).  complex64 below 32
+// points stays on the general kernel: a launch there is mostly latency (28
+// points 28 -> 23 with its wait).
 template <typename F>
 __device__ __forceinline__ void with_factor(int n, F&& f) {
   switch (n) {
