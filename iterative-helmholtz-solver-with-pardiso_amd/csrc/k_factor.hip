@@ -252,8 +252,11 @@ __global__ __launch_bounds__(FR_THREADS) void k_factor_reg(typename Cx<T>::t* __
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
               const C o = a[q][c];
-              a[q][c - 1].x = fma(-fp[q].x, pv[c].x, fma(fp[q].y, pv[c].y, o.x));
-              a[q][c - 1].y = fma(-fp[q].x, pv[c].y, fma(-fp[q].y, pv[c].x, o.y));
+              // the product, then the difference: one rounding at o's size a step
+              // (the two products summed onto o in turn rounded twice: 1.7 times
+              // the error of a chain of 16-column blocks)
+              a[q][c - 1].x = o.x + fma(-fp[q].x, pv[c].x, fp[q].y * pv[c].y);
+              a[q][c - 1].y = o.y - fma(fp[q].x, pv[c].y, fp[q].y * pv[c].x);
             }
 #pragma unroll
           for (int q = 0; q < NQ; ++q) {

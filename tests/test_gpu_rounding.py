@@ -39,3 +39,72 @@ def test_fft_rounding(hz, monkeypatch, nz):
         e[lines] = extended.error(got, want)
     print("nz=%d general %.3g registers %.3g" % (nz, e["16"], e["0"]), flush=True)
     assert e["0"] < 1.15 * e["16"]
+
+
+def _layers(hz, nx, ny, nz, seed):
+    """A box of 10 points per wavelength with four-point layers on every face, a
+    rough medium, and a right-hand side that both precisions hold exactly."""
+    pr = hz.problem
+    h = 1.0 / min(nx, ny, nz)
+    d = pr.cube_geometry((nx, ny, nz), 4, pr.omega_for_ppw(0.7, h, 10), beta=1.0, pml_c=3.0 * np.log(1e6) / (8.0 * h))
+    rng = np.random.default_rng(seed)
+    c = 0.8 + 0.5 * rng.random(d.N)
+    return d, c, (rng.standard_normal(d.N) + 1j * rng.standard_normal(d.N)).astype(np.complex64)
+
+
+def _solve(S, hz, b, prec, adjoint=False):
+    dt = np.complex128 if prec == hz.abi.PREC_FP64 else np.complex64
+    return S.plane_solve(torch.from_numpy(b.astype(dt)).cuda(), prec, adjoint=adjoint).cpu().numpy()
+
+
+def _inverse_c64(A):
+    """Gauss-Jordan in complex64 with partial pivoting, every update's product
+    formed and then subtracted: one rounding at the size of the entry a step."""
+    A = A.astype(np.complex64)
+    S, n, _ = A.shape
+    at, used = np.arange(S), np.zeros((S, n), bool)
+    piv, kof = np.zeros((S, n), int), np.zeros((S, n), int)
+    for k in range(n):
+        size = np.where(used, -1, np.abs(A[:, :, k].real) + np.abs(A[:, :, k].imag))
+        r = np.argmax(size, 1)
+        used[at, r], piv[:, k], kof[at, r] = True, r, k
+        pinv = (1.0 / A[at, r, k].astype(np.complex128)).astype(np.complex64)
+        row = A[at, r].copy()
+        A[at, r] = 0
+        f = A[:, :, k] * pinv[:, None]
+        f[at, r] = -pinv
+        A -= f[:, :, None] * row[:, None, :]
+        A[:, :, k] = -f
+    B = np.empty_like(A)
+    for s in range(S):
+        B[s][np.ix_(kof[s], piv[s])] = A[s]
+    return B
+
+
+def test_factor_rounding(hz, oracle, monkeypatch):
+    """complex64 factors of a long chain of 16-column blocks (a single panel
+    each): the one-directional solve on them against the same solve on numpy's
+    complex64 inverses.  Both round an entry once a step; 20% for scatter."""
+    monkeypatch.setenv("HZ_SOLVE_KERNEL", "fast")
+    nx, ny, nz = 16, 40, 12
+    ratio = []
+    for seed in range(3):
+        d, c, b = _layers(hz, nx, ny, nz, seed)
+        S, P = hz.Solver(d, c), oracle.Problem(d, c)
+        S.factor(hz.abi.PREC_C64)
+        D, low, up, slot = extended.blocks(P, nx, ny)
+        G = extended.chain(D, low, up, _inverse_c64)
+        x = np.empty((nz, ny, nx), np.complex64)
+        B = b.reshape(nz, ny, nx)
+        for k in range(nz):
+            t = [B[k, 0]]
+            for j in range(1, ny):
+                t.append((B[k, j] - low[j] * (G[j - 1][slot[k]] @ t[-1])).astype(np.complex64))
+            x[k, -1] = G[-1][slot[k]] @ t[-1]
+            for j in range(ny - 2, -1, -1):
+                x[k, j] = G[j][slot[k]] @ (t[j] - up[j] * x[k, j + 1]).astype(np.complex64)
+        want = extended.plane_solve(P, d.n, b)
+        e_gpu, e_np = extended.error(_solve(S, hz, b, hz.abi.PREC_C64), want), extended.error(x.reshape(-1), want)
+        print("factor seed %d: %.3g, numpy %.3g" % (seed, e_gpu, e_np), flush=True)
+        ratio.append(e_gpu / e_np)
+    assert np.exp(np.mean(np.log(ratio))) < 1.2, ratio
