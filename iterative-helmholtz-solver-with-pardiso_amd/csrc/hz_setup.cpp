@@ -296,22 +296,29 @@ void setup_tables(hz_problem* p, const double* c) {
 
   // Diagonal scalings D = diag(dx(i) dy(j)) with D^{-1} M_k complex symmetric:
   // d(i) / d(i-1) = cm(i) / cp(i-1) per axis (the reference's symmetry check,
-  // Tests.cpp:686-757), so the block inverses G_j D_j are symmetric.
+  // Tests.cpp:686-757), so the block inverses G_j D_j are symmetric.  Products
+  // in extended precision, and 1 at the middle of the axis: the scalings of the
+  // whole interior are then exactly 1 and round nothing there.
   {
     std::vector<double2> sd;
+    typedef std::complex<long double> lc;
+    const auto down = [](lc v) { return make_double2((double)v.real(), (double)v.imag()); };
     for (int a = 0; a < 2; ++a) {
       const int64_t n = d.n[a];
-      std::vector<zc> dd(n, zc(1.0, 0.0));
+      std::vector<lc> dd(n, lc(1.0L, 0.0L));
       for (int64_t i = 1; i < n; ++i) {
-        const zc den = zz(p->cp[a][i - 1]);
-        dd[i] = std::abs(den) > 0.0 ? dd[i - 1] * zz(p->cm[a][i]) / den : dd[i - 1];
+        const lc num(zz(p->cm[a][i])), den(zz(p->cp[a][i - 1]));
+        dd[i] = std::abs(den) > 0.0L && num != den ? dd[i - 1] * (num / den) : dd[i - 1];
       }
+      const lc mid = dd[n / 2];
       p->symd[a].resize(n);
-      for (int64_t i = 0; i < n; ++i) p->symd[a][i] = d2(dd[i]);
+      for (int64_t i = 0; i < n; ++i) {
+        p->symd[a][i] = down(dd[i] == mid ? lc(1.0L, 0.0L) : dd[i] / mid);
+      }
     }
     for (int a = 0; a < 2; ++a) sd.insert(sd.end(), p->symd[a].begin(), p->symd[a].end());
     for (int a = 0; a < 2; ++a)
-      for (const double2& v : p->symd[a]) sd.push_back(d2(1.0 / zz(v)));
+      for (const double2& v : p->symd[a]) sd.push_back(down(lc(1.0L, 0.0L) / lc(zz(v))));
     p->d_symd.alloc(sd.size() * sizeof(double2));
     HZ_HIP(hipMemcpy(p->d_symd.ptr, sd.data(), sd.size() * sizeof(double2), hipMemcpyHostToDevice));
   }

@@ -108,3 +108,26 @@ def test_factor_rounding(hz, oracle, monkeypatch):
         print("factor seed %d: %.3g, numpy %.3g" % (seed, e_gpu, e_np), flush=True)
         ratio.append(e_gpu / e_np)
     assert np.exp(np.mean(np.log(ratio))) < 1.2, ratio
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(64, 12, 12), (33, 30, 20), (16, 40, 12)])
+def test_twisted_rounding(hz, oracle, monkeypatch, nx, ny, nz):
+    """The twisted solve against the one-directional one, forward: the same
+    operator in the same precision by half as many steps a chain, so no larger
+    an error; 15% for scatter (64 x 12 x 12 is mostly layers, where the scalings
+    of the symmetric factors are not 1)."""
+    ratio = {}
+    for seed in range(3):
+        d, c, b = _layers(hz, nx, ny, nz, seed)
+        S, P = hz.Solver(d, c), oracle.Problem(d, c)
+        want = extended.plane_solve(P, d.n, b)
+        for prec in (hz.abi.PREC_FP64, hz.abi.PREC_C64):
+            S.factor(prec)
+            e = {}
+            for fam in ("fast", "twist"):
+                monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
+                e[fam] = extended.error(_solve(S, hz, b, prec), want)
+            print("twisted %d %d %d prec %d seed %d: %.3g, one-directional %.3g" % (nx, ny, nz, prec, seed, e["twist"], e["fast"]), flush=True)
+            ratio.setdefault(prec, []).append(e["twist"] / e["fast"])
+    for prec, r in ratio.items():
+        assert np.exp(np.mean(np.log(r))) < 1.15, (prec, r)
