@@ -2180,6 +2180,19 @@ bool twist_solve_available(const hz_problem* p, int prec) {
 }
 
 namespace {
+// Whether a complex64 adjoint sweep sums its products in FP64, as the sweep that
+// k_apply walks does: everywhere but on the packed symmetric factors' widths and
+// in whole groups of 8 on the widths with streaming kernels.  The sums' rounding
+// is a third of the error where the layers are strong (reference grid 64^3
+// 7.5e-8, 9.8e-8 with FP32 sums).  Times in ms, k_apply -> FP64 sums (FP32 sums):
+// 48^3 0.43 -> 0.071 (0.064), 64^3 0.77 -> 0.113 (0.096), 96^3 2.64 -> 0.28
+// (0.21), 140^3 7.7 -> 0.81 (0.56), x 16 28.2 -> 7.1 (2.9, rows), 208^3 22.5 ->
+// 1.72 (1.64), 239 x 239 x 150 31.0 -> 2.12 (2.03).
+bool wide_adjoint(const hz_problem* p, int prec, int nrhs) {
+  const int n = (int)p->nx;
+  return prec == HZ_PREC_C64 && !sym_solve_available(prec, n) && !(nrhs % 8 == 0 && stream_solve_available(prec, n));
+}
+
 // Whether plane_solve_kernels takes the twisted solve for this call (the only
 // kernel that runs on an incomplete top-down chain): where it is asked for or
 // tuned; untuned always in complex128, and in complex64 unless 8 and more
@@ -2211,6 +2224,7 @@ bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tun
   if (sk == SK_TWIST) return true;
   if (sk != SK_DEFAULT) return false;
   if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
+  if (adjoint && wide_adjoint(p, prec, nrhs)) return true;
   if (nrhs < 8 || !mfma_solve_available(p, prec) || p->nx > 208) return true;
   if (p->nx <= 96 && 2 * (int64_t)p->nslot * nrhs < 1024) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2435,7 +2449,7 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
              "adjoint plane solve: the dense factors were released by HZ_HODLR_FREE_DENSE");
   }
   if (uses_twist(p, prec, nrhs, adjoint, t, s)) {
-    solve_tri(p, prec, nrhs, x, adjoint, s);
+    solve_tri(p, prec, nrhs, x, adjoint, adjoint && wide_adjoint(p, prec, nrhs), s);
     return;
   }
   if (!f.top_full) ensure_dense(p, prec, s);
@@ -2452,7 +2466,7 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
   // kernel family
   if (adjoint && ny >= 1 && prec == HZ_PREC_C64 &&
       (sk == SK_DEFAULT || sk == SK_SYM || sk == SK_MFMA || sk == SK_TWIST)) {
-    if (sk != SK_SYM && nrhs >= 8 && mfma_solve_available(p, prec)) {
+    if (sk != SK_SYM && nrhs >= 8 && mfma_solve_available(p, prec) && (sk == SK_MFMA || !wide_adjoint(p, prec, nrhs))) {
       solve_rows(p, nrhs, x, true, s);
       return;
     }

@@ -60,10 +60,11 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
 
 
 // Twisted plane solves (k_tri.hip): whether a width has them, the packing of
-// the factor chains (G, Gb) into Gtw, and the solve of nrhs vectors.
+// the factor chains (G, Gb) into Gtw, and the solve of nrhs vectors (wide:
+// complex64 adjoint with the sums in FP64).
 bool tri_available(int nx);
 void pack_tri(hz_problem* p, int prec, hipStream_t s);
-void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s);
+void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, bool wide, hipStream_t s);
 
 // Groups of 8 complex64 right-hand sides on the one-directional factors
 // (k_rows.hip): whether a problem has them, and the solve of nrhs vectors.

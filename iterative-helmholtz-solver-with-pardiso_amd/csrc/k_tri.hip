@@ -39,6 +39,11 @@
 // products keep one sum per p and add the blocks at the row's end; a product
 // with the identity moves a 4 x 4 block from the A to the B layout exactly, and
 // the transposed products then sum over all rows in the accumulator.
+// The complex64 adjoint sums in FP64 wherever the sweep before it did (solve_tri's
+// wide): the same 4x4x4 products on the complex64 tiles, whose layout is the A
+// operand of block b & 3 with k = b >> 2, so that a row's direct sum is complete
+// in the accumulator and the transposed ones are summed over the row groups by
+// row rotations.
 // No value is added to by two waves: the thread of (plane, row) adds the row's
 // direct sum and its transposed partials in a fixed order.
 //
@@ -134,7 +139,8 @@ __device__ __forceinline__ void tri_quad_transpose(float* k, float* l) {
   l[0] = d0; l[1] = d1; l[2] = d2; l[3] = d3;
 }
 
-template <typename T, int NT>
+// T: the stored factors and vectors, A: the arithmetic
+template <typename T, typename A, int NT>
 struct TriShape {
   static constexpr int NW = (NT + 1) / 2;  // waves: tile rows w and w + NW (the last wave of an odd NT: one row)
   static constexpr int NA = NT / 2 + 1;    // tiles of row w
@@ -156,24 +162,25 @@ struct TriShape {
   // 16 registers) a half or a third of them where they would not fit
   static constexpr int RD = sizeof(T) == 4 || NS <= 9 ? NSW : NS <= 10 ? (NS + 1) / 2 : (NS + 2) / 3;
   static constexpr int NSR = (NSW + RD - 1) / RD * RD;  // slots of a block, the last possibly empty
-  static constexpr size_t lds = sizeof(T) * (8 * (size_t)NP + 64 * ((size_t)(NT + 1) * NA + NT + 1));
+  static constexpr size_t lds = sizeof(A) * (8 * (size_t)NP + 64 * ((size_t)(NT + 1) * NA + NT + 1));
 };
 
-template <typename T, int NT, int PH, bool ADJ>
-__global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
+template <typename T, typename A, int NT, int PH, bool ADJ>
+__global__ __launch_bounds__((TriShape<T, A, NT>::THREADS)) void k_solve_tri(
     const typename Cx<T>::t* __restrict__ P, typename Cx<T>::t* __restrict__ X, const double2* __restrict__ cmy,
     const double2* __restrict__ cpy, const double2* __restrict__ symd, int n, int ny, int m, int nz, int64_t n2,
     int64_t N, const int2* __restrict__ slotp, int nslot, int nrhs, typename Cx<T>::t* __restrict__ scr) {
   typedef typename Cx<T>::t C;
-  typedef TriShape<T, NT> S;
-  constexpr bool F32 = sizeof(T) == 4;
+  typedef typename Cx<A>::t CA;
+  typedef TriShape<T, A, NT> S;
+  constexpr bool F32 = sizeof(T) == 4, A32 = sizeof(A) == 4;
   constexpr int NP = S::NP;
   constexpr int BS = NT * (NT + 1) / 2 * 256;  // complex values of a packed block
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* const vq = reinterpret_cast<T*>(smem_raw);  // [4][NP] components of v'
-  T* const vr = vq + 4 * NP;                     // [4][NP] rotated: (-Im A, Re A, -Im B, Re B)
-  T* const dsum = vr + 4 * NP;                   // [NT + 1][2][16][2] direct sums (plane, row, re/im)
-  T* const tsum = dsum + 64 * (NT + 1);          // [C][d][2][16][2] transposed sums of tile (C - d, C)
+  A* const vq = reinterpret_cast<A*>(smem_raw);  // [4][NP] components of v'
+  A* const vr = vq + 4 * NP;                     // [4][NP] rotated: (-Im A, Re A, -Im B, Re B)
+  A* const dsum = vr + 4 * NP;                   // [NT + 1][2][16][2] direct sums (plane, row, re/im)
+  A* const tsum = dsum + 64 * (NT + 1);          // [C][d][2][16][2] transposed sums of tile (C - d, C)
                                                  // (the last of either: sums nobody reads)
 
   // Workgroups go to the 8 XCDs in turn: the right-hand sides of one (slot,
@@ -260,10 +267,10 @@ __global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
   }
 
   // ---- v' of the first block
-  for (int e = tid; e < 8 * NP; e += S::THREADS) vq[e] = (T)0;
+  for (int e = tid; e < 8 * NP; e += S::THREADS) vq[e] = (A)0;
   __syncthreads();
   auto put_v = [&](double2 v) {  // v' = D^-1 v of this thread's row
-    const T a = (T)v.x, b = (T)v.y;
+    const A a = (A)v.x, b = (A)v.y;
     vq[(2 * ps) * NP + pr] = a;
     vq[(2 * ps + 1) * NP + pr] = b;
     vr[(2 * ps) * NP + pr] = -b;
@@ -340,7 +347,7 @@ __global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
     const double2 cf = line.cf, sn = cmul_d(dxir, line.di);
     line = fetch(st + 1 < nsteps ? st + 1 : st);
 
-    if constexpr (F32) {
+    if constexpr (A32) {
       // Software pipeline over the tiles, one scheduling region each: tile t's
       // direct products, transposes and reload, tile t - 1's transposed products
       // and tile t - 2's sum over the row groups.  (Without the fences the
@@ -423,6 +430,55 @@ __global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
         dsum[64 * ra + at] = tri_sum32(tri_sum16(a[0], a[1]), tri_sum16(a[2], a[3]));
         if (!S::SPLIT) dsum[64 * (spare ? NT : rb) + at] = tri_sum32(tri_sum16(b[0], b[1]), tri_sum16(b[2], b[3]));
       }
+    } else if constexpr (F32) {
+      // complex64 tiles, sums in FP64: register e of a lane holds column 4 cg + e
+      // of row 4 rg + qi, the A operand of block rg (k = cg) as it lies.
+      const int i4 = lane >> 4;                  // k of an operand, i of a result
+      const double one = i4 == qi ? 1.0 : 0.0;  // the identity, as B operand
+      double va, vb, dp;
+      auto row_operands = [&](int R) {
+        va = vq[qi * NP + 16 * R + 4 * rg + i4];
+        vb = vr[qi * NP + 16 * R + 4 * rg + i4];
+        dp = 0.0;
+      };
+      auto flush_row = [&](int out) { dsum[64 * out + (qi >> 1) * 32 + (4 * rg + i4) * 2 + (qi & 1)] = dp; };
+      row_operands(ra);
+#pragma unroll
+      for (int t = 0; t < S::NSW; ++t) {
+        if (t == S::NA) {
+          flush_row(ra);
+          row_operands(rb);
+        }
+        const int cc = col_of(t), d = t < S::NA ? t : t - S::NA;
+        const int at0 = qi * NP + 16 * cc + 4 * cg;
+        const double2 u0 = *reinterpret_cast<const double2*>(vq + at0), u1 = *reinterpret_cast<const double2*>(vq + at0 + 2);
+        const double2 w0 = *reinterpret_cast<const double2*>(vr + at0), w1 = *reinterpret_cast<const double2*>(vr + at0 + 2);
+        const double u[4] = {u0.x, u0.y, u1.x, u1.y}, v[4] = {w0.x, w0.y, w1.x, w1.y};
+        double kr[4], ki[4], x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const C k = q[t % S::RD][e / UL].c[e % UL];
+          dp = __builtin_amdgcn_mfma_f64_4x4x4f64((double)k.x, u[e], dp, 0, 0, 0);
+          kr[e] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)k.x, one, 0.0, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f64_4x4x4f64((double)k.y, v[e], dp, 0, 0, 0);
+          ki[e] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)k.y, one, 0.0, 0, 0, 0);
+        }
+        reload(t);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(va, kr[e], 0.0, 0, 0, 0);
+          x[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(vb, ki[e], x[e], 0, 0, 0);
+          // the diagonal tile's own 4 x 4 blocks have no transposed product
+          // (its lower blocks are stored as zeros)
+          if (d == 0) x[e] = qi > rg ? x[e] : 0.0;
+        }
+        // sum over the row groups (lane bits 2, 3): group b gets the columns 4 j + b
+        const double xs4 = tri_pair<0x128>(tri_pair<0x124>(x[0], x[1], b2), tri_pair<0x124>(x[2], x[3], b2), b3);
+        const int at = t < SP0 || !spare ? cc : NT;
+        tsum[64 * (at * S::NA + d) + (i4 >> 1) * 32 + (4 * qi + rg) * 2 + (i4 & 1)] = xs4;
+        __builtin_amdgcn_sched_barrier(0);  // the reloads stay in order
+      }
+      flush_row(S::SPLIT ? ra : spare ? NT : rb);
     } else {
       const int i4 = lane >> 4;  // k of an operand, i of a result
       const double one = i4 == qi ? 1.0 : 0.0;  // the identity, as B operand
@@ -478,26 +534,26 @@ __global__ __launch_bounds__((TriShape<T, NT>::THREADS)) void k_solve_tri(
 
     if (row_ok) {
       const int rt = pr >> 4, at = ps * 32 + (pr & 15) * 2;
-      C y = *reinterpret_cast<const C*>(dsum + 64 * rt + at);
+      CA y = *reinterpret_cast<const CA*>(dsum + 64 * rt + at);
 #pragma unroll
       for (int d = 0; d < S::NA; ++d) {
-        const C u = *reinterpret_cast<const C*>(tsum + 64 * (rt * S::NA + d) + at);
+        const CA u = *reinterpret_cast<const CA*>(tsum + 64 * (rt * S::NA + d) + at);
         // even NT: tile (C - NT/2, C) is kept where C - NT/2 is below NT/2
         const bool kept = NT % 2 != 0 || d < NT / 2 || rt >= NT / 2;
-        y.x += kept ? u.x : (T)0;
-        y.y += kept ? u.y : (T)0;
+        y.x += kept ? u.x : (A)0;
+        y.y += kept ? u.y : (A)0;
       }
       const double2 v = make_double2(f.x - (cf.x * y.x - cf.y * y.y), f.y - (cf.x * y.y + cf.y * y.x));
       if (jn >= 0) put_v(cmul_d(v, sn));
       if (wr && PH == 1 && (half == 0 || st > 0)) {  // x_jb
-        C o = y;
+        C o = mk<C>(y.x, y.y);
         if (ADJ) {
           const double2 z = cmul_d(make_double2(y.x, y.y), sb);
           o = mk<C>(z.x, -z.y);
         }
         xs[(int64_t)jb * n] = o;
       }
-      if (wr && jn == -2) *scr_at(half) = y;                                // y_top / y_bot
+      if (wr && jn == -2) *scr_at(half) = mk<C>(y.x, y.y);                 // y_top / y_bot
       if (wr && PH == 0 && jn >= 0) xs[(int64_t)jn * n] = mk<C>(v.x, v.y);  // t_jn / b_jn
     }
     sb = sn;
@@ -576,42 +632,41 @@ void pack_tri_t(hz_problem* p, int prec, hipStream_t s) {
   }
 }
 
-template <typename T, int NT, bool ADJ>
+template <typename T, typename A, int NT, bool ADJ>
 void launch_tri(hz_problem* p, int prec, int nrhs, void* xv, hipStream_t s) {
   typedef typename Cx<T>::t C;
   const Factors& f = p->fac[prec];
   C* const x = (C*)xv;
-  constexpr size_t lds = TriShape<T, NT>::lds;
+  constexpr size_t lds = TriShape<T, A, NT>::lds;
   static_assert(lds <= 160 * 1024, "LDS");
-  set_max_lds((const void*)&k_solve_tri<T, NT, 0, ADJ>, lds);
-  set_max_lds((const void*)&k_solve_tri<T, NT, 1, ADJ>, lds);
+  set_max_lds((const void*)&k_solve_tri<T, A, NT, 0, ADJ>, lds);
+  set_max_lds((const void*)&k_solve_tri<T, A, NT, 1, ADJ>, lds);
   for (int r0 = 0; r0 < nrhs; r0 += TW_RHS) {
     const int nr = std::min(TW_RHS, nrhs - r0);
-    const dim3 grid((unsigned)((2 * p->nslot + 7) / 8 * 8 * nr)), block(TriShape<T, NT>::THREADS);
+    const dim3 grid((unsigned)((2 * p->nslot + 7) / 8 * 8 * nr)), block(TriShape<T, A, NT>::THREADS);
     C* const xr = x + (size_t)r0 * p->N;
-    hipLaunchKernelGGL((k_solve_tri<T, NT, 0, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
+    hipLaunchKernelGGL((k_solve_tri<T, A, NT, 0, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
                        p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
                        p->d_slotp.as<int2>(), p->nslot, nr, f.tw_scr.as<C>());
-    hipLaunchKernelGGL((k_solve_tri<T, NT, 1, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
+    hipLaunchKernelGGL((k_solve_tri<T, A, NT, 1, ADJ>), grid, block, lds, s, f.Gtw.as<C>(), xr, p->tab(1, 0),
                        p->tab(1, 1), p->d_symd.as<double2>(), (int)p->nx, (int)p->ny, f.tw_m, (int)p->nz, p->n2, p->N,
                        p->d_slotp.as<int2>(), p->nslot, nr, f.tw_scr.as<C>());
     HZ_HIP(hipGetLastError());
   }
 }
 
-template <typename T>
-void solve_tri_t(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s) {
-  switch (((int)p->nx + 15) / 16) {
-#define HZ_TRI(NT)                                                   \
-  case NT:                                                           \
-    if (adjoint) launch_tri<T, NT, true>(p, prec, nrhs, x, s);       \
-    else launch_tri<T, NT, false>(p, prec, nrhs, x, s);              \
-    break;
-    HZ_TRI(1) HZ_TRI(2) HZ_TRI(3) HZ_TRI(4) HZ_TRI(5) HZ_TRI(6) HZ_TRI(7) HZ_TRI(8)
-    HZ_TRI(9) HZ_TRI(10) HZ_TRI(11) HZ_TRI(12) HZ_TRI(13) HZ_TRI(14) HZ_TRI(15) HZ_TRI(16)
-#undef HZ_TRI
-    default: HZ_CHECK(false, HZ_ERR_ARG, "nx=%d", (int)p->nx);
+template <typename T, typename A, bool ADJ>
+void solve_tri_t(hz_problem* p, int prec, int nrhs, void* x, hipStream_t s) {
+  const int nt = ((int)p->nx + 15) / 16;
+#define HZ_TRI(NT) \
+  if (nt == NT) return launch_tri<T, A, NT, ADJ>(p, prec, nrhs, x, s);
+  // 64, 96, 128, 160, 192 and 200 columns
+  HZ_TRI(4) HZ_TRI(6) HZ_TRI(8) HZ_TRI(10) HZ_TRI(12) HZ_TRI(13)
+  if constexpr (!ADJ || sizeof(A) == 8) {  // (the others have no adjoint with FP32 sums)
+    HZ_TRI(1) HZ_TRI(2) HZ_TRI(3) HZ_TRI(5) HZ_TRI(7) HZ_TRI(9) HZ_TRI(11) HZ_TRI(14) HZ_TRI(15) HZ_TRI(16)
   }
+#undef HZ_TRI
+  HZ_CHECK(false, HZ_ERR_ARG, "nx=%d", (int)p->nx);
 }
 
 }  // namespace
@@ -623,9 +678,16 @@ void pack_tri(hz_problem* p, int prec, hipStream_t s) {
   else pack_tri_t<float>(p, prec, s);
 }
 
-void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, hipStream_t s) {
-  if (prec == HZ_PREC_FP64) solve_tri_t<double>(p, prec, nrhs, x, adjoint, s);
-  else solve_tri_t<float>(p, prec, nrhs, x, adjoint, s);
+void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, bool wide, hipStream_t s) {
+  if (prec == HZ_PREC_FP64) {
+    if (adjoint) solve_tri_t<double, double, true>(p, prec, nrhs, x, s);
+    else solve_tri_t<double, double, false>(p, prec, nrhs, x, s);
+  } else if (adjoint) {
+    if (wide) solve_tri_t<float, double, true>(p, prec, nrhs, x, s);
+    else solve_tri_t<float, float, true>(p, prec, nrhs, x, s);
+  } else {
+    solve_tri_t<float, float, false>(p, prec, nrhs, x, s);
+  }
 }
 
 }  // namespace hz

@@ -131,3 +131,32 @@ def test_twisted_rounding(hz, oracle, monkeypatch, nx, ny, nz):
             ratio.setdefault(prec, []).append(e["twist"] / e["fast"])
     for prec, r in ratio.items():
         assert np.exp(np.mean(np.log(r))) < 1.15, (prec, r)
+
+
+def _strong_layers(hz, n, nz, seed):
+    """The reference's geometry: wide strong x/y layers, smooth medium."""
+    pr = hz.problem
+    d = pr.ref_geometry(n_nopml=n - 40, pml=20, spg=2, nz_nopml=nz - 4, length=(3200.0,) * 3, homo=False)
+    rng = np.random.default_rng(seed)
+    return d, pr.ref_sound_speed(d), (rng.standard_normal(d.N) + 1j * rng.standard_normal(d.N)).astype(np.complex64)
+
+
+@pytest.mark.parametrize("nrhs", [1, 9])
+def test_adjoint_sums_in_fp64(hz, oracle, monkeypatch, nrhs):
+    """complex64 adjoint at a width without streaming kernels: as accurate as the
+    one-directional sweep, which sums in FP64.  Half as many steps a chain, so no
+    larger an error; 12% for scatter."""
+    ratio = []
+    for seed in range(3):
+        d, c, b = _strong_layers(hz, 52, 8, seed)
+        S, P = hz.Solver(d, c), oracle.Problem(d, c)
+        S.factor(hz.abi.PREC_C64)
+        want = extended.plane_solve(P, d.n, b, adjoint=True)
+        e = {}
+        for fam in ("fast", ""):
+            monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
+            got = _solve(S, hz, np.tile(b, (nrhs, 1)), hz.abi.PREC_C64, adjoint=True)
+            e[fam] = max(extended.error(g, want) for g in got)
+        print("adjoint seed %d x %d: %.3g, FP64 sums %.3g" % (seed, nrhs, e[""], e["fast"]), flush=True)
+        ratio.append(e[""] / e["fast"])
+    assert np.exp(np.mean(np.log(ratio))) < 1.12, ratio
