@@ -2193,28 +2193,40 @@ bool wide_adjoint(const hz_problem* p, int prec, int nrhs) {
   return prec == HZ_PREC_C64 && !sym_solve_available(prec, n) && !(nrhs % 8 == 0 && stream_solve_available(prec, n));
 }
 
+// Whether an untuned complex64 batch of nrhs >= 8 takes the twisted solve and not
+// the groups of 8 of solve_rows.  A twisted solve has a workgroup per end, slot
+// and vector, and wins while these are few for the 256 compute units: up to about
+// 4 each to 96 columns, 2 each past them, where a workgroup takes more of a unit.
+// Twisted / rows in ms: 48^3 x 16 (800 workgroups) 0.110 / 0.122, 64^3 x 8 (528)
+// 0.16 / 0.19, x 16 (1056) 0.245 / 0.194, 96^3 x 8 (784) 0.53 / 0.51; with 60
+// lines 100 x 12 planes x 8 (112) 0.164 / 0.338, 48 x 9 (450) 0.235 / 0.331, 64 x
+// 8 (528) 0.341 / 0.348, 96 x 8 (784) 0.435 / 0.360; 140 x 12 x 8 0.257 / 0.544
+// (the chunked kernel 0.482), 48 x 9 0.483 / 0.536, 64 x 8 0.720 / 0.625; 208 x 12
+// x 8 0.342 / 1.11 (chunked 0.995), 48 x 8 (400) 0.672 / 1.18, 64 x 8 0.986 /
+// 1.19, 48 x 16 (800) 1.27 / 1.15; 140^3 x 8 2.61 / 1.62.  Past 96 columns the
+// widths with streaming kernels keep rows in any batch, so that a tuned call
+// there changes its time alone (200^3 x 8 7.04 / 4.65).  Past 208 columns: 239 x
+// 239 x 150 x 8 6.9 / 8.1.
+bool twist_for_groups(const hz_problem* p, int prec, int nrhs) {
+  const int n = (int)p->nx;
+  if (!mfma_solve_available(p, prec) || n > 208) return true;
+  const int64_t groups = 2 * (int64_t)p->nslot * nrhs;
+  return n <= 96 ? groups < 1024 : groups <= 512 && !stream_solve_available(prec, n);
+}
+
 // Whether plane_solve_kernels takes the twisted solve for this call (the only
 // kernel that runs on an incomplete top-down chain): where it is asked for or
 // tuned; untuned always in complex128, and in complex64 unless 8 and more
-// right-hand sides go to the groups of solve_rows, up to 208 columns.
+// right-hand sides go to the groups of solve_rows.
 // One right-hand side, best kernel of before -> twisted, in ms: complex64 48^3
 // 0.234 -> 0.063, 64^3 0.167 -> 0.093, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
-// 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.55 -> 1.52, 140 x 140 x 150
-// 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.2; adjoint 64^3 0.77 -> 0.10, 128^3
-// 0.80 -> 0.35, 200^3 2.19 -> 1.55; complex128 24 x 22 x 28 0.115 -> 0.044,
-// 64^3 0.25 -> 0.11, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140 x 150
-// 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the other kernels:
+// 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.60 -> 1.55, 140 x 140 x 150
+// 1.60 -> 0.55, 239 x 239 x 299 16.9 -> 4.1; adjoint 128^3 0.80 -> 0.35, 200^3
+// 2.19 -> 1.55 (other widths: wide_adjoint); complex128 24 x 22 x 28 0.115 ->
+// 0.044, 64^3 0.25 -> 0.11, 128^3 1.54 -> 0.57 (adjoint 5.51 -> 0.57), 140 x 140
+// x 150 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the other kernels:
 // complex128 128^3 x 8 1.73 against 2.76, 192 x 192 x 100 x 8 4.8 against 7.5;
-// complex64 192^3 x 4 3.59 against 3.70.  Twisted against rows, complex64 x 8
-// and x 16: 64^3 0.16 / 0.19 and 0.245 / 0.194, 96^3 0.53 / 0.51 and 0.88 /
-// 0.54, 128^3 1.15 / 1.07 and 1.93 / 1.14, 140^3 2.61 / 1.62 and 4.70 / 2.95,
-// 192^3 6.25 / 3.46 and 11.6 / 6.08, 200^3 7.04 / 4.65 and 13.1 / 8.26, but 239
-// x 239 x 150 x 8 6.9 / 8.1.  A twisted solve has a workgroup per end, slot and
-// vector, and wins while these are fewer than about 4 for each of the 256
-// compute units (48^3 x 16, 800 of them: 0.110 / 0.122; 64^3 x 16, 1056: rows).
-// That line is drawn up to 96 columns; past them the rows stay on the factors that the other
-// group families also run on, so that a tuned call changes its time alone
-// (few planes pay for it: 131 x 40 x 30 x 8 0.37 against 0.19, 0.63 before).
+// complex64 192^3 x 4 3.59 against 3.70.
 // Under stream capture an untuned call also takes it while the top-down chain
 // is incomplete, which cannot be completed there.
 bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
@@ -2225,8 +2237,7 @@ bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tun
   if (sk != SK_DEFAULT) return false;
   if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
   if (adjoint && wide_adjoint(p, prec, nrhs)) return true;
-  if (nrhs < 8 || !mfma_solve_available(p, prec) || p->nx > 208) return true;
-  if (p->nx <= 96 && 2 * (int64_t)p->nslot * nrhs < 1024) return true;
+  if (nrhs < 8 || twist_for_groups(p, prec, nrhs)) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
   return !f.top_full && cs != hipStreamCaptureStatusNone;
