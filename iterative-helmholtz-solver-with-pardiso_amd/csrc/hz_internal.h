@@ -109,7 +109,7 @@ struct Factors {
   bool tw_ready = false;
   int tw_m = 0;
   // the top-down chain G_j is complete for every j (with the twisted factors
-  // it stops at tw_m - 1 until a one-directional kernel first needs it)
+  // it may stop at tw_m - 1 until a one-directional kernel first needs it)
   bool top_full = true;
   DevBuf Gb, Gtw, tw_scr;
   Hodlr hodlr;

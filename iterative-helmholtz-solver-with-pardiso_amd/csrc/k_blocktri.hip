@@ -2207,9 +2207,11 @@ bool wide_adjoint(const hz_problem* p, int prec, int nrhs) {
 // widths with streaming kernels keep rows in any batch, so that a tuned call
 // there changes its time alone (200^3 x 8 7.04 / 4.65).  Past 208 columns: 239 x
 // 239 x 150 x 8 6.9 / 8.1.
+constexpr int GROUP_ROWS_MAX = 208;
+
 bool twist_for_groups(const hz_problem* p, int prec, int nrhs) {
   const int n = (int)p->nx;
-  if (!mfma_solve_available(p, prec) || n > 208) return true;
+  if (!mfma_solve_available(p, prec) || n > GROUP_ROWS_MAX) return true;
   const int64_t groups = 2 * (int64_t)p->nslot * nrhs;
   return n <= 96 ? groups < 1024 : groups <= 512 && !stream_solve_available(prec, n);
 }
@@ -2304,6 +2306,23 @@ void run_factor(hz_problem* p, int prec, int blocks, int* st, int mode, int m, i
   else run_factor_mem<float>(p, prec, blocks, st, mode, m, jbeg, jend, s);
 }
 
+// Whether a factorisation with twisted factors runs the whole top-down chain all
+// the same: where a one-directional family is tuned or forced for the precision,
+// and where untuned complex64 groups of 8 take the rows, so that no later call
+// pays for the rest of the chain or is refused under capture (112^3 x 8: 2.7 ms
+// for the first call, 7.5 with the chain completed in it).  Not at 128, 160, 192
+// and 200 columns: there the first group or one-directional call completes the
+// chain, and a problem that solves single vectors never does.
+bool wants_top_chain(const hz_problem* p, int prec) {
+  const SolveKernel sk = solve_kernel_choice();
+  if (sk != SK_DEFAULT && sk != SK_TWIST) return true;
+  for (const auto& kv : p->tuned)
+    if (kv.first.first == prec && kv.second.solve_family != HZ_SOLVE_DEFAULT && kv.second.solve_family != HZ_SOLVE_TWIST)
+      return true;
+  const int n = (int)p->nx;
+  return mfma_solve_available(p, prec) && n <= GROUP_ROWS_MAX && !sym_solve_available(prec, n);
+}
+
 }  // namespace
 
 void factor_begin(hz_problem* p, int prec, hipStream_t s) {
@@ -2319,7 +2338,7 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   const bool twist = ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") &&
                      !getenv("HZ_NO_SYM_PACK");
   f.tw_m = twist ? ny / 2 : 0;
-  f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr;
+  f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr || wants_top_chain(p, prec);
   if (twist) {
     const size_t gb = (size_t)p->nslot * (ny - f.tw_m) * (size_t)n * n * f.elem;
     if (f.Gb.bytes != gb) {
@@ -2343,8 +2362,8 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   p->pin_misc.reserve(64);
   *p->pin_misc.as<int>() = -1;
   launch_fill(1, make_double2(0, 0), dscal(p, 63), s);
-  // with the twisted factors the top-down chain stops at tw_m - 1 (the rest is
-  // completed on the first use of a one-directional kernel)
+  // with the twisted factors the top-down chain may stop at tw_m - 1 (the rest
+  // is then completed on the first use of a one-directional kernel)
   if (p->nslot > 0) {
     run_factor(p, prec, twist ? 2 * p->nslot : p->nslot, st, twist ? 1 : 0, f.tw_m, 0, f.top_full ? ny : f.tw_m, s);
     if (twist) run_factor(p, prec, p->nslot, st, 2, f.tw_m, 0, 0, s);

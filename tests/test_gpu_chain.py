@@ -1,0 +1,118 @@
+"""The one-directional factor chain beside the twisted factors: complete after the
+factorisation where a later call would else pay for the rest or be refused, and
+the same blocks where it is completed later."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def hz():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return load_pkg()
+
+
+def _box(hz, n):
+    d = hz.problem.cube_geometry(n, tuple(min(6, v // 4) for v in n), 40.0, beta=0.5, pml_c=30.0)
+    return d, 0.8 + 0.4 * np.random.default_rng(n[0]).random(d.N)
+
+
+def _vectors(d, nrhs, prec, hz, seed=3):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((nrhs, d.N)) + 1j * rng.standard_normal((nrhs, d.N))
+    return torch.from_numpy(x.astype(np.complex128 if prec == hz.abi.PREC_FP64 else np.complex64)).cuda()
+
+
+def _replays(hz, S, prec, x0, want):
+    """Plane solve of x0 captured on a stream of torch's and replayed four times
+    between eager copies: every replay is bit for bit `want`."""
+    lib, st, x = hz.abi.lib(), torch.cuda.Stream(), x0.clone()
+    torch.cuda.synchronize()
+    hz.abi.check(lib.hz_problem_set_stream(S.h, C.c_void_p(st.cuda_stream)), "hz_problem_set_stream")
+    try:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+            rc = lib.hz_plane_solve(S.h, int(prec), 0, x0.shape[0], C.c_void_p(x.data_ptr()))
+        hz.abi.check(rc, "hz_plane_solve under capture")
+        with torch.cuda.stream(st):
+            for _ in range(4):
+                x.copy_(x0)
+                g.replay()
+                st.synchronize()
+                assert torch.equal(x, want)
+    finally:
+        hz.abi.check(lib.hz_problem_set_stream(S.h, C.c_void_p(0)), "hz_problem_set_stream")
+
+
+# complex64 groups at widths whose factorisation always ran the whole chain (rows
+# by default); a forced and a tuned family in complex128
+@pytest.mark.parametrize("n,prec,nrhs,how", [
+    ((112, 6, 66), 1, 8, "untuned"), ((64, 5, 128), 1, 16, "untuned"), ((100, 6, 8), 1, 8, "forced"),
+    ((140, 6, 5), 0, 2, "forced"), ((140, 6, 5), 0, 2, "tuned")])
+def test_first_call_after_a_factorisation_can_be_captured(hz, tmp_path, monkeypatch, n, prec, nrhs, how):
+    d, c = _box(hz, n)
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    monkeypatch.delenv("HZ_FACTOR_FULL", raising=False)
+    if how == "forced":
+        monkeypatch.setenv("HZ_SOLVE_KERNEL", "mfma" if prec == hz.abi.PREC_C64 else "fast")
+    if how == "tuned":
+        line = " | %d 1 16\n" % hz.abi.SOLVE_CHUNKED
+        key = "gfx950 %d %d %d %d %d" % (*n, prec, nrhs)
+        (tmp_path / "t").write_text(key + line + key + " set 2" + line)
+        monkeypatch.setenv("HZ_TUNE_CACHE", str(tmp_path / "t"))
+    x = _vectors(d, nrhs, prec, hz)
+    E, S = hz.Solver(d, c), hz.Solver(d, c)
+    for s in (E, S):
+        s.factor(prec)
+        if how == "tuned":
+            assert s.autotune(prec, nrhs)["from_cache"]
+            s.factor(prec)
+    want = E.plane_solve(x.clone(), prec)  # eager, on a problem of its own
+    _replays(hz, S, prec, x, want)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_untuned_capture_on_an_incomplete_chain(hz, monkeypatch, prec):
+    """128 columns: nothing has completed the chain, and an untuned captured call
+    of any size takes the twisted solve."""
+    d, c = _box(hz, (128, 6, 7))
+    monkeypatch.delenv("HZ_FACTOR_FULL", raising=False)
+    x = _vectors(d, 8, prec, hz)
+    E, S = hz.Solver(d, c), hz.Solver(d, c)
+    monkeypatch.setenv("HZ_SOLVE_KERNEL", "twist")
+    E.factor(prec)
+    want = E.plane_solve(x.clone(), prec)
+    monkeypatch.delenv("HZ_SOLVE_KERNEL")
+    S.factor(prec)
+    _replays(hz, S, prec, x, want)
+
+
+@pytest.mark.parametrize("prec,n", [(1, (160, 20, 9)), (0, (160, 20, 9)), (0, (129, 9, 6)), (0, (64, 12, 6)), (1, (230, 8, 5)), (0, (230, 7, 5))])
+def test_chain_completed_later_is_the_same(hz, monkeypatch, prec, n):
+    """Every one-directional family on a factorisation that stopped halfway, each
+    on a problem of its own (the family's first call completes the chain), equals
+    the one on a factorisation of the whole chain bit for bit."""
+    d, c = _box(hz, n)
+    fams = [("fast", 1, False), ("fast", 1, True), ("mr", 3, False), ("dma", 1, False), ("sym", 1, False), ("sym", 1, True)]
+    if prec == hz.abi.PREC_C64:
+        fams += [("mfma", 9, False), ("mfma", 9, True)]
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    monkeypatch.setenv("HZ_FACTOR_FULL", "1")
+    full = hz.Solver(d, c)
+    full.factor(prec)
+    monkeypatch.delenv("HZ_FACTOR_FULL")
+    for fam, nrhs, adj in fams:
+        monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+        lazy = hz.Solver(d, c)
+        lazy.factor(prec)
+        monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
+        x = _vectors(d, nrhs, prec, hz)
+        assert torch.equal(lazy.plane_solve(x.clone(), prec, adjoint=adj), full.plane_solve(x.clone(), prec, adjoint=adj)), (fam, adj)
