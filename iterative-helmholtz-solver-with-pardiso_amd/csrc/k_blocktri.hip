@@ -2323,6 +2323,46 @@ bool wants_top_chain(const hz_problem* p, int prec) {
   return mfma_solve_available(p, prec) && n <= GROUP_ROWS_MAX && !sym_solve_available(prec, n);
 }
 
+void size_to(DevBuf& b, size_t bytes) {
+  if (b.bytes != bytes) {
+    b.release();
+    b.alloc(bytes);
+  }
+}
+
+// Storage of the twisted factors beside the dense ones: the packed blocks, the
+// workspace of the solves, and the bottom-up blocks that are held until they are
+// packed.  False where the device has not room for them and half as much again
+// as the dense factors take (the vectors of a solve): then none is held and the
+// problem keeps the one-directional factors alone.  HZ_FACTOR_BUDGET caps the
+// free memory that is counted on, in bytes.
+bool twisted_storage(hz_problem* p, int prec, size_t dense, size_t packed) {
+  Factors& f = p->fac[prec];
+  const size_t half = dense / p->ny * (size_t)(p->ny - f.tw_m), scr = (size_t)3 * TW_RHS * p->nz * p->nx * f.elem;
+  size_t free = 0, total = 0;
+  HZ_HIP(hipMemGetInfo(&free, &total));
+  if (const char* e = getenv("HZ_FACTOR_BUDGET")) free = std::min(free, (size_t)strtoull(e, nullptr, 10));
+  const size_t held = f.G.bytes + f.Gb.bytes + f.Gtw.bytes + f.tw_scr.bytes;
+  bool fits = dense + half + packed + scr + dense / 2 <= free + held;
+  if (fits) {
+    try {
+      size_to(f.G, dense);
+      size_to(f.Gb, half);
+      size_to(f.Gtw, packed);
+      size_to(f.tw_scr, scr);
+    } catch (const Error&) {
+      (void)hipGetLastError();
+      fits = false;
+    }
+  }
+  if (!fits) {
+    f.Gb.release();
+    f.Gtw.release();
+    f.tw_scr.release();
+  }
+  return fits;
+}
+
 }  // namespace
 
 void factor_begin(hz_problem* p, int prec, hipStream_t s) {
@@ -2335,26 +2375,19 @@ void factor_begin(hz_problem* p, int prec, hipStream_t s) {
   f.elem = prec == HZ_PREC_FP64 ? sizeof(double2) : sizeof(float2);
   // twisted factors (up to 256 columns, at most two planes a slot): the
   // bottom-up chain runs beside the top-down one in the same launch
-  const bool twist = ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") &&
-                     !getenv("HZ_NO_SYM_PACK");
-  f.tw_m = twist ? ny / 2 : 0;
-  f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr || wants_top_chain(p, prec);
+  bool twist = ny >= 2 && p->slot_pairs && tri_available(n) && !getenv("HZ_NO_TWIST") && !getenv("HZ_NO_SYM_PACK");
+  const size_t bytes = (size_t)p->nslot * ny * (size_t)n * n * f.elem;
+  f.tw_m = ny / 2;
   if (twist) {
-    const size_t gb = (size_t)p->nslot * (ny - f.tw_m) * (size_t)n * n * f.elem;
-    if (f.Gb.bytes != gb) {
-      f.Gb.release();
-      f.Gb.alloc(gb);
-    }
+    twist = twisted_storage(p, prec, bytes, tri_bytes(p, f.elem));
   } else {
     f.Gb.release();
     f.Gtw.release();
     f.tw_scr.release();
   }
-  const size_t bytes = (size_t)p->nslot * ny * (size_t)n * n * f.elem;
-  if (f.G.bytes != bytes) {
-    f.G.release();
-    f.G.alloc(bytes);
-  }
+  if (!twist) f.tw_m = 0;
+  f.top_full = !twist || getenv("HZ_FACTOR_FULL") != nullptr || wants_top_chain(p, prec);
+  size_to(f.G, bytes);
   // status word: device int at the end of the scalar block's misc area, copied
   // to pinned host memory
   grow(p->scal, 4096 * sizeof(double2));
@@ -2376,26 +2409,22 @@ void factor_end(hz_problem* p, int prec, hipStream_t s) {
   Factors& f = p->fac[prec];
   HZ_HIP(hipStreamSynchronize(s));
   HZ_CHECK(*p->pin_misc.as<int>() == 0, HZ_ERR_SINGULAR, "zero pivot while factoring a plane");
-  // symmetric packed copy for the widths the packed solve is instantiated for
-  f.sym_ready = false;
-  if (sym_solve_available(prec, (int)p->nx) && !getenv("HZ_NO_SYM_PACK")) {
-    // with an incomplete top-down chain only the storage is set up here
-    const bool ok = pack_sym_any(p, prec, s, !f.top_full);
-    f.sym_ready = ok && f.top_full;
-    HZ_HIP(hipStreamSynchronize(s));
-  }
   // twisted packed copy; the unpacked bottom-up blocks are not kept
   f.tw_ready = false;
   if (f.Gb.ptr && p->nslot > 0) {
     pack_tri(p, prec, s);
     f.tw_ready = true;
-    const size_t sb = (size_t)3 * TW_RHS * p->nz * p->nx * f.elem;
-    if (f.tw_scr.bytes != sb) {
-      f.tw_scr.release();
-      f.tw_scr.alloc(sb);
-    }
     HZ_HIP(hipStreamSynchronize(s));
     f.Gb.release();
+  }
+  // symmetric packed copy for the widths the packed solve is instantiated for;
+  // with an incomplete top-down chain only the complex64 storage is set up here
+  // (no untuned complex128 call reads the packed copy)
+  f.sym_ready = false;
+  if (sym_solve_available(prec, (int)p->nx) && !getenv("HZ_NO_SYM_PACK") && (f.top_full || prec == HZ_PREC_C64)) {
+    const bool ok = pack_sym_any(p, prec, s, !f.top_full);
+    f.sym_ready = ok && f.top_full;
+    HZ_HIP(hipStreamSynchronize(s));
   }
   f.ready = true;
 }

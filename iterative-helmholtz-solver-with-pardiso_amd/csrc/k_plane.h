@@ -59,10 +59,11 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
                        void* Gb, int jbeg, int jend, hipStream_t s);
 
 
-// Twisted plane solves (k_tri.hip): whether a width has them, the packing of
-// the factor chains (G, Gb) into Gtw, and the solve of nrhs vectors (wide:
-// complex64 adjoint with the sums in FP64).
+// Twisted plane solves (k_tri.hip): whether a width has them, the bytes of the
+// packed blocks, the packing of the factor chains (G, Gb) into Gtw, and the
+// solve of nrhs vectors (wide: complex64 adjoint with the sums in FP64).
 bool tri_available(int nx);
+size_t tri_bytes(const hz_problem* p, size_t elem);
 void pack_tri(hz_problem* p, int prec, hipStream_t s);
 void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, bool wide, hipStream_t s);
 

@@ -613,11 +613,6 @@ void pack_tri_t(hz_problem* p, int prec, hipStream_t s) {
   typedef typename Cx<T>::t C;
   Factors& f = p->fac[prec];
   const int nt = ((int)p->nx + 15) / 16, tiles = nt * (nt + 1) / 2;
-  const size_t bytes = (size_t)p->nslot * p->ny * tiles * 256 * sizeof(C);
-  if (f.Gtw.bytes != bytes) {
-    f.Gtw.release();
-    f.Gtw.alloc(bytes);
-  }
   const double2* dx = p->d_symd.as<double2>();
   // at most 65535 blocks a launch in the second grid dimension
   const int per = 32768 / (int)p->ny > 0 ? 32768 / (int)p->ny : 1;
@@ -672,6 +667,11 @@ void solve_tri_t(hz_problem* p, int prec, int nrhs, void* x, hipStream_t s) {
 }  // namespace
 
 bool tri_available(int nx) { return nx <= 16 * TRI_MAX_NT; }
+
+size_t tri_bytes(const hz_problem* p, size_t elem) {
+  const size_t nt = ((size_t)p->nx + 15) / 16;
+  return (size_t)p->nslot * p->ny * (nt * (nt + 1) / 2) * 256 * elem;
+}
 
 void pack_tri(hz_problem* p, int prec, hipStream_t s) {
   if (prec == HZ_PREC_FP64) pack_tri_t<double>(p, prec, s);

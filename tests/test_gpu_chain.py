@@ -116,3 +116,60 @@ def test_chain_completed_later_is_the_same(hz, monkeypatch, prec, n):
         monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
         x = _vectors(d, nrhs, prec, hz)
         assert torch.equal(lazy.plane_solve(x.clone(), prec, adjoint=adj), full.plane_solve(x.clone(), prec, adjoint=adj)), (fam, adj)
+
+
+@pytest.mark.parametrize("prec,n", [(1, (140, 10, 8)), (0, (129, 7, 9)), (0, (128, 8, 6)), (1, (60, 5, 6))])
+def test_factors_where_the_twisted_ones_do_not_fit(hz, oracle, monkeypatch, prec, n):
+    """With room for the dense factors but not for the twisted ones beside them
+    the factorisation keeps the dense ones (and what the packed widths always
+    held), and every call is that of a problem without twisted factors; with room
+    again it has them."""
+    d, c = _box(hz, n)
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    monkeypatch.delenv("HZ_FACTOR_FULL", raising=False)
+    monkeypatch.setenv("HZ_NO_TWIST", "1")
+    plain = hz.Solver(d, c)
+    plain.factor(prec)
+    monkeypatch.delenv("HZ_NO_TWIST")
+    nx, ny, _ = n
+    dense = plain.slots()[0] * ny * nx * nx * (8 if prec == hz.abi.PREC_C64 else 16)
+    S = hz.Solver(d, c)
+    monkeypatch.setenv("HZ_FACTOR_BUDGET", str(int(1.5 * dense)))
+    S.factor(prec)
+    assert S.factor_bytes() == plain.factor_bytes()
+    for adj in (False, True):
+        for nrhs in (1, 3, 9):
+            x = _vectors(d, nrhs, prec, hz)
+            assert torch.equal(S.plane_solve(x.clone(), prec, adjoint=adj), plain.plane_solve(x.clone(), prec, adjoint=adj))
+    x = np.random.default_rng(5).standard_normal(d.N) + 0j
+    got = S.precond_apply(torch.from_numpy(x).cuda(), prec).cpu().numpy()
+    want = oracle.Problem(d, c).precond_apply(x)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < (1e-4 if prec == hz.abi.PREC_C64 else 1e-10)
+    monkeypatch.delenv("HZ_FACTOR_BUDGET")
+    S.factor(prec)
+    assert S.factor_bytes() > dense
+    y = _vectors(d, 1, prec, hz)
+    monkeypatch.setenv("HZ_SOLVE_KERNEL", "twist")
+    fresh = hz.Solver(d, c)
+    fresh.factor(prec)
+    assert torch.equal(S.plane_solve(y.clone(), prec), fresh.plane_solve(y.clone(), prec))
+
+
+def test_complex128_holds_no_idle_packed_copy(hz, monkeypatch):
+    """At 128 columns untuned complex128 calls read the twisted factors alone: the
+    packed copy of the one-directional ones is there from the first call of a
+    family that reads it, with the same numbers as ever."""
+    d, c = _box(hz, (128, 8, 6))
+    prec = hz.abi.PREC_FP64
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    monkeypatch.delenv("HZ_FACTOR_FULL", raising=False)
+    S = hz.Solver(d, c)
+    S.factor(prec)
+    slots = S.slots()[0]
+    assert S.factor_bytes() == slots * 8 * 16 * (128 * 128 + 36 * 256)  # dense blocks, 36 of 64 tiles
+    x = _vectors(d, 1, prec, hz)
+    monkeypatch.setenv("HZ_SOLVE_KERNEL", "sym")
+    full = hz.Solver(d, c)
+    full.factor(prec)
+    assert torch.equal(S.plane_solve(x.clone(), prec), full.plane_solve(x.clone(), prec))
+    assert S.factor_bytes() == full.factor_bytes()
