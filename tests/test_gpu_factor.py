@@ -46,3 +46,26 @@ def test_factor_widths_vs_oracle(hz, oracle, nx):
         for adj in (False, True):
             e = _rel(S.precond_apply(xd, prec, adjoint=adj).cpu().numpy(), P.precond_apply(x, adjoint=adj))
             assert e < tol, (prec, adj, e)
+
+
+@pytest.mark.parametrize("nx", WIDTHS)
+def test_whole_chain_vs_oracle(hz, oracle, monkeypatch, nx):
+    """The same planes through the one-directional factors, forward and adjoint:
+    the whole top-down chain, in complex128 (and at 128, 160 and 192 columns)
+    completed by the first call from the block where the factorisation stopped."""
+    print("case chain nx=%d" % nx, flush=True)
+    pr = hz.problem
+    ny, nz = 5, 4
+    d = pr.cube_geometry((nx, ny, nz), 0, 37.0, beta=0.02)
+    c = 0.8 + 0.4 * np.random.default_rng(nx).random(d.N)
+    S, P = hz.Solver(d, c), oracle.Problem(d, c)
+    rng = np.random.default_rng(100 + nx)
+    x = rng.standard_normal(d.N) + 1j * rng.standard_normal(d.N)
+    xd = torch.from_numpy(x).cuda()
+    for prec, tol in ((hz.abi.PREC_FP64, 1e-9), (hz.abi.PREC_C64, 1e-3)):
+        monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+        S.factor(prec)
+        monkeypatch.setenv("HZ_SOLVE_KERNEL", "fast")
+        for adj in (False, True):
+            e = _rel(S.precond_apply(xd, prec, adjoint=adj).cpu().numpy(), P.precond_apply(x, adjoint=adj))
+            assert e < tol, (prec, adj, e)

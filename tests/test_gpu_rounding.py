@@ -160,3 +160,17 @@ def test_adjoint_sums_in_fp64(hz, oracle, monkeypatch, nrhs):
         print("adjoint seed %d x %d: %.3g, FP64 sums %.3g" % (seed, nrhs, e[""], e["fast"]), flush=True)
         ratio.append(e[""] / e["fast"])
     assert np.exp(np.mean(np.log(ratio))) < 1.12, ratio
+
+
+def test_adjoint_batches_of_a_streaming_width(hz, monkeypatch):
+    """64 columns, 17 vectors on enough planes for the groups of 8: the groups and
+    the remaining vector, bit for bit, as they come alone."""
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    d, c, _ = _layers(hz, 64, 10, 140, 1)
+    S = hz.Solver(d, c)
+    S.factor(hz.abi.PREC_C64)
+    rng = np.random.default_rng(2)
+    b = (rng.standard_normal((17, d.N)) + 1j * rng.standard_normal((17, d.N))).astype(np.complex64)
+    got = _solve(S, hz, b, hz.abi.PREC_C64, adjoint=True)
+    assert np.array_equal(got[:16], _solve(S, hz, b[:16], hz.abi.PREC_C64, adjoint=True))
+    assert np.array_equal(got[16:], _solve(S, hz, b[16:], hz.abi.PREC_C64, adjoint=True))
