@@ -291,7 +291,7 @@ def plane_solve_kernel(nx, tuning):
     fam = tuning.get("solve_kernel", 0)
     if fam == 6:
         nt = (nx + 15) // 16
-        return "k_solve_tri<%d, 0, false> + k_solve_tri<%d, 1, false>" % (nt, nt)
+        return "k_solve_tri<float, float, %d, 0, false> + k_solve_tri<float, float, %d, 1, false>" % (nt, nt)
     if fam == 5:
         return "k_solve_sym2<%d, false>" % nx
     if fam == 3:
@@ -536,7 +536,8 @@ def bench_config2(a, hz, np, torch, steps, warmup):
 def traffic_source(n, fam):
     """Where roofline.traffic comes from: it is not measured in this run (the
     counter passes need rocprofv3), it is read from the committed summary."""
-    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md"}
+    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md",
+             6: "k_solve_tri_c64_200cube_pmc.md"}
     if n != 200 or fam not in names or not os.path.exists(os.path.join(ROOT, "profiles", names[fam])):
         return None
     return "committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary profiles/%s (not measured in this run)" % names[fam]
@@ -564,7 +565,8 @@ def plane_solve_bytes(dims, fam, nslot):
 def measured_traffic(n, fam):
     """HBM bytes per launch of the plane solve from the committed rocprofv3
     FETCH_SIZE/WRITE_SIZE passes (scaled by a 1 GiB copy), for the 200^3 grid."""
-    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md"}
+    names = {3: "k_solve_dma_c64_200cube_pmc.md", 5: "k_solve_sym2_c64_200cube_pmc.md",
+             6: "k_solve_tri_c64_200cube_pmc.md"}
     if n != 200 or fam not in names:
         return None
     path = os.path.join(ROOT, "profiles", names[fam])

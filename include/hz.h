@@ -218,7 +218,7 @@ int hz_precond_apply_adjoint(hz_problem* p, int prec, int nrhs, const hz_c128* i
  * about nx/64 and nx/8), at most rank 16 per block.  eps < 0 drops the
  * compressed form (back to the dense factors if kept).  A new
  * hz_precond_factor drops it too. */
-/* HZ_HODLR_TWISTED (complex64, where the twisted factors exist): compress the
+/* HZ_HODLR_TWISTED (complex64 twisted factors at nx = 128, 160, 192, 200): compress the
  * twisted factors (chains from both ends of each y-line chain meeting at
  * ny/2) instead of the one-directional ones; the forward applies then run two
  * workgroups per plane over half chains.  No counterpart in the reference,

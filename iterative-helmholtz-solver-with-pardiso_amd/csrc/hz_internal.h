@@ -101,11 +101,11 @@ struct Factors {
   // block columns paired J / T-1-J), for the widths it is built for
   bool sym_ready = false;
   DevBuf Gsym;
-  // twisted factors (complex64): blocks j < tw_m the top-down inverses, block
+  // twisted factors: blocks j < tw_m the top-down inverses, block
   // tw_m the middle inverse, blocks j > tw_m the bottom-up inverses (Gb, dense,
-  // [slot][j - tw_m]), the upper triangles of their symmetric forms packed in
-  // 16 x 16 tiles into Gtw; tw_scr passes y_top, y_bot and f_m between the two
-  // phases (3 x TW_RHS x nz x nx complex64)
+  // [slot][j - tw_m], held while a factorisation runs), their symmetric forms
+  // packed as one half of the 16 x 16 tiles into Gtw; tw_scr passes y_top, y_bot
+  // and f_m between the two phases (3 x TW_RHS x nz x nx complex of the precision)
   bool tw_ready = false;
   int tw_m = 0;
   // the top-down chain G_j is complete for every j (with the twisted factors

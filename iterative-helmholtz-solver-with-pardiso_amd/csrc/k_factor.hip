@@ -29,7 +29,7 @@
 // every step's update (the destination of the multiply-add), so the current
 // column is always the first and the 16 steps are one short loop.  Panel and
 // pivot rows pass to the matrix products through LDS in 16-byte units,
-// swizzled by row so that the operand reads are free of bank conflicts.
+// swizzled by row against bank conflicts of the operand reads.
 #include <type_traits>
 
 #include "hz_internal.h"
@@ -512,12 +512,13 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
   // (complex128: 64, 96, 128, 144).  The line lies where a wave's tiles no longer
   // fit its 256 registers; below it the registers win at every width.  Whole
   // factorisations, panel by panel in memory -> here: complex64 24 x 22 x 28
-  // 0.96 -> 0.47 ms, 64^3 10.8 -> 2.8, 128^3 37.0 -> 9.7, 200^3 136.7 -> 39.8;
-  // complex128 64^3 11.4 -> 3.7, 128^3 77.8 -> 23.7, 140 x 60 x 150 42.4 -> 15.0.
-  // The errors of a preconditioner apply are those of before or smaller (200 x
-  // 40 x 200 complex64 4.1e-6 -> 3.1e-6).  What bounds it now: at 200 columns
-  // the panel wave (one column 1.3 us, 68% of a block's 0.40 ms), the products
-  // taking 345 of 935 thousand cycles beside it.
+  // 0.96 -> 0.54 ms, 64^3 10.8 -> 3.0, 112^3 46.0 -> 14.9, 200^3 (half chains)
+  // 136.8 -> 42.8; complex128 (half chains, whole before) 64^3 11.3 -> 2.4, 128^3
+  // 78.0 -> 13.3.  The errors of a plane solve are those of before or smaller
+  // (one-directional sweeps against 64 bits: complex64 64^3 3.4e-7 -> 2.8e-7, 200 x
+  // 30 x 12 3.9e-5 -> 2.7e-5; complex128 64^3 1.11e-15 -> 0.91e-15).  What bounds
+  // it: one compute unit a chain and, in it, the panel wave; at 200 columns the
+  // matrix units are busy 2.1e10 of 3.8e10 wave cycles, half of which are waits.
   if (prec == HZ_PREC_C64) {
     HZ_FR(float, 3, 1)
     HZ_FR(float, 6, 2)

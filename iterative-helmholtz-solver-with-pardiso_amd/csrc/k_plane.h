@@ -20,9 +20,6 @@ template <typename C> __device__ __forceinline__ C cmul(C a, C b) {
 template <typename C> __device__ __forceinline__ C cfma(C a, C b, C c) {  // a*b + c
   C r; r.x = a.x * b.x - a.y * b.y + c.x; r.y = a.x * b.y + a.y * b.x + c.y; return r;
 }
-template <typename C> __device__ __forceinline__ C cfma_conj(C a, C b, C c) {  // conj(a)*b + c
-  C r; r.x = a.x * b.x + a.y * b.y + c.x; r.y = a.x * b.y - a.y * b.x + c.y; return r;
-}
 template <typename C> __device__ __forceinline__ C cinv(C a) {
   // 1/a with scaling to avoid overflow in |a|^2
   double ax = a.x, ay = a.y;

@@ -52,14 +52,15 @@
 // block's tile as soon as they are read, so a whole block (186 KB at 200
 // columns) is in flight per CU across the two barriers of a step; the loads do
 // not depend on the vector.  Small grids are bound by a step's two barriers, its
-// sums and its update, some 0.6 us, so what the update can know before the
-// products is formed before them.  At 200^3 a solve takes 1.52 ms = 7.5 GB at
-// 4.95 TB/s, the rate of a large device copy there (the products and barriers
+// sums and its update, some 0.6 us, so the update's coefficients are fetched and
+// its scaling is formed before the products.  At 200^3 a solve takes 1.50 to 1.57
+// ms, its 7.84 GB at the rate of a large device copy (the products and barriers
 // alone, without the loads: 1.00 ms); at 64^3 0.093 ms, 1.2 us a step.
 // complex128 at 200^3 2.87 ms (15.0 GB, 5.2 TB/s), at 140 x 140 x 150 0.92 ms.
 // Measured against it: the kernel it replaced at 128, 160, 192 and 200 columns
-// (tiles through an LDS ring per wave) 0.55, 0.81, 1.33 and 1.55 ms against
-// 0.34, 0.71, 1.23 and 1.52.
+// (tiles through an LDS ring per wave) 0.55, 0.81, 1.33 and 1.60 ms against
+// 0.34, 0.71, 1.23 and 1.55.  Registers: complex64 past 240 columns and its
+// adjoint sums in FP64 there spill 2 to 6, nothing else does.
 #include <type_traits>
 
 #include "hz_internal.h"
