@@ -2437,6 +2437,8 @@ void launch_factor(hz_problem* p, int prec, hipStream_t s) {
 void ensure_dense(hz_problem* p, int prec, hipStream_t s) {
   Factors& f = p->fac[prec];
   if (!f.ready || f.top_full) return;
+  HZ_CHECK(f.G.ptr != nullptr || p->nslot == 0, HZ_ERR_STATE,
+           "the dense factors were released by HZ_HODLR_FREE_DENSE, factor again");
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
   HZ_CHECK(cs == hipStreamCaptureStatusNone, HZ_ERR_STATE,
@@ -2521,6 +2523,8 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
     solve_tri(p, prec, nrhs, x, adjoint, adjoint && wide_adjoint(p, prec, nrhs), s);
     return;
   }
+  HZ_CHECK(f.G.ptr != nullptr, HZ_ERR_STATE,
+           "plane solve: the dense factors were released by HZ_HODLR_FREE_DENSE, factor again");
   if (!f.top_full) ensure_dense(p, prec, s);
   const int n = (int)p->nx, ny = (int)p->ny;
   const int ng = std::max(1, APPLY_THREADS / n);

@@ -173,3 +173,25 @@ def test_complex128_holds_no_idle_packed_copy(hz, monkeypatch):
     full.factor(prec)
     assert torch.equal(S.plane_solve(x.clone(), prec), full.plane_solve(x.clone(), prec))
     assert S.factor_bytes() == full.factor_bytes()
+
+
+@pytest.mark.parametrize("twisted", [False, True])
+def test_released_factors_are_an_error(hz, monkeypatch, twisted):
+    """Dense factors released by a compression and the compressed form dropped
+    afterwards: nothing is left to solve with, and every call says so until the
+    next factorisation."""
+    d, c = _box(hz, (128, 8, 6))
+    monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+    prec = hz.abi.PREC_C64
+    S = hz.Solver(d, c)
+    S.factor(prec)
+    x = _vectors(d, 1, prec, hz)
+    want = S.plane_solve(x.clone(), prec)
+    S.compress(prec, eps=1e-4, smallsize=7, free_dense=True, twisted=twisted)
+    S.compress(prec, eps=-1.0, smallsize=7)
+    for call in (lambda: S.plane_solve(x.clone(), prec), lambda: S.plane_solve(x.clone(), prec, adjoint=True),
+                 lambda: S.autotune(prec, 8)):
+        with pytest.raises(hz.abi.HzError):
+            call()
+    S.factor(prec)
+    assert torch.equal(S.plane_solve(x.clone(), prec), want)
