@@ -2181,16 +2181,21 @@ bool twist_solve_available(const hz_problem* p, int prec) {
 
 namespace {
 // Whether a complex64 adjoint sweep sums its products in FP64, as the sweep that
-// k_apply walks does: everywhere but on the packed symmetric factors' widths and
-// in whole groups of 8 on the widths with streaming kernels.  The sums' rounding
-// is a third of the error where the layers are strong (reference grid 64^3
-// 7.5e-8, 9.8e-8 with FP32 sums).  Times in ms, k_apply -> FP64 sums (FP32 sums):
-// 48^3 0.43 -> 0.071 (0.064), 64^3 0.77 -> 0.113 (0.096), 96^3 2.64 -> 0.28
-// (0.21), 140^3 7.7 -> 0.81 (0.56), x 16 28.2 -> 7.1 (2.9, rows), 208^3 22.5 ->
-// 1.72 (1.64), 239 x 239 x 150 31.0 -> 2.12 (2.03).
+// k_apply walks does: to 144 columns, but for the packed symmetric factors' width
+// and whole groups of 8 on the widths with streaming kernels.  On narrow planes
+// with strong layers the sums' rounding shows (adjoint errors of the sweep that
+// k_apply walks, of FP32 and of FP64 sums here: reference grid 64^3 7.3e-8, 9.8e-8
+// and 7.5e-8; FP32 sums against it 68 x 68 x 64 1.31 times, 100 x 100 x 50 1.21,
+// 124 x 124 x 48 1.04, 132 x 132 x 40 1.02); further out the elimination's own
+// errors, smaller than before, cover it (140 x 140 x 40 0.92, 150 x 150 x 60 0.87,
+// 176 x 176 x 48 0.71, 239 x 239 x 44 0.97; boxes of the cube geometry 0.4 to 0.96
+// at 97 to 239 columns).  Times in ms, k_apply -> FP64 sums (FP32 sums): 48^3 0.43
+// -> 0.071 (0.064), 64^3 0.77 -> 0.113 (0.096), 96^3 2.64 -> 0.28 (0.21), 140^3 7.7
+// -> 0.81 (0.56), x 16 28.2 -> 7.1 (2.9, rows).
 bool wide_adjoint(const hz_problem* p, int prec, int nrhs) {
   const int n = (int)p->nx;
-  return prec == HZ_PREC_C64 && !sym_solve_available(prec, n) && !(nrhs % 8 == 0 && stream_solve_available(prec, n));
+  return prec == HZ_PREC_C64 && n <= TRI_WIDE_MAX && !sym_solve_available(prec, n) &&
+         !(nrhs % 8 == 0 && stream_solve_available(prec, n));
 }
 
 // Whether an untuned complex64 batch of nrhs >= 8 takes the twisted solve and not

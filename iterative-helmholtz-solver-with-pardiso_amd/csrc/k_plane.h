@@ -58,7 +58,9 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
 
 // Twisted plane solves (k_tri.hip): whether a width has them, the bytes of the
 // packed blocks, the packing of the factor chains (G, Gb) into Gtw, and the
-// solve of nrhs vectors (wide: complex64 adjoint with the sums in FP64).
+// solve of nrhs vectors (wide: complex64 adjoint with the sums in FP64, to
+// TRI_WIDE_MAX columns).
+constexpr int TRI_WIDE_MAX = 144;
 bool tri_available(int nx);
 size_t tri_bytes(const hz_problem* p, size_t elem);
 void pack_tri(hz_problem* p, int prec, hipStream_t s);

@@ -59,8 +59,8 @@
 // complex128 at 200^3 2.87 ms (15.0 GB, 5.2 TB/s), at 140 x 140 x 150 0.92 ms.
 // Measured against it: the kernel it replaced at 128, 160, 192 and 200 columns
 // (tiles through an LDS ring per wave) 0.55, 0.81, 1.33 and 1.60 ms against
-// 0.34, 0.71, 1.23 and 1.55.  Registers: complex64 past 240 columns and its
-// adjoint sums in FP64 there spill 2 to 6, nothing else does.
+// 0.34, 0.71, 1.23 and 1.55.  Registers: complex64 past 240 columns spills 6, its
+// adjoint past 208 columns 2 to 26, nothing else does.
 #include <type_traits>
 
 #include "hz_internal.h"
@@ -656,10 +656,16 @@ void solve_tri_t(hz_problem* p, int prec, int nrhs, void* x, hipStream_t s) {
   const int nt = ((int)p->nx + 15) / 16;
 #define HZ_TRI(NT) \
   if (nt == NT) return launch_tri<T, A, NT, ADJ>(p, prec, nrhs, x, s);
-  // 64, 96, 128, 160, 192 and 200 columns
-  HZ_TRI(4) HZ_TRI(6) HZ_TRI(8) HZ_TRI(10) HZ_TRI(12) HZ_TRI(13)
-  if constexpr (!ADJ || sizeof(A) == 8) {  // (the others have no adjoint with FP32 sums)
-    HZ_TRI(1) HZ_TRI(2) HZ_TRI(3) HZ_TRI(5) HZ_TRI(7) HZ_TRI(9) HZ_TRI(11) HZ_TRI(14) HZ_TRI(15) HZ_TRI(16)
+  // complex64 adjoint: FP64 sums to TRI_WIDE_MAX columns, FP32 sums past them and
+  // at 64, 96 and 128
+  constexpr bool WIDE = ADJ && sizeof(T) != sizeof(A), C64ADJ = ADJ && sizeof(T) == 4;
+  HZ_TRI(4) HZ_TRI(6) HZ_TRI(8)
+  if constexpr (!C64ADJ || WIDE) {
+    HZ_TRI(1) HZ_TRI(2) HZ_TRI(3) HZ_TRI(5) HZ_TRI(7) HZ_TRI(9)
+  }
+  if constexpr (!WIDE) {
+    static_assert(TRI_WIDE_MAX == 16 * 9, "");
+    HZ_TRI(10) HZ_TRI(11) HZ_TRI(12) HZ_TRI(13) HZ_TRI(14) HZ_TRI(15) HZ_TRI(16)
   }
 #undef HZ_TRI
   HZ_CHECK(false, HZ_ERR_ARG, "nx=%d", (int)p->nx);
