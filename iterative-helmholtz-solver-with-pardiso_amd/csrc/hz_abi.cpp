@@ -515,7 +515,8 @@ int hz_problem_info(const hz_problem* p, int64_t* dims, double* factor_bytes) {
   if (factor_bytes) {
     double b = 0;
     for (int q = 0; q < 2; ++q)
-      b += (double)(p->fac[q].G.bytes + p->fac[q].Gsym.bytes + p->fac[q].Gtw.bytes + p->fac[q].hodlr.pool.bytes);
+      b += (double)(p->fac[q].G.bytes + p->fac[q].Gsym.bytes + p->fac[q].Gb.bytes + p->fac[q].Gtw.bytes +
+                    p->fac[q].hodlr.pool.bytes);
     *factor_bytes = b;
   }
   HZ_API_END
@@ -568,7 +569,7 @@ int hz_precond_hodlr_info(const hz_problem* p, int prec, hz_hodlr_info* out) {
   out->eps = h.eps;
   out->mean_rank = h.mean_rank;
   out->bytes = h.bytes;
-  out->dense_bytes = (double)(f.G.bytes + f.Gsym.bytes + f.Gtw.bytes);
+  out->dense_bytes = (double)(f.G.bytes + f.Gsym.bytes + f.Gb.bytes + f.Gtw.bytes);
   HZ_API_END
 }
 

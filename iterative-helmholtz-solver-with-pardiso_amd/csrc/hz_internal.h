@@ -103,7 +103,8 @@ struct Factors {
   DevBuf Gsym;
   // twisted factors: blocks j < tw_m the top-down inverses, block
   // tw_m the middle inverse, blocks j > tw_m the bottom-up inverses (Gb, dense,
-  // [slot][j - tw_m], held while a factorisation runs), their symmetric forms
+  // [slot][j - tw_m], held while a factorisation runs, and after it where groups
+  // of 8 complex64 vectors use them), their symmetric forms
   // packed as one half of the 16 x 16 tiles into Gtw; tw_scr passes y_top, y_bot
   // and f_m between the two phases (3 x TW_RHS x nz x nx complex of the precision)
   bool tw_ready = false;

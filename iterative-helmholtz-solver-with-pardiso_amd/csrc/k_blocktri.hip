@@ -2127,9 +2127,9 @@ bool try_launch_mr(int n, int ny, int nz, int nrhs, int cap, hipStream_t s, cons
   return true;
 }
 
-// Plane-solve kernel family: HZ_SOLVE_KERNEL=mr|dma|fast|mfma|mfma_sym|sym|twist forces one for
+// Plane-solve kernel family: HZ_SOLVE_KERNEL=mr|dma|fast|mfma|mfma_sym|sym|twist|rows forces one for
 // timing; otherwise the tuned (or default) choice applies.
-enum SolveKernel { SK_DEFAULT, SK_MR, SK_DMA, SK_FAST, SK_MFMA, SK_SYM, SK_MFMA_SYM, SK_TWIST };
+enum SolveKernel { SK_DEFAULT, SK_MR, SK_DMA, SK_FAST, SK_MFMA, SK_SYM, SK_MFMA_SYM, SK_TWIST, SK_ROWS };
 SolveKernel solve_kernel_choice() {
   const char* v = getenv("HZ_SOLVE_KERNEL");
   if (!v || !v[0]) return SK_DEFAULT;
@@ -2140,6 +2140,7 @@ SolveKernel solve_kernel_choice() {
   if (!strcmp(v, "mfma_sym")) return SK_MFMA_SYM;
   if (!strcmp(v, "sym")) return SK_SYM;
   if (!strcmp(v, "twist")) return SK_TWIST;
+  if (!strcmp(v, "rows")) return SK_ROWS;
   return SK_DEFAULT;
 }
 
@@ -2191,40 +2192,50 @@ namespace {
 // 176 x 176 x 48 0.71, 239 x 239 x 44 0.97; boxes of the cube geometry 0.4 to 0.96
 // at 97 to 239 columns).  Times in ms, k_apply -> FP64 sums (FP32 sums): 48^3 0.43
 // -> 0.071 (0.064), 64^3 0.77 -> 0.113 (0.096), 96^3 2.64 -> 0.28 (0.21), 140^3 7.7
-// -> 0.81 (0.56), x 16 28.2 -> 7.1 (2.9, rows).
+// -> 0.81 (0.56).
 bool wide_adjoint(const hz_problem* p, int prec, int nrhs) {
   const int n = (int)p->nx;
   return prec == HZ_PREC_C64 && n <= TRI_WIDE_MAX && !sym_solve_available(prec, n) &&
          !(nrhs % 8 == 0 && stream_solve_available(prec, n));
 }
 
-// Whether an untuned complex64 batch of nrhs >= 8 takes the twisted solve and not
-// the groups of 8 of solve_rows.  A twisted solve has a workgroup per end, slot
-// and vector, and wins while these are few for the 256 compute units: up to about
-// 4 each to 96 columns, 2 each past them, where a workgroup takes more of a unit.
-// Twisted / rows in ms: 48^3 x 16 (800 workgroups) 0.110 / 0.122, 64^3 x 8 (528)
-// 0.16 / 0.19, x 16 (1056) 0.245 / 0.194, 96^3 x 8 (784) 0.53 / 0.51; with 60
-// lines 100 x 12 planes x 8 (112) 0.164 / 0.338, 48 x 9 (450) 0.235 / 0.331, 64 x
-// 8 (528) 0.341 / 0.348, 96 x 8 (784) 0.435 / 0.360; 140 x 12 x 8 0.257 / 0.544
-// (the chunked kernel 0.482), 48 x 9 0.483 / 0.536, 64 x 8 0.720 / 0.625; 208 x 12
-// x 8 0.342 / 1.11 (chunked 0.995), 48 x 8 (400) 0.672 / 1.18, 64 x 8 0.986 /
-// 1.19, 48 x 16 (800) 1.27 / 1.15; 140^3 x 8 2.61 / 1.62.  Past 96 columns the
-// widths with streaming kernels keep rows in any batch, so that a tuned call
-// there changes its time alone (200^3 x 8 7.04 / 4.65).  Past 208 columns: 239 x
-// 239 x 150 x 8 6.9 / 8.1.
+// Whether an untuned complex64 batch of nrhs >= 8 takes solve_tri and not groups
+// of 8.  A twisted solve of single vectors has a workgroup per end, slot and
+// vector, those of a (slot, end) on one XCD; while no XCD has more than its 32
+// compute units of them it is the faster one.  solve_tri / groups on twisted blocks
+// in ms, 60 lines: 48 x 12 planes x 16 (32 on an XCD) 0.074 / 0.077, 24 x 9 (36)
+// 0.091 / 0.078; 64 x 24 x 8 (32) 0.094 / 0.091, x 9 0.117 / 0.091, 64 x 16 0.222 /
+// 0.093; 96 x 24 x 8 0.142 / 0.157, x 9 0.198 / 0.158; 140 x 24 x 8 0.266 / 0.302,
+// x 9 0.473 / 0.304, 64 x 16 1.15 / 0.356; 208 x 24 x 8 0.364 / 0.628, x 9 0.635 /
+// 0.639, 64 x 8 0.969 / 0.669.  Adjoint with FP64 sums 48 x 24 x 8 0.087 / 0.114, x 9
+// 0.112 / 0.113, 140 x 24 x 8 0.378 / 0.504, x 9 0.706 / 0.504, 64 x 16 1.71 / 0.516.
+// 128, 160, 192 and 200 columns take the one-directional rows in any batch, as
+// their other group families, so that a tuned call changes its time alone (200^3
+// x 8 7.04 / 4.65).  Past 208 columns: 239 x 239 x 150 x 8 6.9, one-directional
+// rows 8.1.
 constexpr int GROUP_ROWS_MAX = 208;
 
 bool twist_for_groups(const hz_problem* p, int prec, int nrhs) {
   const int n = (int)p->nx;
   if (!mfma_solve_available(p, prec) || n > GROUP_ROWS_MAX) return true;
-  const int64_t groups = 2 * (int64_t)p->nslot * nrhs;
-  return n <= 96 ? groups < 1024 : groups <= 512 && !stream_solve_available(prec, n);
+  if (sym_solve_available(prec, n)) return false;
+  return (2 * (int64_t)p->nslot + 7) / 8 * nrhs <= 32;
 }
 
-// Whether plane_solve_kernels takes the twisted solve for this call (the only
-// kernel that runs on an incomplete top-down chain): where it is asked for or
-// tuned; untuned always in complex128, and in complex64 unless 8 and more
-// right-hand sides go to the groups of solve_rows.
+// Chains of a few blocks, where a launch costs more than the steps that two ends
+// save: groups of 8 go one way in one launch (64 x 2 x 200 x 8 0.021 ms, 0.030 from
+// both ends; 64 x 6 x 200 x 8 0.030 and 0.039, x 17 0.048 and 0.057; 64 x 20 x 200 x
+// 17 0.117 and 0.113), on a chain that the factorisation runs whole.
+bool short_chain(const hz_problem* p) { return p->ny < 8; }
+
+// The kernels that work on the twisted factors, hence on an incomplete top-down
+// chain: solve_tri, and for groups of 8 complex64 vectors solve_rows_twisted
+// where the dense twisted blocks are kept (keeps_ends).
+enum TwistRoute { TW_NONE, TW_TRI, TW_ROWS };
+
+// What plane_solve_kernels takes of them for this call: what is asked for or
+// tuned; untuned solve_tri always in complex128, and in complex64 unless 8 and
+// more right-hand sides go to groups.
 // One right-hand side, best kernel of before -> twisted, in ms: complex64 48^3
 // 0.234 -> 0.063, 64^3 0.167 -> 0.093, 96^3 0.41 -> 0.20, 128^3 0.55 -> 0.34,
 // 160^3 0.81 -> 0.71, 192^3 1.33 -> 1.23, 200^3 1.60 -> 1.55, 140 x 140 x 150
@@ -2234,20 +2245,22 @@ bool twist_for_groups(const hz_problem* p, int prec, int nrhs) {
 // x 150 3.08 -> 0.92, 200^3 4.42 -> 2.87.  Several, against the other kernels:
 // complex128 128^3 x 8 1.73 against 2.76, 192 x 192 x 100 x 8 4.8 against 7.5;
 // complex64 192^3 x 4 3.59 against 3.70.
-// Under stream capture an untuned call also takes it while the top-down chain
-// is incomplete, which cannot be completed there.
-bool uses_twist(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
+// Under stream capture an untuned call also takes solve_tri while the top-down
+// chain is incomplete, which cannot be completed there.
+TwistRoute twist_route(const hz_problem* p, int prec, int nrhs, bool adjoint, const Tuning& t, hipStream_t s) {
   const Factors& f = p->fac[prec];
-  if (!f.tw_ready) return false;
+  if (!f.tw_ready) return TW_NONE;
   const SolveKernel sk = solve_kernel_choice();
-  if (sk == SK_TWIST) return true;
-  if (sk != SK_DEFAULT) return false;
-  if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST;
-  if (adjoint && wide_adjoint(p, prec, nrhs)) return true;
-  if (nrhs < 8 || twist_for_groups(p, prec, nrhs)) return true;
+  if (sk == SK_TWIST) return TW_TRI;
+  if (sk == SK_ROWS && f.Gb.ptr) return TW_ROWS;
+  if (sk != SK_DEFAULT && sk != SK_ROWS) return TW_NONE;
+  if (!adjoint && t.solve_family != HZ_SOLVE_DEFAULT) return t.solve_family == HZ_SOLVE_TWIST ? TW_TRI : TW_NONE;
+  if (nrhs < 8 || twist_for_groups(p, prec, nrhs)) return TW_TRI;
+  if (f.Gb.ptr) return short_chain(p) && f.top_full && !(adjoint && wide_adjoint(p, prec, nrhs)) ? TW_NONE : TW_ROWS;
+  if (adjoint && wide_adjoint(p, prec, nrhs)) return TW_TRI;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HZ_HIP(hipStreamIsCapturing(s, &cs));
-  return !f.top_full && cs != hipStreamCaptureStatusNone;
+  return !f.top_full && cs != hipStreamCaptureStatusNone ? TW_TRI : TW_NONE;
 }
 }  // namespace
 
@@ -2311,21 +2324,26 @@ void run_factor(hz_problem* p, int prec, int blocks, int* st, int mode, int m, i
   else run_factor_mem<float>(p, prec, blocks, st, mode, m, jbeg, jend, s);
 }
 
+// Whether the dense bottom-up blocks stay beside the top-down ones for the groups
+// of 8 on twisted factors.  Not at 128, 160, 192 and 200 columns, whose groups
+// run on the one-directional factors like the other group families there (the
+// first such call completes the chain), nor past GROUP_ROWS_MAX.
+bool keeps_ends(const hz_problem* p, int prec) {
+  const int n = (int)p->nx;
+  return mfma_solve_available(p, prec) && n <= GROUP_ROWS_MAX && !sym_solve_available(prec, n);
+}
+
 // Whether a factorisation with twisted factors runs the whole top-down chain all
 // the same: where a one-directional family is tuned or forced for the precision,
-// and where untuned complex64 groups of 8 take the rows, so that no later call
-// pays for the rest of the chain or is refused under capture (112^3 x 8: 2.7 ms
-// for the first call, 7.5 with the chain completed in it).  Not at 128, 160, 192
-// and 200 columns: there the first group or one-directional call completes the
-// chain, and a problem that solves single vectors never does.
+// or its untuned groups go one way on a short chain, so that no later call pays
+// for the rest of the chain or is refused under capture.
 bool wants_top_chain(const hz_problem* p, int prec) {
   const SolveKernel sk = solve_kernel_choice();
-  if (sk != SK_DEFAULT && sk != SK_TWIST) return true;
+  if (sk != SK_DEFAULT && sk != SK_TWIST && sk != SK_ROWS) return true;
   for (const auto& kv : p->tuned)
     if (kv.first.first == prec && kv.second.solve_family != HZ_SOLVE_DEFAULT && kv.second.solve_family != HZ_SOLVE_TWIST)
       return true;
-  const int n = (int)p->nx;
-  return mfma_solve_available(p, prec) && n <= GROUP_ROWS_MAX && !sym_solve_available(prec, n);
+  return keeps_ends(p, prec) && short_chain(p);
 }
 
 void size_to(DevBuf& b, size_t bytes) {
@@ -2336,8 +2354,8 @@ void size_to(DevBuf& b, size_t bytes) {
 }
 
 // Storage of the twisted factors beside the dense ones: the packed blocks, the
-// workspace of the solves, and the bottom-up blocks that are held until they are
-// packed.  False where the device has not room for them and half as much again
+// workspace of the solves, and the bottom-up blocks (held until they are packed,
+// or with keeps_ends as long as the factors).  False where the device has not room for them and half as much again
 // as the dense factors take (the vectors of a solve): then none is held and the
 // problem keeps the one-directional factors alone.  HZ_FACTOR_BUDGET caps the
 // free memory that is counted on, in bytes.
@@ -2414,13 +2432,13 @@ void factor_end(hz_problem* p, int prec, hipStream_t s) {
   Factors& f = p->fac[prec];
   HZ_HIP(hipStreamSynchronize(s));
   HZ_CHECK(*p->pin_misc.as<int>() == 0, HZ_ERR_SINGULAR, "zero pivot while factoring a plane");
-  // twisted packed copy; the unpacked bottom-up blocks are not kept
+  // twisted packed copy
   f.tw_ready = false;
   if (f.Gb.ptr && p->nslot > 0) {
     pack_tri(p, prec, s);
     f.tw_ready = true;
     HZ_HIP(hipStreamSynchronize(s));
-    f.Gb.release();
+    if (!keeps_ends(p, prec)) f.Gb.release();
   }
   // symmetric packed copy for the widths the packed solve is instantiated for;
   // with an incomplete top-down chain only the complex64 storage is set up here
@@ -2514,18 +2532,11 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
     HZ_CHECK(f.G.ptr != nullptr, HZ_ERR_STATE,
              "adjoint plane solve: the dense factors were released by HZ_HODLR_FREE_DENSE");
   }
-  if (adjoint && nrhs > 8 && wide_adjoint(p, prec, nrhs)) {
-    // whole groups that go to the rows, then the rest with FP64 sums (64 x 2 x 200
-    // x 17 0.037 ms, 0.072 with FP64 sums for all)
-    const int whole = nrhs / 8 * 8;
-    if (!wide_adjoint(p, prec, whole) && !uses_twist(p, prec, whole, true, t, s)) {
-      plane_solve_kernels(p, prec, whole, x, true, t, s);
-      x = reinterpret_cast<float2*>(x) + (size_t)whole * p->N;
-      nrhs -= whole;
-    }
-  }
-  if (uses_twist(p, prec, nrhs, adjoint, t, s)) {
-    solve_tri(p, prec, nrhs, x, adjoint, adjoint && wide_adjoint(p, prec, nrhs), s);
+  const TwistRoute route = twist_route(p, prec, nrhs, adjoint, t, s);
+  if (route != TW_NONE) {
+    const bool wide = adjoint && wide_adjoint(p, prec, nrhs);
+    if (route == TW_ROWS) solve_rows_twisted(p, nrhs, x, adjoint, wide, s);
+    else solve_tri(p, prec, nrhs, x, adjoint, wide, s);
     return;
   }
   HZ_CHECK(f.G.ptr != nullptr, HZ_ERR_STATE,
@@ -2538,6 +2549,7 @@ void plane_solve_kernels(hz_problem* p, int prec, int nrhs, void* x, bool adjoin
   const double2* cpy = p->tab(1, 1);
   dim3 grid((unsigned)p->nz, (unsigned)nrhs);
   SolveKernel sk = solve_kernel_choice();
+  if (sk == SK_ROWS) sk = SK_DEFAULT;  // no twisted blocks to run on
   // adjoint sweeps (the tuned families are forward kernels): complex64 groups
   // of 8 on the matrix cores, the rest on the packed symmetric factors with
   // G_j^H = conj(D_j^-1 P_j conj(.)), unless the environment asks for another

@@ -1211,6 +1211,7 @@ void hodlr_compress(hz_problem* p, int prec, double eps, int small, int flags) {
     f.G.release();
     f.Gsym.release();
     f.sym_ready = false;
+    f.Gb.release();
     f.Gtw.release();
     if (!twisted) f.tw_scr.release();  // the twisted sweep keeps its workspace
     f.tw_ready = false;

@@ -70,5 +70,8 @@ void solve_tri(hz_problem* p, int prec, int nrhs, void* x, bool adjoint, bool wi
 // (k_rows.hip): whether a problem has them, and the solve of nrhs vectors.
 bool rows_available(const hz_problem* p);
 void solve_rows(hz_problem* p, int nrhs, void* x, bool adjoint, hipStream_t s);
+// The same on the dense twisted blocks (G below tw_m, Gb from there on), to 208
+// columns; wide as for solve_tri.
+void solve_rows_twisted(hz_problem* p, int nrhs, void* x, bool adjoint, bool wide, hipStream_t s);
 
 }  // namespace hz

@@ -163,17 +163,18 @@ def test_adjoint_sums_in_fp64(hz, oracle, monkeypatch, nrhs):
 
 
 def test_adjoint_batches_of_a_streaming_width(hz, monkeypatch):
-    """64 columns, 17 vectors on enough planes for the groups of 8: the groups and
-    the remaining vector, bit for bit, as they come alone."""
+    """64 columns, 17 vectors on enough planes for groups of 8: all of them with
+    FP64 sums, within 12% of the error of single vectors, which have them."""
     monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
-    d, c, _ = _layers(hz, 64, 10, 140, 1)
+    d, c, b = _strong_layers(hz, 64, 40, 1)
     S = hz.Solver(d, c)
+    S.factor(hz.abi.PREC_FP64)
     S.factor(hz.abi.PREC_C64)
-    rng = np.random.default_rng(2)
-    b = (rng.standard_normal((17, d.N)) + 1j * rng.standard_normal((17, d.N))).astype(np.complex64)
-    got = _solve(S, hz, b, hz.abi.PREC_C64, adjoint=True)
-    assert np.array_equal(got[:16], _solve(S, hz, b[:16], hz.abi.PREC_C64, adjoint=True))
-    assert np.array_equal(got[16:], _solve(S, hz, b[16:], hz.abi.PREC_C64, adjoint=True))
+    want = _solve(S, hz, b, hz.abi.PREC_FP64, adjoint=True)
+    one = _solve(S, hz, b, hz.abi.PREC_C64, adjoint=True)
+    got = _solve(S, hz, np.tile(b, (17, 1)), hz.abi.PREC_C64, adjoint=True)
+    e1 = np.linalg.norm(one - want)
+    assert max(np.linalg.norm(g - want) for g in got) < 1.12 * e1
 
 
 @pytest.mark.parametrize("n,nrhs", [(140, 1), (140, 8), (150, 1), (150, 8), (176, 1), (206, 3), (224, 1)])

@@ -75,19 +75,24 @@ def test_tri_widths_past_the_tiles(hz, oracle):
             assert _rel(got, P.precond_apply(x, adjoint=adj)) < tol
 
 
-# complex64 groups past 96 columns: the twisted solve to 512 ends x slots x
-# vectors at widths without streaming kernels (slots: nz // 2 + 1), rows beyond
+# complex64 batches: single vectors while no XCD has more than 32 workgroups,
+# ceil(2 slots / 8) x vectors (slots: nz // 2 + 1), groups beyond, on the
+# one-directional factors for fewer than 8 lines; always those at 128 columns
 @pytest.mark.parametrize("nx,ny,nz,nrhs,fam", [
-    (140, 10, 12, 8, "twist"), (100, 6, 62, 8, "twist"), (100, 6, 64, 8, "mfma"), (208, 4, 40, 12, "twist"),
-    (208, 4, 42, 12, "mfma"), (97, 5, 9, 51, "twist"), (97, 5, 9, 52, "mfma"), (128, 6, 12, 8, "mfma"), (96, 6, 12, 8, "twist")])
+    (140, 10, 12, 8, "twist"), (100, 6, 24, 8, "twist"), (100, 8, 24, 9, "rows"), (208, 8, 40, 12, "rows"),
+    (97, 5, 9, 16, "twist"), (97, 9, 9, 17, "rows"), (128, 6, 12, 8, "mfma"), (96, 6, 12, 8, "twist"), (48, 8, 40, 8, "rows"),
+    (150, 7, 24, 9, "mfma"), (209, 4, 40, 8, "twist")])
 def test_groups_take_the_faster_kernel(hz, monkeypatch, nx, ny, nz, nrhs, fam):
-    """Untuned batches are bit for bit the batches of the family the rule names."""
+    """Untuned batches, forward and adjoint, are bit for bit the batches of the
+    family the rule names."""
     d, c = _case(hz, "s7", nx, ny, nz)
     monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
     S = hz.Solver(d, c)
     S.factor(hz.abi.PREC_C64)
     rng = np.random.default_rng(nz)
     x = torch.from_numpy((rng.standard_normal((nrhs, d.N)) + 1j * rng.standard_normal((nrhs, d.N))).astype(np.complex64)).cuda()
-    got = S.plane_solve(x.clone(), hz.abi.PREC_C64)
-    monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
-    assert torch.equal(got, S.plane_solve(x.clone(), hz.abi.PREC_C64))
+    for adj in (False, True):
+        monkeypatch.delenv("HZ_SOLVE_KERNEL", raising=False)
+        got = S.plane_solve(x.clone(), hz.abi.PREC_C64, adjoint=adj)
+        monkeypatch.setenv("HZ_SOLVE_KERNEL", fam)
+        assert torch.equal(got, S.plane_solve(x.clone(), hz.abi.PREC_C64, adjoint=adj)), adj
