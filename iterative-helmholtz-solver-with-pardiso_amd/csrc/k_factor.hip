@@ -512,9 +512,9 @@ bool launch_factor_reg(hz_problem* p, int prec, const PlaneTabs& tb, int blocks,
   // (complex128: 64, 96, 128, 144).  The line lies where a wave's tiles no longer
   // fit its 256 registers; below it the registers win at every width.  Whole
   // factorisations, panel by panel in memory -> here: complex64 24 x 22 x 28
-  // 0.96 -> 0.54 ms, 64^3 10.8 -> 3.0, 112^3 46.0 -> 14.9, 200^3 (half chains)
-  // 136.8 -> 42.8; complex128 (half chains, whole before) 64^3 11.3 -> 2.4, 128^3
-  // 78.0 -> 13.3.  The errors of a plane solve are those of before or smaller
+  // 0.96 -> 0.54 ms; half chains, whole before: 64^3 10.8 -> 1.55, 112^3 46.0 ->
+  // 7.5, 140^3 88.5 -> 15.1, complex128 64^3 11.3 -> 2.4, 128^3 78.0 -> 13.3; half
+  // chains before and now: 200^3 136.8 -> 42.8.  The errors of a plane solve are those of before or smaller
   // (one-directional sweeps against 64 bits: complex64 64^3 3.4e-7 -> 2.8e-7, 200 x
   // 30 x 12 3.9e-5 -> 2.7e-5; complex128 64^3 1.11e-15 -> 0.91e-15).  What bounds
   // it: one compute unit a chain and, in it, the panel wave; at 200 columns the

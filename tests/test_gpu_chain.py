@@ -52,10 +52,11 @@ def _replays(hz, S, prec, x0, want):
         hz.abi.check(lib.hz_problem_set_stream(S.h, C.c_void_p(0)), "hz_problem_set_stream")
 
 
-# complex64 groups at widths whose factorisation always ran the whole chain (rows
-# by default); a forced and a tuned family in complex128
+# complex64 groups by default: one way on a short chain, from both ends on a chain
+# that stopped halfway; a forced family in either precision and a tuned one
 @pytest.mark.parametrize("n,prec,nrhs,how", [
-    ((112, 6, 66), 1, 8, "untuned"), ((64, 5, 128), 1, 16, "untuned"), ((100, 6, 8), 1, 8, "forced"),
+    ((112, 6, 66), 1, 8, "untuned"), ((64, 5, 128), 1, 16, "untuned"), ((112, 9, 66), 1, 8, "untuned"),
+    ((100, 6, 8), 1, 8, "forced"),
     ((140, 6, 5), 0, 2, "forced"), ((140, 6, 5), 0, 2, "tuned")])
 def test_first_call_after_a_factorisation_can_be_captured(hz, tmp_path, monkeypatch, n, prec, nrhs, how):
     d, c = _box(hz, n)
